@@ -373,6 +373,20 @@ int lng_table_grad(const void* grad_memory, int mem_dtype, const void* codes, in
                    const uint8_t* valid_mask, int64_t B, int64_t T, int32_t R, int32_t route_start, int32_t mem_dim,
                    int32_t order, int32_t bits, int64_t table_rows, float* table_grad, void* stream);
 
+/* The same gradient (lngram_v2.py:1084-1092, :454) written instead of added: every row of routes
+ * route_start .. route_start + R - 1 of table_grad [table_rows, mem_dim] (out_dtype f32 or bf16) gets
+ * the fp32 sum of the gradient rows of its windows, rounded once (zero where none names it); other
+ * rows are not touched.  grad_memory's rows are grad_stride elements apart in (b, t, r) order (a
+ * slice of wider rows needs no copy); rows, table and workspace 16-byte aligned, grad_stride a
+ * multiple of 16 bytes.  The windows are sorted by row in the workspace
+ * (lng_table_grad_workspace_bytes; 0 for shapes it does not serve: bits * order > 13), which is
+ * written by the call before it is read; the order of a row's sum varies between calls. */
+size_t lng_table_grad_workspace_bytes(int64_t B, int64_t T, int32_t R, int32_t order, int32_t bits);
+int lng_table_grad_rows(const void* grad_memory, int mem_dtype, int64_t grad_stride, const void* codes,
+                        int codes_dtype, const uint8_t* valid_mask, int64_t B, int64_t T, int32_t R,
+                        int32_t route_start, int32_t mem_dim, int32_t order, int32_t bits, int64_t table_rows,
+                        void* workspace, size_t workspace_bytes, void* table_grad, int out_dtype, void* stream);
+
 /* ---------------------------------------------------------------- serving layout and host-RAM rows */
 /* Device address of pinned host memory (hipHostGetDevicePointer): the serving movers below read
  * host-RAM tables through it (zero-copy over the host link).  LNG_E_HIP for memory that is not

@@ -81,7 +81,7 @@ class _LngramSurrogate(torch.autograd.Function):
 
 class _TableRows(torch.autograd.Function):
     """One order's looked-up rows ``[B, T, R, D]`` (zero where masked; ``lng_route_tokens``) with
-    the gather's table gradient (``lng_table_grad``), the embedding backward of
+    the gather's table gradient (``lng_table_grad_rows``), the embedding backward of
     ``lngram_v2.py:1084-1092``."""
 
     @staticmethod
@@ -97,8 +97,8 @@ class _TableRows(torch.autograd.Function):
     def backward(ctx, grad: Tensor):
         codes_chunk, valid_mask = ctx.saved_tensors
         order, bits, route_start, rows, dtype = ctx.cfg
-        g = ops.table_grad(grad, codes_chunk, valid_mask, order, bits, route_start, rows)
-        return (g.to(dtype),) + (None,) * 9
+        g = ops.table_grad_rows(grad, codes_chunk, valid_mask, order, bits, route_start, rows, dtype)
+        return (g,) + (None,) * 9
 
 
 class RMSNorm(nn.Module):

@@ -112,6 +112,9 @@ SIGNATURES = {
     "lng_surrogate_grad_ws": (_int, [_p, _p, _int, _p, _int, _p, _int, _p, _i64, _p, _i64, _i64, _i32, _i32, _i32, _i32,
                                      _i32, _f, _f, _int, _p, ctypes.c_size_t, _p, _int, _p]),
     "lng_table_grad": (_int, [_p, _int, _p, _int, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i64, _p, _p]),
+    "lng_table_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32]),
+    "lng_table_grad_rows": (_int, [_p, _int, _i64, _p, _int, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i64, _p,
+                                   ctypes.c_size_t, _p, _int, _p]),
     "lng_host_device_pointer": (_int, [_p, ctypes.POINTER(_p)]),
     "lng_permute_table": (_int, [_p, _p, _int, _i32, _i32, _i32, _i32, _p]),
     "lng_serving_address": (_int, [_p, _int, _i64, _i64, _i32, _i32, _i32, _p, _p]),

@@ -837,6 +837,55 @@ def table_grad(grad_memory: torch.Tensor, codes: torch.Tensor, valid_mask: torch
     return out
 
 
+def _row_stride(t: torch.Tensor) -> int | None:
+    """Elements between consecutive rows of ``t [..., D]`` when its leading indices collapse into one
+    row index and 16-byte pieces of the rows are aligned; None otherwise."""
+    es = t.element_size()
+    if t.stride(-1) != 1 or t.data_ptr() % 16:
+        return None
+    rs, n = None, 1                       # row stride, rows spanned by the dimensions seen so far
+    for size, stride in zip(reversed(t.shape[:-1]), reversed(t.stride()[:-1])):
+        if size == 1:
+            continue
+        if rs is None:
+            rs = stride
+        elif stride != rs * n:
+            return None
+        n *= size
+    rs = t.shape[-1] if rs is None else rs
+    return rs if rs >= t.shape[-1] and rs * es % 16 == 0 else None
+
+
+def table_grad_rows(grad_memory: torch.Tensor, codes: torch.Tensor, valid_mask: torch.Tensor | None, order: int,
+                    bits: int, route_start: int, table_rows: int, dtype: torch.dtype) -> torch.Tensor:
+    """``table_grad`` in ``dtype`` (fp32 sums rounded once), without atomics where
+    ``lng_table_grad_rows`` serves the shape; a gradient that is a slice of wider rows is read in place."""
+    dev = _dev(grad_memory, codes, valid_mask)
+    b, t, r, md = grad_memory.shape
+    nws = lib().lng_table_grad_workspace_bytes(b, t, r, int(order), int(bits))
+    if not nws or md not in (32, 64, 128, 256) or dtype not in (torch.float32, torch.bfloat16):
+        return table_grad(grad_memory, codes, valid_mask, order, bits, route_start, table_rows).to(dtype)
+    if tuple(codes.shape) != (b, t, r):
+        raise ValueError("table_grad: codes must be [B, T, R]")
+    if valid_mask is not None and tuple(valid_mask.shape) != (b, t):
+        raise ValueError("table_grad: valid_mask must be [B, T]")
+    g = grad_memory if grad_memory.dtype in (torch.float32, torch.bfloat16) else grad_memory.float()
+    rs = _row_stride(g)
+    if rs is None:
+        g = _c(g)
+        rs = md
+    cc = _c(codes if codes.dtype in (torch.uint8, torch.int32, torch.int64) else codes.to(torch.int64))
+    vm = None if valid_mask is None else _c(valid_mask.to(torch.uint8))
+    whole = int(route_start) == 0 and r << (int(bits) * int(order)) == int(table_rows)
+    out = (torch.empty if whole else torch.zeros)(int(table_rows), md, dtype=dtype, device=dev)
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    rc = _timed("table_grad", dev, lambda: lib().lng_table_grad_rows(
+        _ptr(g), dtype_code(g.dtype), rs, _ptr(cc), dtype_code(cc.dtype), _ptr(vm), b, t, r, int(route_start), md,
+        int(order), int(bits), int(table_rows), _ptr(ws), ws.numel(), _ptr(out), dtype_code(dtype), _stream(dev)))
+    check(rc, "table_grad_rows")
+    return out
+
+
 # ----------------------------------------------------------------------------- serving layout
 def table_address(t: torch.Tensor) -> int:
     """Device-visible address of a table's first element: a GPU tensor's own, or the mapping of a
