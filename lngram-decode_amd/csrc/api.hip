@@ -98,6 +98,60 @@ __global__ void k_ngram_rows(CodeView codes, int64_t B, int64_t T, int32_t R, in
   rows[i] = static_cast<RowT>(ngram_row(codes, T, R, b, t, r, ords.v[oi], bits, seg, valid));
 }
 
+// Rows of 2^lpr_log2 16-byte pieces: a block owns 64 consecutive positions of one route.  One thread
+// forms each (position, order) row index into LDS (masks, divisions and index arithmetic once a row,
+// not once a piece), then 2^lpr_log2 lanes copy each row.  The blocks of one XCD (the dispatcher deals
+// blocks to the 8 XCDs in turn) work on one route at a time, so a route's block of the tables (1.06 MB
+// for orders 2 and 3, mem_dim 128, bf16) stays in that XCD's L2 and the copy is bound by its stores.
+// NT: stores that do not stay in the caches, for outputs past them (cached ones evict the tables).
+// At 8 x 2048 positions, 184 routes, 1.54 GB of rows: 308 us (5.0 TB/s stored); with cached stores 536,
+// in token order with non-temporal stores 748, one thread a piece in token order (k_route_tokens) 882.
+constexpr int RR_POS = 64;
+constexpr int64_t RR_NT_BYTES = int64_t{32} << 20;  // past the eight L2s together
+// Below this many bytes a launch is one short wave of blocks and its time is the chain codes -> index
+// -> row -> store, which one thread a piece walks without the barrier (a tree's 1.5 MB: 4.8 against
+// 5.1 us).
+constexpr int64_t RR_MIN_BYTES = int64_t{4} << 20;
+template <bool NT>
+__global__ __launch_bounds__(256) void k_route_rows(CodeView codes, int64_t T, int64_t t_first, int64_t T_out,
+                                                    int64_t W, int32_t R, int32_t rs, int32_t rw, OrderList ords,
+                                                    int32_t bits, const char* t0, const char* t1, const char* t2,
+                                                    const char* t3, int32_t lpr_log2, const int32_t* seg,
+                                                    const uint8_t* valid, char* __restrict__ out) {
+  __shared__ int64_t row[RR_POS * 4];
+  const int tid = threadIdx.x;
+  const int64_t xcd = blockIdx.x & 7, k8 = blockIdx.x >> 3;
+  const int64_t tiles = (W + RR_POS - 1) / RR_POS;
+  const int64_t r = (k8 / tiles) * 8 + xcd;
+  const int64_t w0 = (k8 % tiles) * RR_POS;
+  if (r >= rw) return;  // the whole block
+  const int n = ords.n;
+  const int rows = static_cast<int>(W - w0 < RR_POS ? W - w0 : RR_POS) * n;  // (position, order) pairs
+  const uint32_t seg_bytes = 16u << lpr_log2;
+  if (tid < rows) {
+    const int64_t w = w0 + tid / n;
+    row[tid] = ngram_row(codes, T, R, w / T_out, t_first + w % T_out, rs + static_cast<int32_t>(r), ords.v[tid % n],
+                         bits, seg, valid, (int64_t(1) << bits) - 1);
+  }
+  __syncthreads();
+  const int piece = tid & ((1 << lpr_log2) - 1), grp = tid >> lpr_log2, ng = 256 >> lpr_log2;
+  const int64_t pos_bytes = static_cast<int64_t>(rw) * n * seg_bytes;  // the host checks 64 of them fit 31 bits
+  const __amdgpu_buffer_rsrc_t ors =
+      dev_buf(out + w0 * pos_bytes + r * n * static_cast<int64_t>(seg_bytes), static_cast<uint32_t>(RR_POS * pos_bytes));
+#pragma unroll 4
+  for (int i = grp; i < rows; i += ng) {
+    const int oi = i % n, pl = i / n;
+    const int64_t x = row[i];
+    u32x4 v{0u, 0u, 0u, 0u};
+    if (x >= 0) {
+      const char* tab = oi == 0 ? t0 : oi == 1 ? t1 : oi == 2 ? t2 : t3;
+      v = *reinterpret_cast<const u32x4*>(tab + x * seg_bytes + piece * 16);
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(v, ors, pl * static_cast<uint32_t>(pos_bytes) + oi * seg_bytes + piece * 16, 0,
+                                           NT ? CPOL_NT : 0);
+  }
+}
+
 // One thread copies one `vec`-byte piece of an output route token.  Output
 // [B, T_out, rw, n_orders * mem_dim]; segment = (b, t, r, order), mem_dim*esize bytes.
 template <typename V>
@@ -315,7 +369,20 @@ int lng_route_tokens(const void* codes, int codes_dtype, int64_t B, int64_t T, i
                        n_orders > 3 ? tables[3] : nullptr};
   CodeView cv{codes, codes_dtype};
   hipStream_t s = as_stream(stream);
-  if (seg_bytes % 16 == 0) {
+  // whole 16-byte pieces, a power of two of them up to a block's threads, a tile's bytes and the grid
+  // in range: the tiled copy; small outputs and other row widths: one thread a piece
+  const int64_t W = B * t_out;
+  const int64_t blocks = 8 * cdiv(rw, 8) * cdiv(W, RR_POS);
+  if (segs * seg_bytes >= RR_MIN_BYTES && seg_bytes % 16 == 0 && (seg_bytes & (seg_bytes - 1)) == 0 &&
+      seg_bytes <= 4096 && blocks < (int64_t{1} << 31) &&
+      static_cast<int64_t>(rw) * n_orders * seg_bytes * RR_POS < (int64_t{1} << 31)) {
+    const bool nt = segs * seg_bytes > RR_NT_BYTES;
+    auto* kern = nt ? k_route_rows<true> : k_route_rows<false>;
+    const char* const* ct = reinterpret_cast<const char* const*>(tp);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, cv, T, T - t_out, t_out, W, R,
+                       route_start, rw, ol, bits, ct[0], ct[1], ct[2], ct[3], __builtin_ctz(seg_bytes / 16),
+                       segment_ids, valid_tokens, static_cast<char*>(out));
+  } else if (seg_bytes % 16 == 0) {
     const int64_t n = segs * (seg_bytes / 16);
     hipLaunchKernelGGL(k_route_tokens<u32x4>, dim3(cdiv(n, 256)), dim3(256), 0, s, cv, B, T, T - t_out, t_out, R,
                        route_start, rw, ol, bits, tp[0], tp[1], tp[2], tp[3], seg_bytes, segment_ids, valid_tokens,

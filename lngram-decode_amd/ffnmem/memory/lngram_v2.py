@@ -101,6 +101,44 @@ class _TableRows(torch.autograd.Function):
         return (g,) + (None,) * 9
 
 
+class _SurrogateLookup(torch.autograd.Function):
+    """Every order's looked-up rows ``[B, T, R, len(orders) * D]`` in one gather
+    (``lng_route_tokens``), with what ``_TableRows`` and ``_LngramSurrogate`` give order by order on
+    the backward: the tables' gather gradients and the sum of the orders' surrogate route-logit
+    gradients.  The rows are not kept: the surrogate reads them from the tables."""
+
+    @staticmethod
+    def forward(ctx, q_logits: Tensor, route_codes: Tensor, codes_chunk: Tensor, cfg: tuple,
+                segment_ids: Optional[Tensor], valid_tokens: Optional[Tensor], *masks_and_tables: Tensor) -> Tensor:
+        """``cfg`` = (orders, bits, route_start, route_end, temperature, scale, exact); then one
+        ``_valid_mask`` per order and one table per order."""
+        orders, bits, route_start, route_end = cfg[:4]
+        n = len(orders)
+        ctx.cfg = cfg
+        ctx.save_for_backward(q_logits, codes_chunk, *masks_and_tables)
+        return ops.route_tokens(route_codes, [t.detach() for t in masks_and_tables[n:]], orders, bits, route_start,
+                                route_end, segment_ids, valid_tokens, None)
+
+    @staticmethod
+    def backward(ctx, grad: Tensor):
+        orders, bits, route_start, _, temperature, scale, exact = ctx.cfg
+        q_logits, codes = ctx.saved_tensors[:2]
+        n = len(orders)
+        masks, tables = ctx.saved_tensors[2:2 + n], ctx.saved_tensors[2 + n:]
+        width = tables[0].shape[1]
+        grad_q, grad_t = None, [None] * n
+        for i, (order, valid, table) in enumerate(zip(orders, masks, tables)):
+            part = grad[..., i * width:(i + 1) * width]
+            if ctx.needs_input_grad[0]:
+                g = ops.surrogate_grad(part, None, q_logits.detach(), codes, table.detach(), valid, order, bits,
+                                       route_start, temperature, scale, exact)
+                grad_q = g if grad_q is None else grad_q + g
+            if ctx.needs_input_grad[6 + n + i]:
+                grad_t[i] = ops.table_grad_rows(part, codes, valid, order, bits, route_start, table.shape[0],
+                                                table.dtype)
+        return (grad_q,) + (None,) * (5 + n) + tuple(grad_t)
+
+
 class RMSNorm(nn.Module):
     """RMSNorm (``lngram_v2.py:36-53``): ``F.rms_norm`` semantics, the row normalised and
     multiplied by ``weight`` in fp32 and rounded once to the input dtype.  Runs ``lng_rmsnorm``."""
@@ -407,6 +445,13 @@ class _RouteNgramMemoryBase(nn.Module):
         b, t, _ = route_codes.shape
         codes = route_codes[:, :, route_start:route_end].contiguous()
         q_chunk = q_logits_btrm[:, :, route_start:route_end, :]
+        tables = [self.tables[f"ngram_{order}"].weight for order in self.ngrams]
+        if len({(t.dtype, t.shape[1]) for t in tables}) == 1:
+            masks = [self._valid_mask(order, b, t, route_codes.device, segment_ids, valid_tokens)
+                     for order in self.ngrams]
+            cfg = (self.ngrams, self.bits_per_route, route_start, route_end, self.q_surrogate_temperature,
+                   self.q_surrogate_scale, self.q_surrogate_mode == "exact")
+            return _SurrogateLookup.apply(q_chunk, route_codes, codes, cfg, segment_ids, valid_tokens, *masks, *tables)
         parts = []
         for order in self.ngrams:
             valid = self._valid_mask(order, b, t, route_codes.device, segment_ids, valid_tokens)

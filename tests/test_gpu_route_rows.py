@@ -1,0 +1,48 @@
+"""The tiled route-token gather (``lng_route_tokens``) at its edges, bit for bit against the oracle's
+rows: tiles of 64 positions, row widths of one piece to a block's threads, masks, route ranges and
+tails, and outputs on both sides of the non-temporal store line."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from lngram_hip import ops
+from oracle import memory as om
+
+pytestmark = pytest.mark.gpu
+
+# (B, T, R, route_start, route_end, D, orders, bits, dtype, target_length, masked)
+CASES = [
+    (1, 1, 1, 0, 1, 8, (2, 3), 4, torch.bfloat16, None, False),          # small: one thread a piece
+    (1, 63, 184, 0, 184, 128, (2, 3), 4, torch.bfloat16, None, True),    # 5.9 MB: one short tile
+    (1, 64, 201, 3, 201, 64, (1, 2, 3, 4), 2, torch.bfloat16, None, True),
+    (3, 65, 181, 0, 181, 128, (2, 3), 4, torch.bfloat16, 31, True),      # tails across tiles
+    (64, 400, 11, 0, 11, 8, (2, 3), 4, torch.bfloat16, None, False),     # one-piece rows
+    (2, 260, 3, 0, 3, 1024, (1,), 4, torch.float32, None, False),        # 4 KB rows: one row a block pass
+    (9, 129, 40, 1, 39, 32, (2, 3), 4, torch.float32, None, True),
+    (2, 300, 97, 0, 97, 24, (2, 3), 4, torch.bfloat16, None, True),      # 48 bytes: one thread a piece
+    (5, 391, 33, 0, 33, 128, (2, 3), 4, torch.bfloat16, None, True),     # 33.0 MB: non-temporal stores
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[f"{i}" for i in range(len(CASES))])
+@pytest.mark.parametrize("codes_dtype", [torch.uint8, torch.int64])
+def test_rows_equal_the_oracle(dev, case, codes_dtype):
+    B, T, R, r0, r1, D, orders, bits, dt, tail, masked = case
+    gen = torch.Generator().manual_seed(T)
+    codes = torch.randint(0, 1 << bits, (B, T, R), generator=gen)
+    tables = [torch.randn(R << (bits * o), D, generator=gen).to(dt) for o in orders]
+    seg = val = None
+    if masked:
+        seg = torch.zeros(B, T, dtype=torch.int64)
+        seg[:, T // 2:] = 1
+        val = torch.rand(B, T, generator=gen) > 0.1
+    got = ops.route_tokens(codes.to(codes_dtype).to(dev), [t.to(dev) for t in tables], orders, bits, r0, r1,
+                           None if seg is None else seg.to(dev), None if val is None else val.to(dev), tail)
+    rows = torch.from_numpy(om.route_rows(codes.numpy(), orders, bits, 0, R, segment_ids=None if seg is None else
+                                          seg.numpy(), valid_tokens=None if val is None else val.numpy()))
+    want = torch.cat([torch.where((rows[..., i] >= 0)[..., None], tab[rows[..., i].clamp_min(0)], torch.zeros(1, dtype=dt))
+                      for i, tab in enumerate(tables)], -1)[:, :, r0:r1]
+    want = want if tail is None else want[:, -tail:]
+    assert torch.equal(got.cpu(), want)
