@@ -387,6 +387,23 @@ int lng_table_grad_rows(const void* grad_memory, int mem_dtype, int64_t grad_str
                         int32_t route_start, int32_t mem_dim, int32_t order, int32_t bits, int64_t table_rows,
                         void* workspace, size_t workspace_bytes, void* table_grad, int out_dtype, void* stream);
 
+/* The whole backward of the training lookup of orders 2 and 3 (lngram_v2.py:430-447, :1084-1092):
+ * grad_q [B, T, R, bits] (out_dtype f32 or bf16) = lng_surrogate_grad of order 2 plus that of order 3
+ * (approximate mode, looked-up rows from the tables), each rounded to out_dtype before the addition,
+ * and grad_table2 / grad_table3 (bf16, the tables' shapes) = lng_table_grad_rows of each, from one
+ * reading of grad_memory [B, T, R, 2 * mem_dim] (order 2's half first, rows grad_stride elements
+ * apart).  Any of the three gradients may be null (not wanted).  Serves the shapes for which
+ * lng_lookup_grad_workspace_bytes gives a size (bf16 rows of 128, 4-bit codes, exact = 0, R <= 256,
+ * B*T < 2^20); rows and tables 16-byte aligned, the workspace (written before it is read) 256-byte. */
+size_t lng_lookup_grad_workspace_bytes(int64_t B, int64_t T, int32_t R, int32_t mem_dim, int32_t bits, int mem_dtype,
+                                       int exact);
+int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t grad_stride, const void* q_logits, int q_dtype,
+                    const void* codes, int codes_dtype, const void* table2, const void* table3, int64_t table2_rows,
+                    int64_t table3_rows, const uint8_t* valid2, const uint8_t* valid3, int64_t B, int64_t T, int32_t R,
+                    int32_t route_start, int32_t mem_dim, int32_t bits, float temperature, float scale,
+                    void* workspace, size_t workspace_bytes, void* grad_q, int out_dtype, void* grad_table2,
+                    void* grad_table3, void* stream);
+
 /* ---------------------------------------------------------------- serving layout and host-RAM rows */
 /* Device address of pinned host memory (hipHostGetDevicePointer): the serving movers below read
  * host-RAM tables through it (zero-copy over the host link).  LNG_E_HIP for memory that is not

@@ -14,12 +14,11 @@
 // form (k_table_grad) adds W * R * D fp32 values one atomic each into a cleared fp32 table, which the
 // caller then rounds: 10.5 ms an order at 8 x 2048 positions, 184 routes, D 128, bf16, whatever the
 // order, against the whole training lookup with its backward at 3.9 ms (25.2 ms before).
-#include "common.h"
+#include "window_sort.h"
 
 namespace lng {
 
 
-constexpr uint32_t TG_DEAD = 0xFFFF;  // key of a position without a gradient (never an address: S <= 2^13)
 constexpr int TG_LONG = 1024;        // a row of more windows than this is summed by its whole block
 
 struct TgWs {  // byte offsets in the workspace
@@ -63,7 +62,7 @@ __global__ __launch_bounds__(256) void k_tg_keys(TgArgs a, uint16_t* __restrict_
     const int wl = i >> 6, rl = i & 63;
     const int64_t w = w0 + wl;
     const int r = r0 + rl;
-    uint32_t key = TG_DEAD;
+    uint32_t key = WIN_DEAD;
     if (w < a.W && r < a.R && w % a.T >= a.order - 1 && (a.valid == nullptr || a.valid[w])) {
       key = 0;
       for (int k = 0; k < a.order; ++k)
@@ -78,62 +77,11 @@ __global__ __launch_bounds__(256) void k_tg_keys(TgArgs a, uint16_t* __restrict_
   }
 }
 
-// keys are read 8 a thread (16 bytes: a route's row of keys is a multiple of 128 bytes)
 __global__ __launch_bounds__(1024) void k_tg_sort(TgArgs a, const uint16_t* __restrict__ keys,
                                                   uint32_t* __restrict__ start, uint32_t* __restrict__ perm) {
-  extern __shared__ uint32_t cnt[];  // [S], then [16] wave totals
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = blockIdx.x;
-  const int S = 1 << a.shift;
-  uint32_t* wsum = cnt + S;
-  const u32x4* kr = reinterpret_cast<const u32x4*>(keys + static_cast<int64_t>(r) * a.kstride);
-  const int64_t nv = a.kstride / 8;
-  for (int i = tid; i < S; i += 1024) cnt[i] = 0;
-  __syncthreads();
-  for (int64_t i = tid; i < nv; i += 1024) {
-    const u32x4 q = kr[i];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t key = (q[j >> 1] >> (16 * (j & 1))) & 0xFFFF;
-      if (key != TG_DEAD) atomicAdd(&cnt[key], 1u);
-    }
-  }
-  __syncthreads();
-  // exclusive scan of the counters: a thread's S / 1024 consecutive ones, then the threads' totals
-  const int per = S > 1024 ? S / 1024 : 1;
-  const int c0 = tid * per;
-  uint32_t sum = 0;
-  if (c0 < S)
-    for (int i = 0; i < per; ++i) sum += cnt[c0 + i];
-  uint32_t inc = sum;
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t o = __shfl_up(inc, d);
-    if (lane >= d) inc += o;
-  }
-  if (lane == 63) wsum[wave] = inc;
-  __syncthreads();
-  uint32_t base = inc - sum;
-  for (int i = 0; i < wave; ++i) base += wsum[i];
-  uint32_t* st = start + static_cast<int64_t>(r) * (S + 1);
-  if (c0 < S) {
-    for (int i = 0; i < per; ++i) {
-      const uint32_t c = cnt[c0 + i];
-      cnt[c0 + i] = base;
-      st[c0 + i] = base;
-      base += c;
-    }
-    if (c0 + per == S) st[S] = base;
-  }
-  __syncthreads();
-  uint32_t* pm = perm + static_cast<int64_t>(r) * a.W;
-  for (int64_t i = tid; i < nv; i += 1024) {
-    const u32x4 q = kr[i];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t key = (q[j >> 1] >> (16 * (j & 1))) & 0xFFFF;
-      if (key != TG_DEAD) pm[atomicAdd(&cnt[key], 1u)] = static_cast<uint32_t>(i * 8 + j);
-    }
-  }
+  extern __shared__ uint32_t cnt[];  // [S + 16]
+  const int64_t r = blockIdx.x, S = int64_t{1} << a.shift;
+  sort_windows(keys + r * a.kstride, a.kstride, static_cast<int>(S), 0, start + r * (S + 1), perm + r * a.W, cnt);
 }
 
 template <typename TM, int V>

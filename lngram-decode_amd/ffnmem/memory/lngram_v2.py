@@ -104,8 +104,8 @@ class _TableRows(torch.autograd.Function):
 class _SurrogateLookup(torch.autograd.Function):
     """Every order's looked-up rows ``[B, T, R, len(orders) * D]`` in one gather
     (``lng_route_tokens``), with what ``_TableRows`` and ``_LngramSurrogate`` give order by order on
-    the backward: the tables' gather gradients and the sum of the orders' surrogate route-logit
-    gradients.  The rows are not kept: the surrogate reads them from the tables."""
+    the backward (``lng_lookup_grad``): the tables' gather gradients and the sum of the orders'
+    surrogate route-logit gradients.  The rows are not kept: the surrogate reads them from the tables."""
 
     @staticmethod
     def forward(ctx, q_logits: Tensor, route_codes: Tensor, codes_chunk: Tensor, cfg: tuple,
@@ -125,17 +125,9 @@ class _SurrogateLookup(torch.autograd.Function):
         q_logits, codes = ctx.saved_tensors[:2]
         n = len(orders)
         masks, tables = ctx.saved_tensors[2:2 + n], ctx.saved_tensors[2 + n:]
-        width = tables[0].shape[1]
-        grad_q, grad_t = None, [None] * n
-        for i, (order, valid, table) in enumerate(zip(orders, masks, tables)):
-            part = grad[..., i * width:(i + 1) * width]
-            if ctx.needs_input_grad[0]:
-                g = ops.surrogate_grad(part, None, q_logits.detach(), codes, table.detach(), valid, order, bits,
-                                       route_start, temperature, scale, exact)
-                grad_q = g if grad_q is None else grad_q + g
-            if ctx.needs_input_grad[6 + n + i]:
-                grad_t[i] = ops.table_grad_rows(part, codes, valid, order, bits, route_start, table.shape[0],
-                                                table.dtype)
+        want = (ctx.needs_input_grad[0],) + tuple(ctx.needs_input_grad[6 + n:])
+        grad_q, grad_t = ops.lookup_grad(grad, q_logits.detach(), codes, [t.detach() for t in tables], masks, orders,
+                                         bits, route_start, temperature, scale, exact, want)
         return (grad_q,) + (None,) * (5 + n) + tuple(grad_t)
 
 

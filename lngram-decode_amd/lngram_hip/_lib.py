@@ -115,6 +115,9 @@ SIGNATURES = {
     "lng_table_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32]),
     "lng_table_grad_rows": (_int, [_p, _int, _i64, _p, _int, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i64, _p,
                                    ctypes.c_size_t, _p, _int, _p]),
+    "lng_lookup_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32, _int, _int]),
+    "lng_lookup_grad": (_int, [_p, _int, _i64, _p, _int, _p, _int, _p, _p, _i64, _i64, _p, _p, _i64, _i64, _i32, _i32,
+                               _i32, _i32, _f, _f, _p, ctypes.c_size_t, _p, _int, _p, _p, _p]),
     "lng_host_device_pointer": (_int, [_p, ctypes.POINTER(_p)]),
     "lng_permute_table": (_int, [_p, _p, _int, _i32, _i32, _i32, _i32, _p]),
     "lng_serving_address": (_int, [_p, _int, _i64, _i64, _i32, _i32, _i32, _p, _p]),

@@ -886,6 +886,52 @@ def table_grad_rows(grad_memory: torch.Tensor, codes: torch.Tensor, valid_mask: 
     return out
 
 
+def lookup_grad(grad_memory: torch.Tensor, q_logits: torch.Tensor, codes: torch.Tensor, tables, masks, orders,
+                bits: int, route_start: int, temperature: float, scale: float, exact: bool, want) -> tuple:
+    """Backward of the lookup of several orders: ``(route-logit gradient [B, T, R, bits], [table
+    gradients])`` from ``grad_memory [B, T, R, len(orders) * D]``; ``want`` = (logits', each table's),
+    an entry None where not wanted.  One reading of the gradient for orders (2, 3) at the shapes
+    ``lng_lookup_grad`` serves; else ``surrogate_grad`` and ``table_grad_rows`` order by order."""
+    dev = _dev(grad_memory, q_logits, codes, *tables, *masks)
+    b, t, r, _ = grad_memory.shape
+    md = tables[0].shape[1]
+    tabs = [_c(tb) for tb in tables]
+    nws = 0
+    if tuple(orders) == (2, 3) and grad_memory.dtype == tabs[0].dtype and b * t:
+        nws = lib().lng_lookup_grad_workspace_bytes(b, t, r, md, int(bits), dtype_code(tabs[0].dtype), int(bool(exact)))
+    if not nws:
+        grad_q, grads = None, []
+        for i, (order, tab, valid) in enumerate(zip(orders, tabs, masks)):
+            part = grad_memory[..., i * md:(i + 1) * md]
+            if want[0]:
+                g = surrogate_grad(part, None, q_logits, codes, tab, valid, order, bits, route_start, temperature,
+                                   scale, exact)
+                grad_q = g if grad_q is None else grad_q + g
+            grads.append(table_grad_rows(part, codes, valid, order, bits, route_start, tab.shape[0], tab.dtype)
+                         if want[1 + i] else None)
+        return grad_q, grads
+    if tuple(q_logits.shape) != (b, t, r, bits) or tuple(codes.shape) != (b, t, r) or \
+            any(tuple(m.shape) != (b, t) for m in masks):
+        raise ValueError("lookup_grad: q_logits [B,T,R,bits], codes [B,T,R], masks [B,T]")
+    rs = _row_stride(grad_memory)
+    g = grad_memory if rs is not None else _c(grad_memory)
+    q, cc = _c(q_logits), _c(codes if codes.dtype in (torch.uint8, torch.int32, torch.int64) else codes.to(torch.int64))
+    vm = [_c(m.to(torch.uint8)) for m in masks]
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    gq = torch.empty(b, t, r, bits, dtype=q.dtype, device=dev) if want[0] else None
+    grads = []
+    for order, tab, w in zip(orders, tabs, want[1:]):
+        whole = int(route_start) == 0 and r << (int(bits) * order) == tab.shape[0]
+        grads.append((torch.empty_like if whole else torch.zeros_like)(tab) if w else None)
+    rc = _timed("lookup_grad", dev, lambda: lib().lng_lookup_grad(
+        _ptr(g), dtype_code(g.dtype), 2 * md if rs is None else rs, _ptr(q), dtype_code(q.dtype), _ptr(cc),
+        dtype_code(cc.dtype), _ptr(tabs[0]), _ptr(tabs[1]), tabs[0].shape[0], tabs[1].shape[0], _ptr(vm[0]),
+        _ptr(vm[1]), b, t, r, int(route_start), md, int(bits), float(temperature), float(scale), _ptr(ws), ws.numel(),
+        _ptr(gq), dtype_code(q.dtype), _ptr(grads[0]), _ptr(grads[1]), _stream(dev)))
+    check(rc, "lookup_grad")
+    return gq, grads
+
+
 # ----------------------------------------------------------------------------- serving layout
 def table_address(t: torch.Tensor) -> int:
     """Device-visible address of a table's first element: a GPU tensor's own, or the mapping of a
