@@ -7,7 +7,7 @@
 // consecutive output channels of one token: a packed store for plain outputs,
 // and exactly one route's 4 sign bits for the router epilogue.
 // fp32 runs on a VALU tile kernel (the tiny fp32 layer and fp32 routers).
-#include "common.h"
+#include "gemm_tile.h"
 
 namespace lng {
 
@@ -764,6 +764,85 @@ __global__ __launch_bounds__(512, 1) void k_gemm_proj_bf16(const bf16* __restric
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// Tiles for more rows than the skinny kernel's and fewer than fill the chip with 256-row tiles (K % 64
+// == 0): BN x BM of 4 waves (gemm_tile.h).  Bound by the latency of a K stage's loads while blocks are
+// few, then by LDS reads; rowsq (row-statistics partials, as k_gemm_proj_bf16 writes them) needs BN =
+// 128.  XRMS scales row m by rsqrt(mean(x_m^2) + eps) before rounding.
+template <int EPI, bool XRMS, int BN, int BM, int WN, int WM>
+__global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, const bf16* __restrict__ X, int64_t N,
+                                                   int64_t M, int64_t K, int n_tiles, void* __restrict__ out,
+                                                   float* __restrict__ logits, void* __restrict__ codes, int codes_dt,
+                                                   int64_t routes, float* __restrict__ rowsq, float x_eps) {
+  using G = TileGemm<BN, BM, WN, WM, 1, 3>;
+  __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
+  const int nt = static_cast<int>(blockIdx.x) % n_tiles;
+  const int64_t n0 = static_cast<int64_t>(nt) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
+  G g;
+  g.template run<XRMS>(ring, W, X, N, M, K, n0, m0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wn = wave % WN, wm = wave / WN;
+  const int rsel = lane & 15, psel = lane >> 4;
+  float ps[G::FM];
+#pragma unroll
+  for (int j = 0; j < G::FM; ++j) {
+    const int64_t m = m0 + wm * (BM / WM) + j * 16 + rsel;
+    const float rs = XRMS ? __builtin_amdgcn_rsqf(g.xss[j] / static_cast<float>(K) + x_eps) : 1.f;
+    ps[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < G::FN; ++i) {
+      const int64_t n = n0 + wn * (BN / WN) + i * 16 + 4 * psel;
+      f32x4 v = g.acc[i][j];
+      if (XRMS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= rs;
+      }
+      if (EPI == EPI_BF16) {
+        const bf16x4 pk = {static_cast<bf16>(v[0]), static_cast<bf16>(v[1]), static_cast<bf16>(v[2]),
+                           static_cast<bf16>(v[3])};
+        if (rowsq) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float r = static_cast<float>(pk[e]);
+            ps[j] = fmaf(r, r, ps[j]);
+          }
+        }
+        if (m < M && n < N) *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + m * N + n) = pk;  // N % 4 == 0
+      } else if (m < M && n < N) {
+        if (logits) *reinterpret_cast<f32x4*>(logits + m * N + n) = v;
+        if (EPI == EPI_ROUTER) {
+          const int code = (v[0] > 0.f ? 1 : 0) | (v[1] > 0.f ? 2 : 0) | (v[2] > 0.f ? 4 : 0) | (v[3] > 0.f ? 8 : 0);
+          if (codes_dt == LNG_U8)
+            static_cast<uint8_t*>(codes)[m * routes + (n >> 2)] = static_cast<uint8_t>(code);
+          else
+            static_cast<int32_t*>(codes)[m * routes + (n >> 2)] = code;
+        }
+      }
+    }
+  }
+  if (EPI == EPI_BF16 && rowsq) {
+    // partial nt of row m: its 128 columns, summed over the lanes of a row, then over the WN waves
+    float* red = reinterpret_cast<float*>(ring);
+    __syncthreads();  // every wave has left the ring
+#pragma unroll
+    for (int j = 0; j < G::FM; ++j) {
+      float v = ps[j];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (psel == 0) red[wn * BM + wm * (BM / WM) + j * 16 + rsel] = v;
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < BM && m0 + threadIdx.x < M) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < WN; ++w) v += red[w * BM + threadIdx.x];
+      rowsq[static_cast<int64_t>(nt) * M + m0 + threadIdx.x] = v;
+      // the partials come in pairs (256 columns): an odd last one has an empty partner
+      if (nt == n_tiles - 1 && (n_tiles & 1)) rowsq[static_cast<int64_t>(nt + 1) * M + m0 + threadIdx.x] = 0.f;
+    }
+  }
+}
+
 // fp32 VALU tile GEMM: 64x64 tile per 256-thread block, 4x4 outputs per thread,
 // K staged through LDS 16 at a time.  A/B element types may be float or bf16.
 template <typename TA, typename TB, typename TO>
@@ -883,12 +962,59 @@ static int launch_skinny(const bf16* w, const bf16* x, int64_t N, int64_t M, int
   return check_launch("gemm_bf16_skinny");
 }
 
+// The tile of a shape, by the blocks it makes: a block's K loop takes about 5 us at K = 1024 however
+// small the tile, so the smallest tile that still fits the chip at 2-3 blocks a CU wins, and past that
+// the larger tile's fewer operand bytes.  Measured at K = 1024 (us; N 1024: the 128-row DMA tile up to
+// M 1000, then the 256-row projection tile; N 736: the router on the 128-row tile, M 8192 on the wide
+// one):
+//   M             200    500    777   1500   2331   4095   6000   8192
+//   N 1024 before 15.8   16.0   16.2   21.4   22.0   22.2   23.2   25.1
+//          here    5.0    5.5    6.4    8.4   13.0   15.5   23.3  (29.7: not taken)
+//   N 736  before 15.8   15.9   15.8   16.0   16.2   16.6   25.1   26.3
+//          here    5.2    5.6    6.2    7.9    9.2   13.2   20.8   22.1
+//   N 1024 with row statistics before: 34.3 35.6 35.7 21.7 22.0 23.1 24.7; here 7.2 7.3 7.6 9.1 14.1 16.0 24.3
+enum { TILE_NONE, TILE_32_32, TILE_64_32, TILE_64_64, TILE_128_32, TILE_128_64 };
+static int pick_tile(int64_t N, int64_t M, int64_t K, bool rowsq) {
+  if (M <= SK_MAXM || K % 64 != 0 || N % 4 != 0 || N * K * 2 >= (int64_t{1} << 31)) return TILE_NONE;
+  auto blocks = [&](int64_t bn, int64_t bm) { return cdiv(N, bn) * cdiv(M, bm); };
+  if (rowsq) {  // whole 128-column partials
+    if (blocks(128, 32) <= 384) return TILE_128_32;
+  } else {
+    if (blocks(32, 32) <= 640) return TILE_32_32;
+    if (blocks(64, 32) <= 640) return TILE_64_32;
+    if (blocks(64, 64) <= 768) return TILE_64_64;
+  }
+  return blocks(128, 64) <= 768 ? TILE_128_64 : TILE_NONE;
+}
+
+template <int EPI, bool XRMS>
+static int launch_tile(int tile, const bf16* w, const bf16* x, int64_t N, int64_t M, int64_t K, void* out,
+                       float* logits, void* codes, int codes_dt, int64_t routes, float* rowsq, float x_eps,
+                       hipStream_t s) {
+  auto go = [&](auto* kern, int64_t bn, int64_t bm) {
+    const int n_tiles = static_cast<int>(cdiv(N, bn));
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, x, N, M, K,
+                       n_tiles, out, logits, codes, codes_dt, routes, rowsq, x_eps);
+    return check_launch("gemm_bf16_tile");
+  };
+  if (EPI == EPI_BF16 && tile == TILE_128_32) return go(&k_gemm_tile<EPI, XRMS, 128, 32, 4, 1>, 128, 32);
+  switch (tile) {
+    case TILE_32_32: return go(&k_gemm_tile<EPI, XRMS, 32, 32, 2, 2>, 32, 32);
+    case TILE_64_32: return go(&k_gemm_tile<EPI, XRMS, 64, 32, 2, 2>, 64, 32);
+    case TILE_64_64: return go(&k_gemm_tile<EPI, XRMS, 64, 64, 2, 2>, 64, 64);
+    default: return go(&k_gemm_tile<EPI, XRMS, 128, 64, 2, 2>, 128, 64);
+  }
+}
+
 template <int EPI>
 static int launch_mfma(const bf16* w, const bf16* x, int64_t N, int64_t M, int64_t K, void* out, float* logits,
                        void* codes, int codes_dt, int64_t routes, hipStream_t s, float* rowsq = nullptr) {
   if (!rowsq && M <= SK_MAXM && K % 32 == 0 && N % 16 == 0 && (EPI != EPI_ROUTER || N % 4 == 0))
     return launch_skinny<EPI>(w, x, N, M, K, RowMap{M, 0, 0, nullptr}, out ? out : logits, logits, codes, codes_dt,
                               routes, s);
+  if (const int tile = pick_tile(N, M, K, rowsq != nullptr))
+    return launch_tile<EPI, false>(tile, w, x, N, M, K, out, EPI == EPI_F32 && !logits ? static_cast<float*>(out) : logits,
+                                   codes, codes_dt, routes, rowsq, 0.f, s);
   if constexpr (EPI != EPI_BF16) {
     if (K % WT_K == 0 && M >= 4096 && N > GB2 && N <= 2 * WT_N && (N & 3) == 0) {
       const int n_tiles = static_cast<int>(cdiv(N, WT_N));
@@ -953,7 +1079,7 @@ __global__ void k_fold_columns(const bf16* __restrict__ w, const bf16* __restric
 
 // Shared entry for bf16 MFMA linears (used by other translation units).
 int linear_bf16(const void* x, const void* w, int64_t M, int64_t N, int64_t K, void* y, hipStream_t s) {
-  if (proj_shape(N, M, K))
+  if (!pick_tile(N, M, K, false) && proj_shape(N, M, K))
     return launch_proj(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, static_cast<bf16*>(y),
                        nullptr, s);
   return launch_mfma<EPI_BF16>(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, y, nullptr,
@@ -982,7 +1108,7 @@ int lng_linear_rowsq(const void* x, const void* w, int64_t M, int64_t N, int64_t
   if (K % DK) return fail(LNG_E_ARG, "linear_rowsq: needs K % 32 == 0");
   if (!rowsq) return fail(LNG_E_ARG, "linear_rowsq: rowsq buffer required");
   if (M == 0) return LNG_OK;
-  if (proj_shape(N, M, K))
+  if (!pick_tile(N, M, K, true) && proj_shape(N, M, K))
     return launch_proj(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, static_cast<bf16*>(y),
                        rowsq, as_stream(stream));
   return launch_mfma<EPI_BF16>(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, y, nullptr,
@@ -997,6 +1123,9 @@ int lng_linear_rowscale(const void* x, const void* w, int64_t M, int64_t N, int6
   if (M == 0) return LNG_OK;
   if (!proj_shape(N, M, K))
     return fail(LNG_E_ARG, "linear_rowscale: needs M >= 1024, N >= 64, N % 8 == 0 and K % 64 == 0");
+  if (const int tile = pick_tile(N, M, K, false))
+    return launch_tile<EPI_BF16, true>(tile, static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, y,
+                                       nullptr, nullptr, 0, 0, nullptr, eps, as_stream(stream));
   return launch_proj(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, static_cast<bf16*>(y), nullptr,
                      as_stream(stream), true, eps);
 }

@@ -1,0 +1,129 @@
+// bf16 GEMM tiles for the row counts between the skinny kernel and the one-tile-per-CU kernels.
+//
+// y[m, n] = sum_k x[m, k] * w[n, k]: a block of 4 waves computes BN (w rows) x BM (x rows), wave
+// (wn, wm) of the WN x WM grid its BN/WN x BM/WM part in 16x16x32 fragments, accumulating in K order
+// (per output the same instructions as the other bf16 kernels, so equal results).  K advances 64 a
+// stage through a ring of SLOTS LDS stages filled by buffer loads straight into LDS; rows past N or M
+// lie outside the buffers and read as zero.  Piece p (16 bytes) of row r sits in slot p ^ (r & 7): the
+// operand reads are free of bank conflicts.  NP > 1: w is NP consecutive [N, K] matrices whose products
+// with the same x rows add up (an fp32 weight's bf16 pieces).
+#pragma once
+
+#include "common.h"
+
+namespace lng {
+
+template <int BN, int BM, int WN, int WM, int NP, int SLOTS>
+struct TileGemm {
+  static constexpr int NWAVE = WN * WM, NT = 64 * NWAVE;
+  static constexpr int K_ST = 64;
+  static constexpr int ROWS = NP * BN + BM;             // LDS rows of a stage, the w pieces first
+  static constexpr int FN = BN / WN / 16, FM = BM / WM / 16;
+  static constexpr int LOADS = ROWS / 8 / NWAVE;        // 8 rows an instruction
+  static constexpr int W_LOADS = NP * BN / 8 / NWAVE;
+  static constexpr int LDS_ELEMS = SLOTS * ROWS * K_ST;
+  static_assert(ROWS % (8 * NWAVE) == 0 && NP * BN % (8 * NWAVE) == 0 && BN % (16 * WN) == 0 && BM % (16 * WM) == 0, "tile split");
+  static_assert((SLOTS - 2) * LOADS <= 60, "vmcnt");
+
+  f32x4 acc[FN][FM];
+  float xss[FM];  // XRMS: this lane's share of the sum of squares of x row 16 j + (lane & 15)
+
+  // waits until at most `left` later stages of this wave's loads are in flight
+  __device__ __forceinline__ static void wait(int left) {
+    if (left >= SLOTS - 2)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - 2) * LOADS) : "memory");
+    else if (SLOTS > 3 && left == 1)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+
+  template <bool XRMS>
+  __device__ __forceinline__ void run(bf16* ring, const bf16* W, const bf16* X, int64_t N, int64_t M, int64_t K,
+                                      int64_t n0, int64_t m0) {
+    static_assert(SLOTS == 3 || SLOTS == 4, "wait()");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int wn = wave % WN, wm = wave / WN;
+    const int nk = static_cast<int>(K / K_ST);
+    auto clip = [](int64_t b) { return static_cast<int>(b < 0x7fffffffll ? b : 0x7fffffffll); };
+    // one buffer over the pieces: a w row past N is another piece's row or zero, and only feeds columns
+    // past N
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(W + n0 * K), 0, clip((NP * N - n0) * K * 2), BUF_DW3);
+    const __amdgpu_buffer_rsrc_t xrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(X + m0 * K), 0, clip((M - m0) * K * 2), BUF_DW3);
+    // load d of this wave covers stage rows (d NWAVE + wave) 8 ..: the first W_LOADS are w's
+    uint32_t voff[LOADS];
+#pragma unroll
+    for (int d = 0; d < LOADS; ++d) {
+      const int r = (d * NWAVE + wave) * 8 + (lane >> 3);
+      const int64_t rr = r < NP * BN ? r / BN * N + r % BN : r - NP * BN;
+      voff[d] = static_cast<uint32_t>((rr * K + 8 * ((lane & 7) ^ (r & 7))) * 2);
+    }
+    auto issue = [&](int kt) {
+      bf16* dst = ring + (kt % SLOTS) * ROWS * K_ST;
+#pragma unroll
+      for (int d = 0; d < LOADS; ++d) {
+        auto* to = (__attribute__((address_space(3))) void*)(dst + (d * NWAVE + wave) * 8 * K_ST);
+        const uint32_t off = voff[d] + static_cast<uint32_t>(kt) * K_ST * 2;
+        if (d < W_LOADS)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, to, 16, off, 0, 0, 0);
+        else
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, to, 16, off, 0, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < FM; ++j) xss[j] = 0.f;
+    const int rsel = lane & 15, psel = lane >> 4;
+    for (int s = 0; s < SLOTS - 1 && s < nk; ++s) issue(s);
+    for (int kt = 0; kt < nk; ++kt) {
+      wait(nk - 1 - kt);
+      // stage kt has landed for every wave, and every wave has read slot (kt - 1) % SLOTS (no release
+      // fence: it would wait for the stages in flight)
+      __builtin_amdgcn_s_barrier();
+      if (kt + SLOTS - 1 < nk) issue(kt + SLOTS - 1);
+      const bf16* st = ring + (kt % SLOTS) * ROWS * K_ST;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int slot = 8 * ((4 * h + psel) ^ (rsel & 7));
+        bf16x8 b[FM];
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+          b[j] = *reinterpret_cast<const bf16x8*>(st + (NP * BN + wm * (BM / WM) + j * 16 + rsel) * K_ST + slot);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          bf16x8 a[FN];
+#pragma unroll
+          for (int i = 0; i < FN; ++i)
+            a[i] = *reinterpret_cast<const bf16x8*>(st + (p * BN + wn * (BN / WN) + i * 16 + rsel) * K_ST + slot);
+#pragma unroll
+          for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if constexpr (XRMS) {
+#pragma unroll
+          for (int j = 0; j < FM; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const bf16x2 v = {b[j][2 * q], b[j][2 * q + 1]};
+              xss[j] = __builtin_amdgcn_fdot2_f32_bf16(v, v, xss[j], false);
+            }
+        }
+      }
+    }
+    if constexpr (XRMS) {
+#pragma unroll
+      for (int j = 0; j < FM; ++j) {  // the row's other k pieces
+        xss[j] += __shfl_xor(xss[j], 16, 64);
+        xss[j] += __shfl_xor(xss[j], 32, 64);
+      }
+    }
+  }
+};
+
+}  // namespace lng
