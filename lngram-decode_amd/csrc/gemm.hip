@@ -6,7 +6,7 @@
 // The MFMA "A" operand is the weight, so each lane ends up holding 4
 // consecutive output channels of one token: a packed store for plain outputs,
 // and exactly one route's 4 sign bits for the router epilogue.
-// fp32 runs on a VALU tile kernel (the tiny fp32 layer and fp32 routers).
+// fp32 runs on fp32 MFMA tiles; mixed types and odd K on a VALU tile kernel.
 #include "gemm_tile.h"
 
 namespace lng {
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
                                                    int64_t M, int64_t K, int n_tiles, void* __restrict__ out,
                                                    float* __restrict__ logits, void* __restrict__ codes, int codes_dt,
                                                    int64_t routes, float* __restrict__ rowsq, float x_eps) {
-  using G = TileGemm<BN, BM, WN, WM, 1, 3>;
+  using G = TileGemm<bf16, BN, BM, WN, WM, 1, 3>;
   __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
   const int nt = static_cast<int>(blockIdx.x) % n_tiles;
   const int64_t n0 = static_cast<int64_t>(nt) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
@@ -840,6 +840,84 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
       // the partials come in pairs (256 columns): an odd last one has an empty partner
       if (nt == n_tiles - 1 && (n_tiles & 1)) rowsq[static_cast<int64_t>(nt + 1) * M + m0 + threadIdx.x] = 0.f;
     }
+  }
+}
+
+// fp32 on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products and sums): K % 32 == 0.  512 x 128 x
+// 128 takes 3.3 us and 32768 x 256 x 1024 143 us (120 TFLOP/s); the VALU tile below 18.9 and 393 (few
+// blocks, a scalar LDS read for every two FMAs).  Same error against fp64: 2.03e-7 relative at K = 128,
+// 5.74e-7 at K = 1024, over twelve seeds.
+template <int BN, int BM>
+__global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__ W, const float* __restrict__ X,
+                                                       int64_t N, int64_t M, int64_t K, int n_tiles,
+                                                       float* __restrict__ Y) {
+  using G = TileGemm<float, BN, BM, 2, 2, 1, 3>;
+  __shared__ __attribute__((aligned(16))) float ring[G::LDS_ELEMS];
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x % n_tiles) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
+  G g;
+  g.template run<false>(ring, W, X, N, M, K, n0, m0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wn = wave % 2, wm = wave / 2;
+#pragma unroll
+  for (int j = 0; j < G::FM; ++j) {
+    const int64_t m = m0 + wm * (BM / 2) + j * 16 + (lane & 15);
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < G::FN; ++i) {
+      const int64_t n = n0 + wn * (BN / 2) + i * 16 + 4 * (lane >> 4);
+      float* o = Y + m * N + n;
+      if (n + 3 < N && (N & 3) == 0) {
+        *reinterpret_cast<f32x4*>(o) = g.acc[i][j];
+      } else {
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) o[e] = g.acc[i][j][e];
+      }
+    }
+  }
+}
+
+// y = (x . w^T) * rsqrt(mean(x^2) + eps) in fp32 for bf16 x and an fp32 weight split into three bf16
+// pieces (8 + 8 + 8 bits: every product is exact, the sums are fp32); w3 = [3][N][K].
+template <int BN, int BM, int WN, int WM, int SLOTS>
+__global__ __launch_bounds__(64 * WN * WM) void k_gemm_split3(const bf16* __restrict__ w3, const bf16* __restrict__ X,
+                                                              int64_t N, int64_t M, int64_t K, int n_tiles, float eps,
+                                                              float* __restrict__ Y) {
+  using G = TileGemm<bf16, BN, BM, WN, WM, 3, SLOTS>;
+  __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x % n_tiles) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
+  G g;
+  g.template run<true>(ring, w3, X, N, M, K, n0, m0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wn = wave % WN, wm = wave / WN;
+#pragma unroll
+  for (int j = 0; j < G::FM; ++j) {
+    const int64_t m = m0 + wm * (BM / WM) + j * 16 + (lane & 15);
+    const float r = 1.0f / sqrtf(g.xss[j] / static_cast<float>(K) + eps);
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < G::FN; ++i) {
+      const int64_t n = n0 + wn * (BN / WN) + i * 16 + 4 * (lane >> 4);
+      if (n >= N) continue;  // N % 4 == 0
+      f32x4 v = g.acc[i][j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= r;
+      *reinterpret_cast<f32x4*>(Y + m * N + n) = v;
+    }
+  }
+}
+
+// w3[p][n][k]: bf16 pieces of fp32(w[n, k] * s[k]), largest first; a piece past a non-finite one is 0
+__global__ __launch_bounds__(256) void k_split3(const float* __restrict__ w, const float* __restrict__ s, int64_t n,
+                                                int64_t K, bf16* __restrict__ w3) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  float f = w[i] * s[i % K];
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const bf16 b = static_cast<bf16>(f);
+    w3[p * n + i] = b;
+    f -= static_cast<float>(b);
+    if (!(fabsf(f) <= 3.0e38f)) f = 0.f;
   }
 }
 
@@ -1061,8 +1139,25 @@ static int launch_proj(const bf16* w, const bf16* x, int64_t N, int64_t M, int64
   return check_launch("gemm_bf16_proj");
 }
 
+static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N, int64_t K, float* y, hipStream_t s) {
+  auto go = [&](auto* kern, int64_t bn, int64_t bm) {
+    const int n_tiles = static_cast<int>(cdiv(N, bn));
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, x, N, M, K,
+                       n_tiles, y);
+    return check_launch("gemm_f32_tile");
+  };
+  // small tiles while they make few blocks a CU: 584 blocks of 32 x 32 took 18.8 us at 2331 x 256 x 1024
+  // against 24.2 in 64 x 64; 8192 of them 177 us at 32768 x 256 x 1024 against 143 (128 x 64: 138)
+  if (cdiv(N, 32) * cdiv(M, 32) <= 1024) return go(&k_gemm_tile_f32<32, 32>, 32, 32);
+  return go(&k_gemm_tile_f32<64, 64>, 64, 64);
+}
+
 template <typename TA, typename TB, typename TO>
 static int launch_f32(const void* x, const void* w, int64_t M, int64_t N, int64_t K, void* y, hipStream_t s) {
+  if constexpr (sizeof(TA) == 4 && sizeof(TB) == 4 && sizeof(TO) == 4) {
+    if (K % 32 == 0 && N * K * 4 < (int64_t{1} << 31))
+      return launch_tile_f32(static_cast<const float*>(x), static_cast<const float*>(w), M, N, K, static_cast<float*>(y), s);
+  }
   dim3 grid(static_cast<unsigned>(cdiv(N, 64)), static_cast<unsigned>(cdiv(M, 64)));
   hipLaunchKernelGGL((k_gemm_nt_f32<TA, TB, TO>), grid, dim3(256), 0, s, static_cast<const TA*>(x),
                      static_cast<const TB*>(w), M, N, K, static_cast<TO*>(y));
@@ -1128,6 +1223,40 @@ int lng_linear_rowscale(const void* x, const void* w, int64_t M, int64_t N, int6
                                        nullptr, nullptr, 0, 0, nullptr, eps, as_stream(stream));
   return launch_proj(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K, static_cast<bf16*>(y), nullptr,
                      as_stream(stream), true, eps);
+}
+
+static bool split3_shape(int64_t N, int64_t K) {
+  return N > 0 && K > 0 && N % 4 == 0 && K % 64 == 0 && 3 * N * K * 2 < (int64_t{1} << 31);
+}
+size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K) {
+  return split3_shape(N, K) ? static_cast<size_t>(3 * N * K * 2) : 0;
+}
+
+int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t M, int64_t N, int64_t K, float eps,
+                     void* workspace, size_t workspace_bytes, float* y, void* stream) {
+  if (M < 0 || !split3_shape(N, K))
+    return fail(LNG_E_ARG, "linear_split: needs N % 4 == 0 and K % 64 == 0 (lng_linear_split_workspace_bytes)");
+  if (M == 0) return LNG_OK;
+  if (!x || !norm_w || !w || !workspace || !y) return fail(LNG_E_ARG, "linear_split: null buffer");
+  if (workspace_bytes < lng_linear_split_workspace_bytes(N, K)) return fail(LNG_E_ARG, "linear_split: workspace too small");
+  auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (!al(x) || !al(workspace) || !al(y)) return fail(LNG_E_ARG, "linear_split: buffers must be 16-byte aligned");
+  hipStream_t s = as_stream(stream);
+  bf16* w3 = static_cast<bf16*>(workspace);
+  const bf16* xp = static_cast<const bf16*>(x);
+  hipLaunchKernelGGL(k_split3, dim3(static_cast<unsigned>(cdiv(N * K, 256))), dim3(256), 0, s, w, norm_w, N * K, K, w3);
+  auto go = [&](auto* kern, int64_t bn, int64_t bm, int threads) {
+    const int n_tiles = static_cast<int>(cdiv(N, bn));
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(threads), 0, s, w3, xp, N, M, K,
+                       n_tiles, eps, y);
+    return check_launch("linear_split");
+  };
+  // by blocks, as pick_tile (N 256, K 1024, the split included; us):  M  200  2048  4096  8192  32768
+  //   32 x 32 9.1 12.4 19.1 30.6 112;  64 x 64 15.2 15.7 17.0 20.9 68.5;  64 x 128 18.6 18.4 19.8 20.9 61.0
+  // norm pass, fp32 copy and VALU product before: 165 190 193 216 474
+  if (cdiv(N, 32) * cdiv(M, 32) <= 768) return go(&k_gemm_split3<32, 32, 2, 2, 3>, 32, 32, 256);
+  if (cdiv(N, 64) * cdiv(M, 64) <= 512) return go(&k_gemm_split3<64, 64, 2, 2, 2>, 64, 64, 256);
+  return go(&k_gemm_split3<64, 128, 2, 4, 2>, 64, 128, 512);
 }
 
 int lng_linear(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, void* y, void* stream) {

@@ -1,22 +1,25 @@
-// bf16 GEMM tiles for the row counts between the skinny kernel and the one-tile-per-CU kernels.
+// GEMM tiles: bf16 projections between the skinny kernel's rows and the one-tile-per-CU kernels', bf16
+// rows against fp32 weights split into bf16 pieces, and fp32.
 //
-// y[m, n] = sum_k x[m, k] * w[n, k]: a block of 4 waves computes BN (w rows) x BM (x rows), wave
-// (wn, wm) of the WN x WM grid its BN/WN x BM/WM part in 16x16x32 fragments, accumulating in K order
-// (per output the same instructions as the other bf16 kernels, so equal results).  K advances 64 a
-// stage through a ring of SLOTS LDS stages filled by buffer loads straight into LDS; rows past N or M
-// lie outside the buffers and read as zero.  Piece p (16 bytes) of row r sits in slot p ^ (r & 7): the
-// operand reads are free of bank conflicts.  NP > 1: w is NP consecutive [N, K] matrices whose products
-// with the same x rows add up (an fp32 weight's bf16 pieces).
+// y[m, n] = sum_k x[m, k] * w[n, k]: a block of WN x WM waves computes BN (w rows) x BM (x rows), wave
+// (wn, wm) its BN/WN x BM/WM part in 16x16 fragments, accumulating in one K order whatever the tile
+// (bf16: 16x16x32 products in K order, as the other bf16 kernels, so equal results; fp32: 16x16x4
+// products, four of every 16 k apart).  K advances 128 bytes a stage through a ring of SLOTS LDS stages
+// filled by buffer loads straight into LDS; rows past N or M lie outside the buffers and read as zero.
+// Piece p (16 bytes) of row r sits in slot p ^ (r & 7): the operand reads are free of bank conflicts.
+// NP > 1: w is NP consecutive [N, K] matrices whose products with the same x rows add up.
 #pragma once
 
 #include "common.h"
 
 namespace lng {
 
-template <int BN, int BM, int WN, int WM, int NP, int SLOTS>
+template <typename T, int BN, int BM, int WN, int WM, int NP, int SLOTS>
 struct TileGemm {
   static constexpr int NWAVE = WN * WM, NT = 64 * NWAVE;
-  static constexpr int K_ST = 64;
+  static constexpr int K_ST = 128 / sizeof(T);          // k of a stage: 64 bf16 or 32 fp32
+  static constexpr int PE = 16 / sizeof(T);             // elements of a piece
+  typedef T Frag __attribute__((ext_vector_type(PE)));  // an operand lane's share of 4 pieces' k
   static constexpr int ROWS = NP * BN + BM;             // LDS rows of a stage, the w pieces first
   static constexpr int FN = BN / WN / 16, FM = BM / WM / 16;
   static constexpr int LOADS = ROWS / 8 / NWAVE;        // 8 rows an instruction
@@ -27,6 +30,16 @@ struct TileGemm {
 
   f32x4 acc[FN][FM];
   float xss[FM];  // XRMS: this lane's share of the sum of squares of x row 16 j + (lane & 15)
+
+  __device__ __forceinline__ static f32x4 mma(Frag a, Frag b, f32x4 c) {
+    if constexpr (sizeof(T) == 2) {
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < PE; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+      return c;
+    }
+  }
 
   // waits until at most `left` later stages of this wave's loads are in flight
   __device__ __forceinline__ static void wait(int left) {
@@ -39,9 +52,10 @@ struct TileGemm {
   }
 
   template <bool XRMS>
-  __device__ __forceinline__ void run(bf16* ring, const bf16* W, const bf16* X, int64_t N, int64_t M, int64_t K,
-                                      int64_t n0, int64_t m0) {
-    static_assert(SLOTS == 3 || SLOTS == 4, "wait()");
+  __device__ __forceinline__ void run(T* ring, const T* W, const T* X, int64_t N, int64_t M, int64_t K, int64_t n0,
+                                      int64_t m0) {
+    static_assert(SLOTS >= 2 && SLOTS <= 4, "wait()");
+    constexpr int ES = sizeof(T);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     const int wn = wave % WN, wm = wave / WN;
     const int nk = static_cast<int>(K / K_ST);
@@ -49,23 +63,23 @@ struct TileGemm {
     // one buffer over the pieces: a w row past N is another piece's row or zero, and only feeds columns
     // past N
     const __amdgpu_buffer_rsrc_t wrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(W + n0 * K), 0, clip((NP * N - n0) * K * 2), BUF_DW3);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(W + n0 * K), 0, clip((NP * N - n0) * K * ES), BUF_DW3);
     const __amdgpu_buffer_rsrc_t xrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(X + m0 * K), 0, clip((M - m0) * K * 2), BUF_DW3);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(X + m0 * K), 0, clip((M - m0) * K * ES), BUF_DW3);
     // load d of this wave covers stage rows (d NWAVE + wave) 8 ..: the first W_LOADS are w's
     uint32_t voff[LOADS];
 #pragma unroll
     for (int d = 0; d < LOADS; ++d) {
       const int r = (d * NWAVE + wave) * 8 + (lane >> 3);
       const int64_t rr = r < NP * BN ? r / BN * N + r % BN : r - NP * BN;
-      voff[d] = static_cast<uint32_t>((rr * K + 8 * ((lane & 7) ^ (r & 7))) * 2);
+      voff[d] = static_cast<uint32_t>((rr * K + PE * ((lane & 7) ^ (r & 7))) * ES);
     }
     auto issue = [&](int kt) {
-      bf16* dst = ring + (kt % SLOTS) * ROWS * K_ST;
+      T* dst = ring + (kt % SLOTS) * ROWS * K_ST;
 #pragma unroll
       for (int d = 0; d < LOADS; ++d) {
         auto* to = (__attribute__((address_space(3))) void*)(dst + (d * NWAVE + wave) * 8 * K_ST);
-        const uint32_t off = voff[d] + static_cast<uint32_t>(kt) * K_ST * 2;
+        const uint32_t off = voff[d] + static_cast<uint32_t>(kt) * 128;
         if (d < W_LOADS)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, to, 16, off, 0, 0, 0);
         else
@@ -86,24 +100,24 @@ struct TileGemm {
       // fence: it would wait for the stages in flight)
       __builtin_amdgcn_s_barrier();
       if (kt + SLOTS - 1 < nk) issue(kt + SLOTS - 1);
-      const bf16* st = ring + (kt % SLOTS) * ROWS * K_ST;
+      const T* st = ring + (kt % SLOTS) * ROWS * K_ST;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int slot = 8 * ((4 * h + psel) ^ (rsel & 7));
-        bf16x8 b[FM];
+        const int slot = PE * ((4 * h + psel) ^ (rsel & 7));
+        Frag b[FM];
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-          b[j] = *reinterpret_cast<const bf16x8*>(st + (NP * BN + wm * (BM / WM) + j * 16 + rsel) * K_ST + slot);
+          b[j] = *reinterpret_cast<const Frag*>(st + (NP * BN + wm * (BM / WM) + j * 16 + rsel) * K_ST + slot);
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-          bf16x8 a[FN];
+          Frag a[FN];
 #pragma unroll
           for (int i = 0; i < FN; ++i)
-            a[i] = *reinterpret_cast<const bf16x8*>(st + (p * BN + wn * (BN / WN) + i * 16 + rsel) * K_ST + slot);
+            a[i] = *reinterpret_cast<const Frag*>(st + (p * BN + wn * (BN / WN) + i * 16 + rsel) * K_ST + slot);
 #pragma unroll
           for (int i = 0; i < FN; ++i)
 #pragma unroll
-            for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < FM; ++j) acc[i][j] = mma(a[i], b[j], acc[i][j]);
         }
         if constexpr (XRMS) {
 #pragma unroll

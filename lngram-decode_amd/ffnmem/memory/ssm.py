@@ -41,8 +41,7 @@ class DiagonalSSM(nn.Module):
 
     def inputs(self, emb: Tensor) -> Tensor:
         """``u[t]`` in fp32: ``[B, T, d]`` -> ``[B, T, N]`` (``ssm.py:41-43``)."""
-        x = emb.float()
-        return ops.linear(ops.rmsnorm(x, self.norm.weight.float(), self.norm.eps), self.w_in.weight.float())
+        return ops.norm_linear_fp32(emb, self.norm.weight, self.w_in.weight, self.norm.eps)
 
     def forward(self, emb: Tensor) -> Tensor:
         return chunked_scan(self.decay(), self.inputs(emb), self.chunk)

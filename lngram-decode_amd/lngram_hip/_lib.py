@@ -92,6 +92,8 @@ SIGNATURES = {
                                       _p, _p]),
     "lng_linear_rowsq_partials": (_i32, [_i64]),
     "lng_linear_rowsq": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p]),
+    "lng_linear_split_workspace_bytes": (ctypes.c_size_t, [_i64, _i64]),
+    "lng_linear_split": (_int, [_p, _p, _p, _i64, _i64, _i64, _f, _p, ctypes.c_size_t, _p, _p]),
     "lng_linear_rowscale_ok": (_i32, [_i64, _i64, _i64]),
     "lng_linear_rowscale": (_int, [_p, _p, _i64, _i64, _i64, _f, _p, _p]),
     "lng_row_sumsq": (_int, [_p, _i64, _i32, _p, _p]),
