@@ -413,6 +413,35 @@ int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t grad_stride,
                     void* workspace, size_t workspace_bytes, void* grad_q, int out_dtype, void* grad_table2,
                     void* grad_table3, void* stream);
 
+/* ---------------------------------------------------------------- the layer's launches in one call */
+/* One memory layer (RouteNgramMemoryV2, lngram_v2.py:842-1010) in one dtype (bf16 or f32): shapes and
+ * device pointers of its weights, contiguous and 16-byte aligned.  fused: the shape of
+ * lng_memory_readout_fused, w_q then being readout_q_proj.weight with the query norm folded in
+ * (lng_fold_columns) and kv the packed key/value weight (lng_memory_readout_pack). */
+typedef struct lng_memory_layer {
+  int32_t hidden, routes, bits, n_orders;
+  int32_t orders[4];
+  int32_t mem_dim, q_heads, kv_heads, head_dim, conv_k, conv_dilation, dtype, fused;
+  float q_eps, mem_eps, conv_eps, scale, sink_logit;
+  const void *w_q, *q_norm, *tables[4], *kv, *mem_norm, *w_o, *conv_norm, *conv_w;
+} lng_memory_layer;
+size_t lng_memory_layer_size(void);
+
+/* RouteNgramMemoryV2.forward without segments and valid tokens (lngram_v2.py:1361-1407), from the route
+ * codes [B, T, R] (uint8 where fused): query projection, lookup and sink readout, output projection
+ * and short conv, by the entry points above.  h, out [B, T, hidden]. */
+size_t lng_memory_forward_workspace_bytes(const lng_memory_layer* layer, int64_t B, int64_t T);
+int lng_memory_forward(const lng_memory_layer* layer, const void* h, const void* codes, int codes_dtype, int64_t B,
+                       int64_t T, void* workspace, size_t workspace_bytes, void* out, void* stream);
+
+/* memory_step (ffnmem/infer.py:152-182) of a fused layer for B * n <= 64 new positions at pos0: their
+ * codes [B, n, R] into code_cache [B, max_len, R], the readout over the cache, the output projection
+ * into conv_cache [B, max_len, hidden] and the conv over its window.  The workspace holds two
+ * [B * n, hidden] buffers (each rounded up to 256 bytes). */
+int lng_memory_step(const lng_memory_layer* layer, const void* h, const void* codes, int codes_dtype, int64_t B,
+                    int64_t n, int64_t pos0, uint8_t* code_cache, void* conv_cache, int64_t max_len, void* workspace,
+                    size_t workspace_bytes, void* out, void* stream);
+
 /* ---------------------------------------------------------------- serving layout and host-RAM rows */
 /* Device address of pinned host memory (hipHostGetDevicePointer): the serving movers below read
  * host-RAM tables through it (zero-copy over the host link).  LNG_E_HIP for memory that is not

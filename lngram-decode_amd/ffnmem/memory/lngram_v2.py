@@ -496,6 +496,10 @@ class _RouteNgramMemoryBase(nn.Module):
         return self.short_conv.forward_residual(mixed)
 
     # ------------------------------------------------------------------ fused path
+    # Layers whose intermediates fit this run as one call (lng_memory_forward); past it the host's share
+    # of a layer is small and the op-by-op form frees each intermediate as it goes.
+    _NATIVE_WORKSPACE = 64 << 20
+
     def _fused_shape_ok(self, hidden_states: Tensor, tables: bool = True) -> bool:
         """Whether the fused readout serves this layer (``tables``: reading its own tables, which
         must then be on the device, not offloaded)."""
@@ -527,6 +531,42 @@ class _RouteNgramMemoryBase(nn.Module):
             self._fused_cache = (key, ops.memory_readout_pack(w.detach()))
         return self._fused_cache[1]
 
+    def _native_layer(self, dtype: torch.dtype, device: torch.device, fused: bool):
+        """``lng_memory_layer`` of this layer, or None where its forward is not the launches of
+        ``lng_memory_forward`` (a subclass, hooks on the norms that the op-by-op form calls as modules,
+        weights of other types, devices or layouts, launches being timed one by one).  Built per call
+        from the current parameters."""
+        if type(self) is not RouteNgramMemoryV2 or ops.KernelTimer._active:
+            return None
+        mods = self._modules
+        conv = mods["short_conv"]
+        norms = (mods["readout_query_norm"], mods["readout_memory_norm"])
+        try:
+            wq, qn = mods["readout_q_proj"]._parameters["weight"], norms[0]._parameters["weight"]
+            kv, mn = mods["readout_kv_proj"]._parameters["weight"], norms[1]._parameters["weight"]
+            wo = mods["readout_o_proj"]._parameters["weight"]
+            cn = conv._modules["norm"]._parameters["weight"]
+            cw, bias = conv._modules["conv"]._parameters["weight"], conv._modules["conv"]._parameters["bias"]
+            tables = [mods["tables"]._modules[f"ngram_{n}"]._parameters["weight"] for n in self.ngrams]
+        except KeyError:                                   # a parametrised weight
+            return None
+        if bias is not None or len(tables) > 4 or any(x is None for x in (wq, qn, kv, mn, wo, cn, cw, *tables)):
+            return None
+        if not fused and (torch.nn.modules.module._has_any_global_hook()
+                          or any(n._forward_hooks or n._forward_pre_hooks or type(n) is not RMSNorm for n in norms)):
+            return None
+        if fused:
+            wq, kv = self._folded_query_weight(), self._fused_weights()
+        return ops.memory_layer(
+            dtype, device,
+            {"hidden": self.hidden_size, "routes": self.num_routes, "bits": self.bits_per_route, "orders": self.ngrams,
+             "mem_dim": self.memory_dim, "q_heads": self.readout_num_heads, "kv_heads": self.readout_num_kv_heads,
+             "head_dim": self.readout_head_dim, "conv_k": conv.kernel_size, "conv_dilation": conv.dilation,
+             "fused": int(fused)},
+            {"q_eps": norms[0].eps, "mem_eps": norms[1].eps, "conv_eps": conv._modules["norm"].eps,
+             "scale": self.softmax_scale, "sink_logit": self.readout_sink_logit},
+            tables, {"w_q": wq, "q_norm": qn, "kv": kv, "mem_norm": mn, "w_o": wo, "conv_norm": cn, "conv_w": cw})
+
     def forward(self, hidden_states: Tensor, route_codes_btr: Tensor, q_logits: Optional[Tensor] = None,
                 segment_ids: Optional[Tensor] = None, valid_tokens: Optional[Tensor] = None) -> Tensor:
         """``RouteNgramMemoryV2.forward`` (``lngram_v2.py:1361-1407``), eval.
@@ -547,7 +587,18 @@ class _RouteNgramMemoryBase(nn.Module):
                 raise ValueError(f"q_logits shape={tuple(q_logits.shape)}, expected {expected}")
             q_btrm = q_logits.reshape(b, t, self.num_routes, self.bits_per_route)
         self._check_inference(q_btrm)
-        if segment_ids is None and valid_tokens is None and self._fused_shape_ok(hidden_states):
+        plain = segment_ids is None and valid_tokens is None
+        fused = plain and self._fused_shape_ok(hidden_states)
+        if plain and b * t and self.bits_per_route <= 8 and hidden_states.is_cuda and \
+                hidden_states.dtype in (torch.bfloat16, torch.float32):
+            layer = self._native_layer(hidden_states.dtype, hidden_states.device, fused)
+            if layer is not None:
+                out = ops.memory_forward(layer, hidden_states,
+                                         route_codes_btr.to(torch.uint8) if fused else route_codes_btr,
+                                         self._NATIVE_WORKSPACE)
+                if out is not None:
+                    return out
+        if fused:
             # the query RMSNorm's weight is folded into the projection and its row scale applied in
             # the readout kernel, so the normalised hidden states are never written out
             kv_pack = self._fused_weights()

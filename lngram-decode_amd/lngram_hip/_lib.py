@@ -62,6 +62,21 @@ class Sketch(ctypes.Structure):
 
 _PS = ctypes.POINTER(Sketch)
 
+
+class MemoryLayer(ctypes.Structure):
+    """``lng_memory_layer`` (include/lngram_hip.h): one memory layer's shapes and weights."""
+
+    _fields_ = [(n, ctypes.c_int32) for n in ("hidden", "routes", "bits", "n_orders")] + [
+        ("orders", ctypes.c_int32 * 4)] + [
+        (n, ctypes.c_int32) for n in ("mem_dim", "q_heads", "kv_heads", "head_dim", "conv_k", "conv_dilation", "dtype",
+                                      "fused")] + [
+        (n, ctypes.c_float) for n in ("q_eps", "mem_eps", "conv_eps", "scale", "sink_logit")] + [
+        ("w_q", ctypes.c_void_p), ("q_norm", ctypes.c_void_p), ("tables", ctypes.c_void_p * 4)] + [
+        (n, ctypes.c_void_p) for n in ("kv", "mem_norm", "w_o", "conv_norm", "conv_w")]
+
+
+_PL = ctypes.POINTER(MemoryLayer)
+
 # name -> (restype, argtypes); must cover every function declared in the header
 SIGNATURES = {
     "lng_abi_version": (_int, []),
@@ -120,6 +135,10 @@ SIGNATURES = {
     "lng_lookup_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32, _int, _int]),
     "lng_lookup_grad": (_int, [_p, _int, _i64, _p, _int, _p, _int, _p, _p, _i64, _i64, _p, _p, _i64, _i64, _i32, _i32,
                                _i32, _i32, _f, _f, _p, ctypes.c_size_t, _p, _int, _p, _p, _p]),
+    "lng_memory_layer_size": (ctypes.c_size_t, []),
+    "lng_memory_forward_workspace_bytes": (ctypes.c_size_t, [_PL, _i64, _i64]),
+    "lng_memory_forward": (_int, [_PL, _p, _p, _int, _i64, _i64, _p, ctypes.c_size_t, _p, _p]),
+    "lng_memory_step": (_int, [_PL, _p, _p, _int, _i64, _i64, _i64, _p, _p, _i64, _p, ctypes.c_size_t, _p, _p]),
     "lng_host_device_pointer": (_int, [_p, ctypes.POINTER(_p)]),
     "lng_permute_table": (_int, [_p, _p, _int, _i32, _i32, _i32, _i32, _p]),
     "lng_serving_address": (_int, [_p, _int, _i64, _i64, _i32, _i32, _i32, _p, _p]),

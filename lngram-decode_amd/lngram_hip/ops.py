@@ -28,18 +28,18 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def _dev(*ts) -> torch.device:
-    dev = None
+    first = None
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError("lngram_hip ops need tensors on a ROCm GPU device; there is no CPU path "
                                f"(got a tensor on {t.device})")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
-    return dev
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} vs {t.device}")
+    return None if first is None else first.device
 
 
 def _stream(dev: torch.device) -> int:
@@ -58,11 +58,17 @@ def _c(t: torch.Tensor | None) -> torch.Tensor | None:
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_LIB = None
 
 
 def lib():
-    return _lib.load()
+    global _LIB
+    if _LIB is None:
+        _LIB = _lib.load()
+    return _LIB
 
 
 class KernelTimer:
@@ -104,6 +110,8 @@ class KernelTimer:
 
 
 def _timed(name: str, dev: torch.device, launch):
+    if not KernelTimer._active:
+        return launch()
     timers = []
     for t in KernelTimer._active:
         if name in t.names:
@@ -327,6 +335,64 @@ def route_tokens(codes: torch.Tensor, tables, orders, bits: int, route_start: in
     check(lib().lng_route_tokens(_ptr(cc), dtype_code(cc.dtype), b, t, r, route_start, route_end, _orders(orders),
                                  len(orders), bits, tp, dtype_code(dt), mem_dim, _ptr(seg), _ptr(val),
                                  int(target_length or 0), _ptr(out), _stream(dev)), "route_tokens")
+    return out
+
+
+# ----------------------------------------------------------------------------- the layer in one call
+def memory_layer(dtype: torch.dtype, device: torch.device, shape: dict, floats: dict, tables, weights: dict):
+    """``lng_memory_layer`` of a layer whose weights are all ``dtype`` on ``device``, contiguous and 16-byte
+    aligned; None when one is not.  The tensors have to outlive the calls that take it."""
+    L = _lib.MemoryLayer()
+    for t in (*tables, *weights.values()):
+        if t.dtype != dtype or t.device != device or not t.is_contiguous() or t.data_ptr() % 16:
+            return None
+    for k, v in weights.items():
+        setattr(L, k, v.data_ptr())
+    for i, t in enumerate(tables):
+        L.tables[i] = t.data_ptr()
+    for k, v in shape.items():
+        if k == "orders":
+            for i, o in enumerate(v):
+                L.orders[i] = o
+            L.n_orders = len(v)
+        else:
+            setattr(L, k, v)
+    for k, v in floats.items():
+        setattr(L, k, v)
+    L.dtype = dtype_code(dtype)
+    return L
+
+
+def memory_forward(layer, h: torch.Tensor, codes: torch.Tensor, max_workspace: int):
+    """The layer's output ``[B, T, hidden]`` (``lng_memory_forward``), or None when the intermediates
+    take more than ``max_workspace`` bytes."""
+    dev = _dev(h, codes)
+    b, t, _ = h.shape
+    L = ctypes.byref(layer)
+    nws = lib().lng_memory_forward_workspace_bytes(L, b, t)
+    if not 0 < nws <= max_workspace:
+        return None
+    hc, cc = _c(h), _codes_ok(codes)
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    out = torch.empty(h.shape, dtype=h.dtype, device=dev)
+    check(lib().lng_memory_forward(L, _ptr(hc), _ptr(cc), dtype_code(cc.dtype), b, t, _ptr(ws), nws, _ptr(out),
+                                   _stream(dev)), "memory_forward")
+    return out
+
+
+def memory_step(layer, h: torch.Tensor, codes: torch.Tensor, pos0: int, code_cache: torch.Tensor,
+                conv_cache: torch.Tensor) -> torch.Tensor:
+    """The cached step's output ``[B, n, hidden]`` (``lng_memory_step``): ``codes [B, n, R]`` into
+    ``code_cache`` and the projected rows into ``conv_cache`` at ``pos0`` on."""
+    dev = _dev(h, codes, code_cache, conv_cache)
+    b, n, d = h.shape
+    hc, cc = _c(h), _codes_ok(codes)
+    nws = 2 * (-(-b * n * d * h.element_size() // 256) * 256)
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    out = torch.empty(h.shape, dtype=h.dtype, device=dev)
+    check(lib().lng_memory_step(ctypes.byref(layer), _ptr(hc), _ptr(cc), dtype_code(cc.dtype), b, n, int(pos0),
+                                _ptr(code_cache), _ptr(conv_cache), code_cache.shape[1], _ptr(ws), nws, _ptr(out),
+                                _stream(dev)), "memory_step")
     return out
 
 
