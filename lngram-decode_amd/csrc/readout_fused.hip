@@ -19,6 +19,9 @@
 // read back as the score MFMA's A operand (ds_read_b128) and, transposed, as the
 // B operand of P.X (ds_read_b64_tr_b16).  The next chunk's rows are in flight while a
 // chunk is processed.
+//
+// Few tokens (decode steps, draft trees, short prompts, the remainder of a large launch) run one token
+// a block with its route chunks split over the waves (readout_body<.., true>): see readout_launch.
 #include "common.h"
 
 namespace lng {
@@ -88,23 +91,30 @@ __device__ __forceinline__ float sumsq8(const bf16x8 v, float acc) {
 // 32-row region reused as qkw (rows 0..15, phase A -> B), the route chunk (rows 0..31, phase B)
 // and u (rows 0..15, phase B -> C); per wave the token's row indices [order][route parity]
 // [route / 2] (-1 = zero row); the memory-norm weight.
+//
+// SPLIT: the block's FR_TOK waves share one token (tok0), wave w taking route chunks w, w + FR_TOK, ..;
+// their softmax states and weighted sums are merged in LDS before phase C.
 template <int FR_TOK>
-__global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const bf16* __restrict__ q,
-                                                          const bf16* __restrict__ q_rows, float q_eps,
-                                                          const uint8_t* __restrict__ codes,
-                                                          int64_t B, int64_t T, int32_t R, int64_t cstride,
-                                                          int64_t pos0, const int32_t* __restrict__ pos0_dev,
-                                                          const bf16* __restrict__ table2,
-                                                          const bf16* __restrict__ table3,
-                                                          const bf16* __restrict__ kv_pack,
-                                                          const bf16* __restrict__ w_mem, float eps, float scale,
-                                                          float sink, bf16* __restrict__ head_out) {
-  __shared__ __attribute__((aligned(16))) bf16 xs_lds[FR_TOK * FR_TS];
-  __shared__ __attribute__((aligned(16))) int32_t rowsh[FR_TOK][2][4][FR_RQ + 4];  // rows 272 B apart
+struct ReadoutLds {
+  __attribute__((aligned(16))) bf16 xs[FR_TOK * FR_TS];
+  __attribute__((aligned(16))) int32_t rowsh[FR_TOK][2][4][FR_RQ + 4];  // rows 272 B apart
+  __attribute__((aligned(16))) bf16 wms[FR_DT];
+  float qscale[FR_TOK];
+};
+
+template <int FR_TOK, bool SPLIT>
+__device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t tok0, const bf16* __restrict__ q,
+                                             const bf16* __restrict__ q_rows, float q_eps,
+                                             const uint8_t* __restrict__ codes, int64_t B, int64_t T, int32_t R,
+                                             int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
+                                             const bf16* __restrict__ table2, const bf16* __restrict__ table3,
+                                             const bf16* __restrict__ kv_pack, const bf16* __restrict__ w_mem,
+                                             float eps, float scale, float sink, bf16* __restrict__ head_out) {
+  auto& rowsh = lds.rowsh;
+  auto& wms = lds.wms;
+  auto& qscale = lds.qscale;
   // element (row, c) of token t's region (see fr_tok)
-  auto XS = [&](int t, int row, int c) -> bf16& { return xs_lds[fr_tok(t) + row * FR_LD + c]; };
-  __shared__ __attribute__((aligned(16))) bf16 wms[FR_DT];
-  __shared__ float qscale[FR_TOK];
+  auto XS = [&](int t, int row, int c) -> bf16& { return lds.xs[fr_tok(t) + row * FR_LD + c]; };
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
   if (threadIdx.x < FR_DT) wms[threadIdx.x] = w_mem[threadIdx.x];
@@ -113,7 +123,7 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
   // reduces the row of token w (2 KB, two 16 B pieces per lane)
   const int64_t ntok_all = B * T;
   bf16x8 hq[2];
-  const int64_t tq_own = static_cast<int64_t>(blockIdx.x) * FR_TOK + w;
+  const int64_t tq_own = SPLIT ? tok0 : tok0 + w;
   if (q_rows) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -122,15 +132,16 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
 
   // phase-A operands first (no dependence on the codes), so their latency overlaps stage 0:
   // wave w takes head h = w & 3 and feature tiles ft0 .. ft0 + NFT-1; column tile tt = tokens 4tt .. 4tt+3
-  constexpr int NTT = FR_TOK / 4, NFT = 16 / NTT, NDT = 4 / NTT;
+  constexpr int NTT = SPLIT ? 1 : FR_TOK / 4, NFT = 64 / FR_TOK, NDT = 16 / FR_TOK;
   const int a_h = w & 3, a_ft0 = NFT * (w >> 2), a_hg = a_h * 4 + (li & 3);
   bf16x8 bq[NTT][2], wa[NFT][2];
 #pragma unroll
   for (int tt = 0; tt < NTT; ++tt) {
-    const int64_t tq = static_cast<int64_t>(blockIdx.x) * FR_TOK + 4 * tt + (li >> 2);
+    const int64_t tq = tok0 + 4 * tt + (li >> 2);
+    const bool own = SPLIT ? li < 4 : tq < B * T;  // split: the other columns stay zero
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-      bq[tt][ks] = tq < B * T ? ldq(q, tq * (FR_H * FR_HD) + a_hg * FR_HD + 32 * ks + 8 * lg) : zero8();
+      bq[tt][ks] = own ? ldq(q, tq * (FR_H * FR_HD) + a_hg * FR_HD + 32 * ks + 8 * lg) : zero8();
   }
 #pragma unroll
   for (int ft = 0; ft < NFT; ++ft)
@@ -138,8 +149,7 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
     for (int ks = 0; ks < 2; ++ks)
       wa[ft][ks] = ld16(kv_pack + (((a_h * 16 + a_ft0 + ft) * 2 + ks) * 64 + lane) * 8);
   const int64_t ntok = B * T;
-  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * FR_TOK;
-  const int64_t tok = tok0 + w;
+  const int64_t tok = SPLIT ? tok0 : tok0 + w;
   const bool tok_ok = tok < ntok;
   // token (b, i) of the B x T outputs sits at position pos0 (+ *pos0_dev) + i of its sequence; its
   // codes at position t are codes[(b * cstride + t) * R ..] (cstride = T, pos0 = 0: a whole
@@ -234,8 +244,10 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
       *reinterpret_cast<u32x4*>(&XS(w, 4 * (m >> 1) + g_sub, (m & 1) * 128 + 8 * g_piece)) = g[m];
   };
 
+  constexpr int C_STEP = SPLIT ? 32 * FR_TOK : 32;
+  const int c_first = SPLIT ? 32 * w : 0;
   u32x4 g[16];
-  gather(0, g);  // first chunk in flight during phase A
+  if (!SPLIT || c_first < R) gather(c_first, g);  // first chunk in flight during phase A
 
   if (q_rows) {
     const float ss = wave_sum(sumsq8(hq[1], sumsq8(hq[0], 0.f)));
@@ -267,18 +279,19 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
   // ---------------- phase B: one token per wave
   bf16x8 qb[8];
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) qb[kk] = *reinterpret_cast<const bf16x8*>(&XS(w, li, fr_col(lg, kk)));
+  for (int kk = 0; kk < 8; ++kk) qb[kk] = *reinterpret_cast<const bf16x8*>(&XS(SPLIT ? 0 : w, li, fr_col(lg, kk)));
+  if (SPLIT) __syncthreads();  // every wave has the query before wave 0's rows replace it
 
   float m_run = sink, l_part = 0.f;
   f32x4 acc[16];
 #pragma unroll
   for (int ft = 0; ft < 16; ++ft) acc[ft] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int c0 = 0; c0 < R; c0 += 32) {
+  for (int c0 = c_first; c0 < R; c0 += C_STEP) {
     stash(g);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    if (c0 + 32 < R) gather(c0 + 32, g);
+    if (c0 + C_STEP < R) gather(c0 + C_STEP, g);
 
     // scores: A = route rows (lane: route 16tt + li, features fr_col(lg, kk) ..+8), B = qkw
     float sr[2];
@@ -367,17 +380,57 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
   // normalise and stage u = w_mem . U / l for the value projection
   float lt = l_part + __shfl_xor(l_part, 16, 64);
   lt += __shfl_xor(lt, 32, 64);
-  lt += __builtin_amdgcn_exp2f((sink - m_run) * 1.4426950408889634f);
-  const float inv = 1.0f / lt;
-  float iD[4];
+  if constexpr (SPLIT) {
+    // head li's (m, l) of every wave (every m is at least the sink), then each wave's sums scaled to
+    // the common maximum and total, as [head][256] fp32 in its region, are added up
+    float2* ml = reinterpret_cast<float2*>(&rowsh[0][0][0][0]);  // the row indices are spent
+    __syncthreads();
+    if (lg == 0) ml[w * 16 + li] = float2{m_run, lt};
+    __syncthreads();
+    float m_all = sink;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) iD[i] = __shfl(inv, 4 * lg + i, 64);
+    for (int k = 0; k < FR_TOK; ++k) m_all = fmaxf(m_all, ml[k * 16 + li].x);
+    float l_all = __builtin_amdgcn_exp2f((sink - m_all) * 1.4426950408889634f);
 #pragma unroll
-  for (int ft = 0; ft < 16; ++ft) {
-    const int f = 16 * ft + li;
+    for (int k = 0; k < FR_TOK; ++k)
+      l_all += ml[k * 16 + li].y * __builtin_amdgcn_exp2f((ml[k * 16 + li].x - m_all) * 1.4426950408889634f);
+    const float fac = __builtin_amdgcn_exp2f((m_run - m_all) * 1.4426950408889634f) / l_all;
+    float fD[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fD[i] = __shfl(fac, 4 * lg + i, 64);
+    float* mine = reinterpret_cast<float*>(&XS(w, 0, 0));  // 16 rows of 272 fp32: the region's 32 x 544 B
+#pragma unroll
+    for (int ft = 0; ft < 16; ++ft)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[(4 * lg + i) * 272 + 16 * ft + li] = acc[ft][i] * fD[i];
+    __syncthreads();
+    // a thread: one feature of 64 / FR_TOK heads
+    constexpr int NH = 64 / FR_TOK;
+    const int f = threadIdx.x & 255, h0 = (threadIdx.x >> 8) * NH;
+    float u[NH];
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) {
+      u[hd] = 0.f;
+#pragma unroll
+      for (int k = 0; k < FR_TOK; ++k) u[hd] += reinterpret_cast<const float*>(&XS(k, 0, 0))[(h0 + hd) * 272 + f];
+    }
+    __syncthreads();
     const float wm = to_f32(wms[f]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) XS(w, 4 * lg + i, f) = static_cast<bf16>(acc[ft][i] * iD[i] * wm);
+    for (int hd = 0; hd < NH; ++hd) XS(0, h0 + hd, f) = static_cast<bf16>(u[hd] * wm);
+  } else {
+    lt += __builtin_amdgcn_exp2f((sink - m_run) * 1.4426950408889634f);
+    const float inv = 1.0f / lt;
+    float iD[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) iD[i] = __shfl(inv, 4 * lg + i, 64);
+#pragma unroll
+    for (int ft = 0; ft < 16; ++ft) {
+      const int f = 16 * ft + li;
+      const float wm = to_f32(wms[f]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) XS(w, 4 * lg + i, f) = static_cast<bf16>(acc[ft][i] * iD[i] * wm);
+    }
   }
   __syncthreads();
 
@@ -394,7 +447,7 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
       f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt][ks], ub[ks], d, 0, 0, 0);
-      if (tc < ntok) {
+      if (SPLIT ? li < 4 : tc < ntok) {
         bf16x4 o;
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = static_cast<bf16>(d[i]);
@@ -402,6 +455,38 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(const
       }
     }
   }
+}
+
+// Blocks 0 .. full_blocks - 1 take FR_TOK tokens each, the others one token each (SPLIT).
+template <int FR_TOK>
+__global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(
+    const bf16* __restrict__ q, const bf16* __restrict__ q_rows, float q_eps, const uint8_t* __restrict__ codes,
+    int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
+    const bf16* __restrict__ table2, const bf16* __restrict__ table3, const bf16* __restrict__ kv_pack,
+    const bf16* __restrict__ w_mem, float eps, float scale, float sink, bf16* __restrict__ head_out,
+    uint32_t full_blocks) {
+  __shared__ ReadoutLds<FR_TOK> lds;
+  if constexpr (FR_TOK == 4) {
+    if (blockIdx.x >= full_blocks) {
+      readout_body<FR_TOK, true>(lds, static_cast<int64_t>(full_blocks) * FR_TOK + (blockIdx.x - full_blocks), q, q_rows,
+                                 q_eps, codes, B, T, R, cstride, pos0, pos0_dev, table2, table3, kv_pack, w_mem, eps,
+                                 scale, sink, head_out);
+      return;
+    }
+  }
+  readout_body<FR_TOK, false>(lds, static_cast<int64_t>(blockIdx.x) * FR_TOK, q, q_rows, q_eps, codes, B, T, R, cstride,
+                              pos0, pos0_dev, table2, table3, kv_pack, w_mem, eps, scale, sink, head_out);
+}
+
+// One token a block of eight waves, a route chunk a wave (up to 256 routes).
+__global__ __launch_bounds__(512, 1) void k_readout_token(
+    const bf16* __restrict__ q, const bf16* __restrict__ q_rows, float q_eps, const uint8_t* __restrict__ codes,
+    int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
+    const bf16* __restrict__ table2, const bf16* __restrict__ table3, const bf16* __restrict__ kv_pack,
+    const bf16* __restrict__ w_mem, float eps, float scale, float sink, bf16* __restrict__ head_out) {
+  __shared__ ReadoutLds<8> lds;
+  readout_body<8, true>(lds, blockIdx.x, q, q_rows, q_eps, codes, B, T, R, cstride, pos0, pos0_dev, table2, table3,
+                        kv_pack, w_mem, eps, scale, sink, head_out);
 }
 
 // kv [512, 256] -> packed operand order (one thread per 16-byte piece, 16384 pieces).
@@ -427,6 +512,9 @@ __global__ __launch_bounds__(256) void k_readout_pack(const bf16* __restrict__ k
 
 using namespace lng;
 
+constexpr int64_t FR_ROUND = 4 * 2 * 256;  // tokens of a round of 4-token blocks, two a CU
+constexpr int64_t FR_TOKEN_MAX = 256, FR_SPLIT_MAX = 512;
+
 static int readout_launch(const void* q, const void* q_rows, float q_eps, const uint8_t* codes, int64_t B, int64_t T,
                           int32_t R, int64_t cstride, int64_t pos0, const int32_t* pos0_dev, const void* table2,
                           const void* table3, const void* kv_pack, const void* w_mem, float eps, float scale,
@@ -436,16 +524,38 @@ static int readout_launch(const void* q, const void* q_rows, float q_eps, const 
   if (R > FR_MAXR) return fail(LNG_E_ARG, "memory_readout_fused: at most 256 routes");
   const int64_t ntok = B * T;
   if (ntok == 0) return LNG_OK;
-  const int64_t blocks = cdiv(ntok, FR_TOK);
+  int64_t blocks = cdiv(ntok, FR_TOK);
   if (blocks > 0x7fffffffLL) return fail(LNG_E_ARG, "memory_readout_fused: too many tokens");
   // buffer offsets are 32-bit: the token-major activations (2 KB per token) stay under 4 GB; the
   // 3-gram table (R <= 256 routes x 4096 rows x 256 B) always does
   if (ntok > (int64_t{1} << 21)) return fail(LNG_E_ARG, "memory_readout_fused: more than 2^21 tokens per launch");
+  // Few tokens leave the chip idle while each waits for its own chain of six chunks (184 routes), so
+  // their routes are split over a block's waves.  Times in us (184 routes), tokens:
+  //                            8     64    200    256    400    512    700   2331
+  //   four tokens a block   18.7   18.8   19.3   19.7   20.4   20.7   21.3   47.1
+  //   a token a block of 4  11.7   11.9   12.6   13.1   17.8   19.5   28.4   45.9 (the last 283 tokens)
+  //   a token a block of 8  10.5   10.8   11.8   12.4   24.0   26.3   38.4
+  // (one block of 8 waves or two of 4 fit a CU).  Past a whole round of 4-token blocks (2 x 256 of them)
+  // a remainder of up to 512 tokens is split too: the last round is then as short.
+  if (ntok <= FR_TOKEN_MAX) {
+    hipLaunchKernelGGL(k_readout_token, dim3(static_cast<unsigned>(ntok)), dim3(512), 0, as_stream(stream),
+                       static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes, B, T, R, cstride, pos0,
+                       pos0_dev, static_cast<const bf16*>(table2), static_cast<const bf16*>(table3),
+                       static_cast<const bf16*>(kv_pack), static_cast<const bf16*>(w_mem), eps, scale, sink_logit,
+                       static_cast<bf16*>(head_out));
+    return check_launch("memory_readout_fused (token)");
+  }
+  int64_t full = blocks;
+  const int64_t rem = ntok % FR_ROUND;
+  if (FR_TOK == 4 && rem <= FR_SPLIT_MAX) {
+    full = (ntok - rem) / 4;
+    blocks = full + rem;
+  }
   hipLaunchKernelGGL(k_readout_fused<FR_TOK>, dim3(static_cast<unsigned>(blocks)), dim3(64 * FR_TOK), 0,
                      as_stream(stream), static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes,
                      B, T, R, cstride, pos0, pos0_dev, static_cast<const bf16*>(table2),
                      static_cast<const bf16*>(table3), static_cast<const bf16*>(kv_pack),
-                     static_cast<const bf16*>(w_mem), eps, scale, sink_logit, static_cast<bf16*>(head_out));
+                     static_cast<const bf16*>(w_mem), eps, scale, sink_logit, static_cast<bf16*>(head_out), static_cast<uint32_t>(full));
   return check_launch("memory_readout_fused");
 }
 
