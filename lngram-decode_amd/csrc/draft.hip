@@ -933,8 +933,9 @@ __device__ void sl_score(const lng_drafter& D, const int32_t* ids, int n, const 
 }
 
 // The candidate list of position j (RefDrafter._shortlist): sl[0 .. n) in LDS, n returned (0: empty
-// list).  Called by every thread of a 256-thread block; the hash table and selection state are
-// this function's own LDS.
+// list).  Called by every thread of an NTH-thread block; the hash table and selection state are this
+// function's own LDS.
+template <int NTH>
 __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, int j, int32_t* sl) {
   __shared__ __attribute__((aligned(16))) int32_t hkey[SL_SLOTS];
   __shared__ __attribute__((aligned(16))) unsigned long long hval[SL_SLOTS];
@@ -945,18 +946,19 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
   __shared__ int32_t slot_rows[DR_MAXN];
   __shared__ const int32_t* idp[DR_MAXN];
   __shared__ const int64_t* cnp[DR_MAXN];
-  __shared__ unsigned long long red_t[4];
-  __shared__ int32_t red_i[4], red_s[4];
+  constexpr int NW = NTH / 64;
+  __shared__ unsigned long long red_t[NW];
+  __shared__ int32_t red_i[NW], red_s[NW];
   __shared__ int32_t rad[4];  // selected digit, keys above it, keys in it; list length
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int L = *D.length;
   const int R = D.R, SK = S.K, cap = S.cap, tb = S.tbits, TS = 1 << tb, TM = TS - 1;
-  for (int e = 4 * tid; e < TS; e += 1024) {
+  for (int e = 4 * tid; e < TS; e += 4 * NTH) {
     *reinterpret_cast<int4*>(&hkey[e]) = int4{SL_EMPTY, SL_EMPTY, SL_EMPTY, SL_EMPTY};
     *reinterpret_cast<ulonglong2*>(&hval[e]) = ulonglong2{0ull, 0ull};
     *reinterpret_cast<ulonglong2*>(&hval[e + 2]) = ulonglong2{0ull, 0ull};
   }
-  for (int e = tid; e < S.n_fallback; e += 256) fb[e] = S.fallback[e];
+  for (int e = tid; e < S.n_fallback; e += NTH) fb[e] = S.fallback[e];
   if (tid < DR_MAXN) slot_rows[tid] = tid < D.maxn ? dr_resolve(W.slot[j][tid], L) : -1;
   if (tid == 0) {
 #pragma unroll
@@ -966,23 +968,24 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
     }
   }
   __syncthreads();
-  for (int e = tid; e < D.n_orders * R; e += 256) {
+  for (int e = tid; e < D.n_orders * R; e += NTH) {
     const int o = e / R, r = e % R;
     const int64_t row = idp[o] ? dr_row(D, slot_rows, o, r) : -1;
     rowsh[e] = row >= 0 ? row * SK : -1;
   }
   __syncthreads();
-  // sum the counts per token, SL_LOADS slots in flight per thread (at most TS distinct tokens:
+  // sum the counts per token, LOADS slots in flight per thread (at most TS distinct tokens:
   // every probe sequence ends); slot e is element e % K of sketch row e / K (order, route)
+  constexpr int LOADS = SL_LOADS * 256 / NTH > 8 ? SL_LOADS * 256 / NTH : 8;
   const int M = D.n_orders * R * SK;
   const bool k_pow2 = (SK & (SK - 1)) == 0;
   const int k_shift = __ffs(SK) - 1;
-  for (int e0 = 0; e0 < M; e0 += 256 * SL_LOADS) {
-    int32_t idv[SL_LOADS];
-    int64_t cv[SL_LOADS];
+  for (int e0 = 0; e0 < M; e0 += NTH * LOADS) {
+    int32_t idv[LOADS];
+    int64_t cv[LOADS];
 #pragma unroll
-    for (int u = 0; u < SL_LOADS; ++u) {
-      const int e = e0 + u * 256 + tid;
+    for (int u = 0; u < LOADS; ++u) {
+      const int e = e0 + u * NTH + tid;
       idv[u] = -1;
       cv[u] = 0;
       if (e < M) {
@@ -997,7 +1000,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
       }
     }
 #pragma unroll
-    for (int u = 0; u < SL_LOADS; ++u) {
+    for (int u = 0; u < LOADS; ++u) {
       const int32_t id = idv[u];
       if (cv[u] <= 0 || id < 0 || id >= D.V) continue;
       uint32_t h = sl_hash(id, tb);
@@ -1012,16 +1015,16 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
     }
   }
   __syncthreads();
-  // the list: every slot's (id, total) into registers once (thread tid owns slots 1024 g + 4 tid
+  // the list: every slot's (id, total) into registers once (thread tid owns slots 4 NTH g + 4 tid
   // .. +3, read 16 bytes at a time); distinct tokens and largest total
-  constexpr int KQ = SL_SLOTS / 256;
+  constexpr int KQ = SL_SLOTS / NTH;
   int32_t kid[KQ];
   unsigned long long key[KQ];
   unsigned long long tmax = 0ull;
   int cnt = 0;
 #pragma unroll
   for (int g = 0; g < KQ / 4; ++g) {
-    const int e = (g << 10) + 4 * tid;
+    const int e = g * 4 * NTH + 4 * tid;
     int4 k4 = int4{SL_EMPTY, SL_EMPTY, SL_EMPTY, SL_EMPTY};
     ulonglong2 t01 = ulonglong2{0ull, 0ull}, t23 = t01;
     if (e < TS) {
@@ -1056,7 +1059,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
   __syncthreads();
   tmax = red_t[0];
   cnt = red_i[0];
-  for (int q = 1; q < 4; ++q) {
+  for (int q = 1; q < NW; ++q) {
     tmax = red_t[q] > tmax ? red_t[q] : tmax;
     cnt += red_i[q];
   }
@@ -1081,7 +1084,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
         const int lo = hi > ib ? ib : 0;
         const int width = min(8, hi - lo), shift = hi - width;
         const unsigned long long dm = (1ull << width) - 1ull;
-        hist[tid] = 0;
+        if (tid < 256) hist[tid] = 0;
         __syncthreads();
         if (shift >= ib && width <= 3) {
           // a pass over the totals sees few distinct digits: counted per wave with ballots
@@ -1157,12 +1160,12 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
       if (k && k >= thr) {
         const int pos = atomicAdd(&rad[3], 1);  // keys are unique: exactly `want` pass
         if (pos < SL_MAXCAP) selk[pos] = k;
-        hkey[((q >> 2) << 10) + 4 * tid + (q & 3)] |= SL_TAKEN;
+        hkey[(q >> 2) * 4 * NTH + 4 * tid + (q & 3)] |= SL_TAKEN;
       }
     }
     __syncthreads();
     m = min(rad[3], cap);
-    for (int i = tid; i < m; i += 256) {
+    for (int i = tid; i < m; i += NTH) {
       const unsigned long long k = selk[i];
       int rank = 0;
       for (int i2 = 0; i2 < m; ++i2) rank += selk[i2] > k ? 1 : 0;
@@ -1173,7 +1176,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
     for (; m < cap; ++m) {
       unsigned long long bt = 0ull;
       int32_t bi = INT_MAX, bs = -1;
-      for (int e = tid; e < TS; e += 256) {
+      for (int e = tid; e < TS; e += NTH) {
         const int32_t k = hkey[e];
         if (k < 0 || (k & SL_TAKEN)) continue;
         if (sl_better(hval[e], k, bt, bi)) {
@@ -1200,7 +1203,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
       bt = red_t[0];
       bi = red_i[0];
       bs = red_s[0];
-      for (int q = 1; q < 4; ++q)
+      for (int q = 1; q < NW; ++q)
         if (sl_better(red_t[q], red_i[q], bt, bi)) {
           bt = red_t[q];
           bi = red_i[q];
@@ -1218,7 +1221,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
   __syncthreads();
   // fallback padding: first occurrences not in the list, in order
   int added = 0;
-  for (int f0 = 0; f0 < S.n_fallback && m + added < cap; f0 += 256) {
+  for (int f0 = 0; f0 < S.n_fallback && m + added < cap; f0 += NTH) {
     const int jf = f0 + tid;
     bool ok = false;
     int32_t f = -1;
@@ -1245,7 +1248,7 @@ __device__ int sl_build(const lng_drafter& D, const DrWin& W, const SlArgs& S, i
     if (lane == 0) red_s[w] = __popcll(bal);
     __syncthreads();
     int base = 0, tot = 0;
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < NW; ++q) {
       base += q < w ? red_s[q] : 0;
       tot += red_s[q];
     }
@@ -1326,7 +1329,7 @@ __global__ __launch_bounds__(256) void k_draft_shortlist(lng_drafter D, DrWin W,
   __shared__ int64_t sel_id[DR_MAXK];
   __shared__ float sel_sc[DR_MAXK];
   const int j = blockIdx.x, tid = threadIdx.x, cap = S.cap;
-  const int n_sl = sl_build(D, W, S, j, sl);
+  const int n_sl = sl_build<256>(D, W, S, j, sl);
   const float* lg = logits + static_cast<int64_t>(j) * D.V;
   for (int i = tid; i < cap; i += 256) {
     int32_t id = -1;
@@ -2466,6 +2469,7 @@ namespace {
 constexpr int SM_P = 4;       // positions
 constexpr int SM_RC = 8;      // routes per attention block
 constexpr int SM_MAXCH = 32;  // attention blocks per position (R <= 256)
+constexpr int SM_LIST_T = 1024;  // threads of the block that builds a position's sketch shortlist
 
 __device__ __forceinline__ const void* dr_table(const lng_drafter& D, int oi) {
   return oi == 0 ? D.tables[0] : (oi == 1 ? D.tables[1] : (oi == 2 ? D.tables[2] : D.tables[3]));
@@ -2536,20 +2540,23 @@ __global__ __launch_bounds__(256) void k_sm_qkw(lng_drafter D, DrWin W, float* _
 // (device-coherent hand-off; sync[SY_ATT + j] counts the blocks).       grid (nch (+1), P)
 // With LIST, block nch of each position builds its sketch shortlist meanwhile (it needs only the
 // window's codes) into lists [P][1 + cap]: the length, then the ids.
+// The list block has 1024 threads (its slots are summed and searched in LDS by one block: 31 us of
+// the launch with 256), so the launch's blocks do; an attention block keeps its first 256.
 template <bool LIST>
-__global__ __launch_bounds__(256) void k_sm_attend(lng_drafter D, DrWin W, const float* __restrict__ qkw,
+__global__ __launch_bounds__(LIST ? SM_LIST_T : 256) void k_sm_attend(lng_drafter D, DrWin W, const float* __restrict__ qkw,
                                                    float* __restrict__ part_u, float* __restrict__ part_ml,
                                                    float* __restrict__ u, SlArgs S, int32_t* __restrict__ lists) {
   if constexpr (LIST) {
     if (blockIdx.x == gridDim.x - 1) {
       __shared__ int32_t sl[SL_MAXCAP];
       const int j = blockIdx.y;
-      const int n = sl_build(D, W, S, j, sl);
+      const int n = sl_build<SM_LIST_T>(D, W, S, j, sl);
       int32_t* lj = lists + static_cast<int64_t>(j) * (S.cap + 1);
       if (threadIdx.x == 0) lj[0] = n;
-      for (int i = threadIdx.x; i < n; i += 256) lj[1 + i] = sl[i];
+      for (int i = threadIdx.x; i < n; i += SM_LIST_T) lj[1 + i] = sl[i];
       return;
     }
+    if (threadIdx.x >= 256) return;  // whole waves, before any barrier
   }
   __shared__ __attribute__((aligned(16))) float xs[SM_RC][LNG_DR_MAX_DT];
   __shared__ __attribute__((aligned(16))) float qs[LNG_DR_MAX_QH * LNG_DR_MAX_DT];
@@ -3065,7 +3072,7 @@ int dr_front(const lng_drafter& D, const DrWin& W, const DrLayout& l, char* work
     if (int rc = check_launch("drafter_readout(qkw)")) return rc;
     if (sk)
       hipLaunchKernelGGL(k_sm_attend<true>, dim3(static_cast<unsigned>(l.smch + 1), static_cast<unsigned>(P)),
-                         dim3(256), 0, s, D, W, qkw, pu, pml, uo, *sk, reinterpret_cast<int32_t*>(work + l.lists));
+                         dim3(SM_LIST_T), 0, s, D, W, qkw, pu, pml, uo, *sk, reinterpret_cast<int32_t*>(work + l.lists));
     else
       hipLaunchKernelGGL(k_sm_attend<false>, dim3(static_cast<unsigned>(l.smch), static_cast<unsigned>(P)),
                          dim3(256), 0, s, D, W, qkw, pu, pml, uo, SlArgs{}, nullptr);
