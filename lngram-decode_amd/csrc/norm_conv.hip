@@ -9,6 +9,8 @@
 // output, SiLU and the residual add each once more.
 #include "common.h"
 
+#include <type_traits>
+
 namespace lng {
 
 // One wave per row; 4 rows per 256-thread block.
@@ -139,10 +141,6 @@ __global__ __launch_bounds__(256) void k_causal_conv(const T* __restrict__ mixed
 }
 
 // Kernel 4, dilation 3 (the configured short conv: dilation = max n-gram order 3).
-// Block = (b, 16 positions), 128 threads x 8 channels (16-byte accesses).  Row scales of
-// the 16 + 9 rows come first (one wave per row); then each thread slides over the rows
-// keeping the last 10 normalised rows of its channels in registers.
-constexpr int C43_TT = 16;
 constexpr int C43_HALO = 9;
 
 __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
@@ -169,82 +167,95 @@ __device__ __forceinline__ void store8(bf16* p, const float (&v)[8]) {
   *reinterpret_cast<bf16x8*>(p) = a;
 }
 
-template <typename T>
-__global__ __launch_bounds__(128) void k_causal_conv_k4d3(const T* __restrict__ mixed, const T* __restrict__ norm_w,
+// TT positions x all channels a block of 256 threads.  The rows' loads of a wave go out together, then
+// their sums; a thread forms 8 channels of one output from its four rows (the block's rows are in L1 by
+// then).  A lane sums 8 consecutive elements, 512 apart, as k_conv_slots does.  4 x 128 x 128 fp32: 24.5
+// us with one wave-serial pass over the rows and 16 of 128 threads sliding over the positions.
+template <typename T, int TT>
+__global__ __launch_bounds__(256) void k_causal_conv_k4d3(const T* __restrict__ mixed, const T* __restrict__ norm_w,
                                                           const T* __restrict__ conv_w, ConvWin W, int32_t d,
                                                           float eps, int residual, T* __restrict__ out) {
-  __shared__ float scale[C43_TT + C43_HALO];
+  constexpr int NR = TT + C43_HALO, RPW = (NR + 3) / 4;
+  __shared__ float scale[RPW * 4];
   const int64_t b = blockIdx.y;
   const int64_t p0 = conv_p0(W);
-  const int64_t t0 = p0 + static_cast<int64_t>(blockIdx.x) * C43_TT;
+  const int64_t t0 = p0 + static_cast<int64_t>(blockIdx.x) * TT;
   const int64_t T_len = min(W.len, p0 + W.n);  // rows read and outputs end here
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const T* base = mixed + b * W.stride * d;
   if (p0 < 0) return;
-  for (int i = wave; i < C43_TT + C43_HALO; i += 2) {
-    const int64_t t = t0 - C43_HALO + i;
-    float r = 0.f;
-    if (t >= 0 && t < T_len) {
-      float ss = 0.f;
-      for (int c = lane * 8; c < d; c += 64 * 8) {
-        float v[8];
-        load8(base + t * d + c, v);
+  float ss[RPW];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss = fmaf(v[j], v[j], ss);
-      }
-      ss = wave_sum(ss);
-      r = 1.0f / sqrtf(ss / static_cast<float>(d) + eps);
-    }
-    if (lane == 0) scale[i] = r;
-  }
-  __syncthreads();
-  for (int c = threadIdx.x * 8; c < d; c += blockDim.x * 8) {
-    float nw[8], w[4][8];
-    load8(norm_w + c, nw);
+  for (int k = 0; k < RPW; ++k) ss[k] = 0.f;
+  for (int c = lane * 8; c < d; c += 64 * 8) {
+    float v[RPW][8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) w[k][j] = to_f32(conv_w[(c + j) * 4 + k]);
-    float hist[10][8];  // hist[k] = normalised row at t - k
-#pragma unroll
-    for (int k = 0; k < 10; ++k)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) hist[k][j] = 0.f;
-#pragma unroll
-    for (int step = 0; step < C43_TT + C43_HALO; ++step) {
-      const int64_t t = t0 - C43_HALO + step;
-#pragma unroll
-      for (int k = 9; k > 0; --k)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) hist[k][j] = hist[k - 1][j];
-      float x[8];
-      if (t >= 0 && t < T_len) {
-        load8(base + t * d + c, x);
-        const float s = scale[step];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) hist[0][j] = norm_elem<T, true>(x[j], s, nw[j]);
+    for (int k = 0; k < RPW; ++k) {
+      const int i = wave + 4 * k;
+      const int64_t t = t0 - C43_HALO + i;
+      if (i < NR && t >= 0 && t < T_len) {
+        load8(base + t * d + c, v[k]);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          hist[0][j] = 0.f;
-          x[j] = 0.f;
-        }
-      }
-      if (step >= C43_HALO && t < T_len) {
-        float o[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float acc = w[0][j] * hist[9][j];
-          acc = fmaf(w[1][j], hist[6][j], acc);
-          acc = fmaf(w[2][j], hist[3][j], acc);
-          acc = fmaf(w[3][j], hist[0][j], acc);
-          const float y = round_to<T>(acc);
-          const float act = round_to<T>(y / (1.0f + expf(-y)));
-          o[j] = residual ? x[j] + act : act;
-        }
-        store8(out + (b * W.n + t - p0) * d + c, o);
+        for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
       }
     }
+#pragma unroll
+    for (int k = 0; k < RPW; ++k)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss[k] = fmaf(v[k][j], v[k][j], ss[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < RPW; ++k) {
+    const int i = wave + 4 * k;
+    const int64_t t = t0 - C43_HALO + i;
+    const float s = wave_sum(ss[k]);
+    if (lane == 0) scale[i] = t >= 0 && t < T_len ? 1.0f / sqrtf(s / static_cast<float>(d) + eps) : 0.f;
+  }
+  __syncthreads();
+  const int nch = d >> 3;
+  for (int e = threadIdx.x; e < TT * nch; e += 256) {
+    const int tt = e / nch, c = (e - tt * nch) * 8;
+    const int64_t t = t0 + tt;
+    if (t >= T_len) break;  // later items of this thread lie later still
+    float nw[8], x[4][8];  // x[k]: the row of tap k, at t - 9 + 3 k
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (t - C43_HALO + 3 * k >= 0) {
+        load8(base + (t - C43_HALO + 3 * k) * d + c, x[k]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[k][j] = 0.f;
+      }
+    }
+    load8(norm_w + c, nw);
+    float w[8][4];  // channel c + j's taps
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      float p[8];
+      load8(conv_w + static_cast<int64_t>(c + j) * 4, p);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        w[j][k] = p[k];
+        w[j + 1][k] = p[4 + k];
+      }
+    }
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float h[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        h[k] = t - C43_HALO + 3 * k >= 0 ? norm_elem<T, true>(x[k][j], scale[tt + 3 * k], nw[j]) : 0.f;
+      float acc = w[j][0] * h[0];
+      acc = fmaf(w[j][1], h[1], acc);
+      acc = fmaf(w[j][2], h[2], acc);
+      acc = fmaf(w[j][3], h[3], acc);
+      const float y = round_to<T>(acc);
+      const float act = round_to<T>(y / (1.0f + expf(-y)));
+      o[j] = residual ? x[3][j] + act : act;
+    }
+    store8(out + (b * W.n + t - p0) * d + c, o);
   }
 }
 
@@ -673,16 +684,20 @@ static int conv_launch(const void* mixed, const void* norm_w, const void* conv_w
                        static_cast<uint32_t>(d / 4), eps, residual, static_cast<bf16*>(out));
     return check_launch("causal_conv_k4d3_bf16");
   }
-  if (K == 4 && dilation == 3 && d % 8 == 0 && (dtype == LNG_F32 || dtype == LNG_BF16)) {
-    dim3 g43(static_cast<unsigned>(cdiv(n, C43_TT)), static_cast<unsigned>(B));
+  if (K == 4 && dilation == 3 && d % 8 == 0 && (dtype == LNG_F32 || dtype == LNG_BF16) &&
+      (reinterpret_cast<uintptr_t>(conv_w) & 15) == 0) {  // a channel pair's taps are read 16 bytes at a time
+    // 8 positions a block (17 rows) until 16 fill the chip twice over (25 rows, less of them halo)
+    const bool small = B * cdiv(n, 16) < 512;
+    dim3 g43(static_cast<unsigned>(cdiv(n, small ? 8 : 16)), static_cast<unsigned>(B));
+    auto go = [&](auto* kern, auto* type) {
+      using T = std::remove_pointer_t<decltype(type)>;
+      hipLaunchKernelGGL(kern, g43, dim3(256), 0, s, static_cast<const T*>(mixed), static_cast<const T*>(norm_w),
+                         static_cast<const T*>(conv_w), W, d, eps, residual, static_cast<T*>(out));
+    };
     if (dtype == LNG_F32)
-      hipLaunchKernelGGL(k_causal_conv_k4d3<float>, g43, dim3(128), 0, s, static_cast<const float*>(mixed),
-                         static_cast<const float*>(norm_w), static_cast<const float*>(conv_w), W, d, eps, residual,
-                         static_cast<float*>(out));
+      go(small ? &k_causal_conv_k4d3<float, 8> : &k_causal_conv_k4d3<float, 16>, static_cast<float*>(nullptr));
     else
-      hipLaunchKernelGGL(k_causal_conv_k4d3<bf16>, g43, dim3(128), 0, s, static_cast<const bf16*>(mixed),
-                         static_cast<const bf16*>(norm_w), static_cast<const bf16*>(conv_w), W, d, eps, residual,
-                         static_cast<bf16*>(out));
+      go(small ? &k_causal_conv_k4d3<bf16, 8> : &k_causal_conv_k4d3<bf16, 16>, static_cast<bf16*>(nullptr));
     return check_launch("causal_conv_k4d3");
   }
   dim3 grid(static_cast<unsigned>(cdiv(n, CONV_TT)), static_cast<unsigned>(B));
