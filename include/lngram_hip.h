@@ -162,6 +162,11 @@ int lng_linear_at(const void* x, const void* w, int64_t M, int64_t N, int64_t K,
                   int64_t pos0, const int32_t* pos0_dev, void* y, void* stream);
 int lng_router_codes_at(const void* x, const void* w, int64_t M, int64_t K, int64_t N, int64_t group,
                         int64_t stride, int64_t pos0, const int32_t* pos0_dev, uint8_t* codes, void* stream);
+/* lng_router_codes_at of x [M, router_k] and lng_linear of h [M, q_k] (the folded query weight of
+ * memory_step's readout) in one launch: the same results as the two calls. */
+int lng_router_query_at(const void* x, const void* w_router, int64_t router_k, int64_t router_n, int64_t group,
+                        int64_t stride, int64_t pos0, const int32_t* pos0_dev, uint8_t* codes, const void* h,
+                        const void* w_q, int64_t q_k, int64_t q_n, int64_t M, void* q, void* stream);
 
 /* y[M,N] = x[M,K] . w[N,K]^T in `dtype` (fp32 accumulation, output rounded to
  * dtype).  nn.Linear without bias as used by readout_q_proj / readout_kv_proj /

@@ -847,10 +847,11 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
 // 128 takes 3.3 us and 32768 x 256 x 1024 143 us (120 TFLOP/s); the VALU tile below 18.9 and 393 (few
 // blocks, a scalar LDS read for every two FMAs).  Same error against fp64: 2.03e-7 relative at K = 128,
 // 5.74e-7 at K = 1024, over twelve seeds.
+// codes (N % 4 == 0): also the 4-bit route codes, bit i of route r the sign of output 4 r + i.
 template <int BN, int BM>
 __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__ W, const float* __restrict__ X,
                                                        int64_t N, int64_t M, int64_t K, int n_tiles,
-                                                       float* __restrict__ Y) {
+                                                       float* __restrict__ Y, void* __restrict__ codes, int codes_dt) {
   using G = TileGemm<float, BN, BM, 2, 2, 1, 3>;
   __shared__ __attribute__((aligned(16))) float ring[G::LDS_ELEMS];
   const int64_t n0 = static_cast<int64_t>(blockIdx.x % n_tiles) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
@@ -867,7 +868,15 @@ __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__
       const int64_t n = n0 + wn * (BN / 2) + i * 16 + 4 * (lane >> 4);
       float* o = Y + m * N + n;
       if (n + 3 < N && (N & 3) == 0) {
-        *reinterpret_cast<f32x4*>(o) = g.acc[i][j];
+        const f32x4 v = g.acc[i][j];
+        *reinterpret_cast<f32x4*>(o) = v;
+        if (codes) {
+          const int code = (v[0] > 0.f ? 1 : 0) | (v[1] > 0.f ? 2 : 0) | (v[2] > 0.f ? 4 : 0) | (v[3] > 0.f ? 8 : 0);
+          if (codes_dt == LNG_U8)
+            static_cast<uint8_t*>(codes)[m * (N >> 2) + (n >> 2)] = static_cast<uint8_t>(code);
+          else
+            static_cast<int32_t*>(codes)[m * (N >> 2) + (n >> 2)] = code;
+        }
       } else {
         for (int e = 0; e < 4; ++e)
           if (n + e < N) o[e] = g.acc[i][j][e];
@@ -984,12 +993,11 @@ struct RowMap {
 };
 
 template <int EPI>
-__global__ __launch_bounds__(64, 1) void k_gemm_skinny(const bf16* __restrict__ W, const bf16* __restrict__ X,
-                                                       int64_t N, int64_t M, int64_t K, RowMap map,
-                                                       void* __restrict__ out, float* __restrict__ logits,
-                                                       void* __restrict__ codes, int codes_dt, int64_t routes) {
+__device__ __forceinline__ void skinny_tile(const bf16* __restrict__ W, const bf16* __restrict__ X, int64_t n0,
+                                            int64_t m0, int64_t N, int64_t M, int64_t K, const RowMap& map,
+                                            void* __restrict__ out, float* __restrict__ logits,
+                                            void* __restrict__ codes, int codes_dt, int64_t routes) {
   const int lane = threadIdx.x;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 16, m0 = static_cast<int64_t>(blockIdx.y) * 16;
   const int rsel = lane & 15, psel = lane >> 4;
   const int64_t wr = n0 + rsel < N ? n0 + rsel : N - 1;
   const int64_t xr = m0 + rsel < M ? m0 + rsel : M - 1;
@@ -1030,6 +1038,28 @@ __global__ __launch_bounds__(64, 1) void k_gemm_skinny(const bf16* __restrict__ 
     else
       static_cast<int32_t*>(codes)[row * routes + r] = code;
   }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(64, 1) void k_gemm_skinny(const bf16* __restrict__ W, const bf16* __restrict__ X,
+                                                       int64_t N, int64_t M, int64_t K, RowMap map,
+                                                       void* __restrict__ out, float* __restrict__ logits,
+                                                       void* __restrict__ codes, int codes_dt, int64_t routes) {
+  skinny_tile<EPI>(W, X, static_cast<int64_t>(blockIdx.x) * 16, static_cast<int64_t>(blockIdx.y) * 16, N, M, K, map, out,
+                   logits, codes, codes_dt, routes);
+}
+
+// A decode step's router codes (into the code cache) and query projection in one launch: both read
+// only the step's input rows.  4.2 + 3.5 us and the gap between them as two launches.
+__global__ __launch_bounds__(64, 1) void k_gemm_skinny_pair(const bf16* __restrict__ WR, const bf16* __restrict__ XR,
+                                                            int64_t NR, int64_t KR, RowMap map, uint8_t* __restrict__ codes,
+                                                            const bf16* __restrict__ WQ, const bf16* __restrict__ XQ,
+                                                            int64_t NQ, int64_t KQ, int64_t M, bf16* __restrict__ q) {
+  const int64_t nr = (NR + 15) / 16, m0 = static_cast<int64_t>(blockIdx.y) * 16, b = blockIdx.x;
+  if (b < nr)
+    skinny_tile<EPI_ROUTER>(WR, XR, b * 16, m0, NR, M, KR, map, nullptr, nullptr, codes, LNG_U8, NR / 4);
+  else
+    skinny_tile<EPI_BF16>(WQ, XQ, (b - nr) * 16, m0, NQ, M, KQ, RowMap{M, 0, 0, nullptr}, q, nullptr, nullptr, 0, 0);
 }
 
 template <int EPI>
@@ -1139,11 +1169,14 @@ static int launch_proj(const bf16* w, const bf16* x, int64_t N, int64_t M, int64
   return check_launch("gemm_bf16_proj");
 }
 
-static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N, int64_t K, float* y, hipStream_t s) {
+static bool tile_f32_shape(int64_t N, int64_t K) { return K % 32 == 0 && N * K * 4 < (int64_t{1} << 31); }
+
+static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N, int64_t K, float* y, hipStream_t s,
+                           void* codes = nullptr, int codes_dt = 0) {
   auto go = [&](auto* kern, int64_t bn, int64_t bm) {
     const int n_tiles = static_cast<int>(cdiv(N, bn));
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, x, N, M, K,
-                       n_tiles, y);
+                       n_tiles, y, codes, codes_dt);
     return check_launch("gemm_f32_tile");
   };
   // small tiles while they make few blocks a CU: 584 blocks of 32 x 32 took 18.8 us at 2331 x 256 x 1024
@@ -1155,7 +1188,7 @@ static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N,
 template <typename TA, typename TB, typename TO>
 static int launch_f32(const void* x, const void* w, int64_t M, int64_t N, int64_t K, void* y, hipStream_t s) {
   if constexpr (sizeof(TA) == 4 && sizeof(TB) == 4 && sizeof(TO) == 4) {
-    if (K % 32 == 0 && N * K * 4 < (int64_t{1} << 31))
+    if (tile_f32_shape(N, K))
       return launch_tile_f32(static_cast<const float*>(x), static_cast<const float*>(w), M, N, K, static_cast<float*>(y), s);
   }
   dim3 grid(static_cast<unsigned>(cdiv(N, 64)), static_cast<unsigned>(cdiv(M, 64)));
@@ -1290,6 +1323,9 @@ int lng_router_codes(const void* x, int x_dtype, const void* w, int w_dtype, int
       return rc;
   } else {
     if (!logits) return fail(LNG_E_ARG, "router_codes: fp32 router needs a logits buffer");
+    if (x_dtype == LNG_F32 && w_dtype == LNG_F32 && codes && bits == 4 && tile_f32_shape(N, K))
+      return launch_tile_f32(static_cast<const float*>(x), static_cast<const float*>(w), M, N, K, logits, s, codes,
+                             codes_dtype);
     int rc;
     if (x_dtype == LNG_F32 && w_dtype == LNG_F32)
       rc = launch_f32<float, float, float>(x, w, M, N, K, logits, s);
@@ -1358,6 +1394,20 @@ int lng_router_codes_at(const void* x, const void* w, int64_t M, int64_t K, int6
   return launch_skinny<EPI_ROUTER>(static_cast<const bf16*>(w), static_cast<const bf16*>(x), N, M, K,
                                    RowMap{group, stride, pos0, pos0_dev}, nullptr, nullptr, codes, LNG_U8, N / 4,
                                    as_stream(stream));
+}
+
+int lng_router_query_at(const void* x, const void* w_router, int64_t router_k, int64_t router_n, int64_t group,
+                        int64_t stride, int64_t pos0, const int32_t* pos0_dev, uint8_t* codes, const void* h,
+                        const void* w_q, int64_t q_k, int64_t q_n, int64_t M, void* q, void* stream) {
+  if (M < 0 || M > SK_MAXM || router_n <= 0 || router_n % 16 || q_n <= 0 || q_n % 16 || router_k <= 0 || router_k % 32 ||
+      q_k <= 0 || q_k % 32 || group <= 0 || M % group || pos0 < 0 || stride < 0 || !codes || !q)
+    return fail(LNG_E_ARG, "router_query_at: bf16, 4-bit codes, M <= 64 (a multiple of group), N % 16 == 0, K % 32 == 0");
+  if (M == 0) return LNG_OK;
+  const dim3 g(static_cast<unsigned>(router_n / 16 + q_n / 16), static_cast<unsigned>(cdiv(M, 16)));
+  hipLaunchKernelGGL(k_gemm_skinny_pair, g, dim3(64), 0, as_stream(stream), static_cast<const bf16*>(w_router),
+                     static_cast<const bf16*>(x), router_n, router_k, RowMap{group, stride, pos0, pos0_dev}, codes,
+                     static_cast<const bf16*>(w_q), static_cast<const bf16*>(h), q_n, q_k, M, static_cast<bf16*>(q));
+  return check_launch("router_query_at");
 }
 
 }  // extern "C"

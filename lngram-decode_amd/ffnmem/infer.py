@@ -122,9 +122,11 @@ def router_input_at(model, mem, state: DecodeState, emb: Tensor, s_new: Tensor |
     return mem.router_features(torch.cat((prev, emb), dim=1), s_cat)[:, 1:]
 
 
-def _readout_head(m, h: Tensor, codes: Tensor, pos0: int, pos0_dev: Tensor | None) -> Tensor:
-    """Fused readout of the new positions whose codes sit at ``pos0 (+ pos0_dev)`` of ``codes``."""
-    q_raw = ops.linear(h, m._folded_query_weight())
+def _readout_head(m, h: Tensor, codes: Tensor, pos0: int, pos0_dev: Tensor | None, q_raw: Tensor | None = None) -> Tensor:
+    """Fused readout of the new positions whose codes sit at ``pos0 (+ pos0_dev)`` of ``codes``
+    (``q_raw``: their query projection, where the caller has it)."""
+    if q_raw is None:
+        q_raw = ops.linear(h, m._folded_query_weight())
     return ops.memory_readout_fused_at(q_raw, codes, pos0, m.tables["ngram_2"].weight, m.tables["ngram_3"].weight,
                                        m._fused_weights(), m.readout_memory_norm.weight, m.readout_memory_norm.eps,
                                        m.softmax_scale, m.readout_sink_logit, q_rows=h,
@@ -232,17 +234,22 @@ def static_memory_step(model, pos: int, state: DecodeState, h: Tensor, codes_new
     dev = h.device
     L32 = (L_t if L_t.dtype == torch.int32 else L_t.to(torch.int32)).reshape(1)
     cache = state.codes[pos]
+    fused, q_raw = m._fused_shape_ok(h), None
     if codes_new is None:
         if router_x is None:
             raise ValueError("static_memory_step needs codes_new or router_x")
-        if _skinny_ok(router_x, mem.router.weight) and mem.bits == 4:
+        if (fused and mem.bits == 4 and _skinny_ok(router_x, mem.router.weight) and router_x.shape[:2] == h.shape[:2]
+                and _skinny_ok(h, m.readout_q_proj.weight)):
+            # both read only the step's inputs: one launch
+            q_raw = ops.router_query_at(router_x, mem.router.weight, cache, h, m._folded_query_weight(), 0, L32)
+        elif _skinny_ok(router_x, mem.router.weight) and mem.bits == 4:
             ops.router_codes_at(router_x, mem.router.weight, cache, 0, L32)
         else:
             codes_new = mem.route_codes(router_x)[1]
     if codes_new is not None:
         cache.index_copy_(1, L32.long() + torch.arange(n, device=dev), codes_new.to(cache.dtype))
-    if m._fused_shape_ok(h):
-        head = _readout_head(m, h, cache, 0, L32)
+    if fused:
+        head = _readout_head(m, h, cache, 0, L32, q_raw)
     else:
         hist = m.route_history_length
         hidx = L32.long() - hist + torch.arange(hist + n, device=dev)

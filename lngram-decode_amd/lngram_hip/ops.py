@@ -506,6 +506,24 @@ def router_codes_at(x: torch.Tensor, w: torch.Tensor, cache: torch.Tensor, pos0:
                                     _ptr(pos0_dev), _ptr(cache), _stream(dev)), "router_codes_at")
 
 
+def router_query_at(x: torch.Tensor, w: torch.Tensor, cache: torch.Tensor, h: torch.Tensor, w_q: torch.Tensor,
+                    pos0: int = 0, pos0_dev: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`router_codes_at` of ``x`` into ``cache`` and ``linear(h, w_q)`` in one launch
+    (``lng_router_query_at``; bf16, B*n <= 64)."""
+    dev = _dev(x, w, cache, h, w_q, pos0_dev)
+    _at_args(cache, pos0_dev)
+    b, n, k = x.shape
+    xc, wc, hc, qc = _c(x), _c(w), _c(h), _c(w_q)
+    if (any(t.dtype != torch.bfloat16 for t in (xc, wc, hc, qc)) or cache.dtype != torch.uint8 or cache.shape[0] != b
+            or tuple(wc.shape) != (4 * cache.shape[2], k) or tuple(hc.shape[:2]) != (b, n) or qc.shape[1] != hc.shape[2]):
+        raise ValueError("router_query_at: bf16 x [B, n, K], router [4R, K], h [B, n, d], w_q [N, d], uint8 cache [B, S, R]")
+    q = torch.empty(b, n, qc.shape[0], dtype=torch.bfloat16, device=dev)
+    check(lib().lng_router_query_at(_ptr(xc), _ptr(wc), k, wc.shape[0], n, cache.shape[1], int(pos0), _ptr(pos0_dev),
+                                    _ptr(cache), _ptr(hc), _ptr(qc), qc.shape[1], qc.shape[0], b * n, _ptr(q),
+                                    _stream(dev)), "router_query_at")
+    return q
+
+
 def tree_windows(cache: torch.Tensor, node_codes: torch.Tensor, idx: torch.Tensor, hist: int, L: int,
                  L_dev: torch.Tensor | None, rel: torch.Tensor):
     """The n-gram windows of a draft tree's nodes and the node codes cached (``lng_tree_windows``):
