@@ -312,6 +312,16 @@ int lng_memory_readout_fused_rows(const void* q, const void* q_rows, float q_eps
                                   int64_t n, int32_t R, const void* kv_pack, const void* w_mem, float eps, float scale,
                                   float sink_logit, void* head_out, void* stream);
 
+/* lng_memory_readout_fused of n tokens, each with its own window of codes: win [n, H, R] (the token's code
+ * last), seg [n, H] int32 and val [n, H] as lng_tree_windows writes them; an n-gram whose first code's
+ * segment differs from its last's, or whose last code is not valid, reads zero rows (the lookup's masks,
+ * lngram_v2.py:1027-1045; the ancestor windows of a draft tree, drafting/tree.py:114-136).  Equal to
+ * lng_route_tokens over the windows followed by lng_memory_readout_fused_rows. */
+int lng_memory_readout_fused_windows(const void* q, const void* q_rows, float q_eps, const uint8_t* win,
+                                     const int32_t* seg, const uint8_t* val, int64_t n, int32_t H, int32_t R,
+                                     const void* table2, const void* table3, const void* kv_pack, const void* w_mem,
+                                     float eps, float scale, float sink_logit, void* head_out, void* stream);
+
 /* out[N, K] = w[N, K] * s[K] (bf16, one rounding): a row RMSNorm's weight folded into the projection
  * that follows it (readout_query_norm.weight into readout_q_proj.weight, lngram_v2.py:1115-1118). */
 int lng_fold_columns(const void* w, const void* s, int64_t N, int64_t K, void* out, void* stream);

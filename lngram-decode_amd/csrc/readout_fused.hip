@@ -105,7 +105,8 @@ struct ReadoutLds {
 template <int FR_TOK, bool SPLIT>
 __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t tok0, const bf16* __restrict__ q,
                                              const bf16* __restrict__ q_rows, float q_eps,
-                                             const uint8_t* __restrict__ codes, int64_t B, int64_t T, int32_t R,
+                                             const uint8_t* __restrict__ codes, const int32_t* __restrict__ seg,
+                                             const uint8_t* __restrict__ val, int64_t B, int64_t T, int32_t R,
                                              int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
                                              const bf16* __restrict__ table2, const bf16* __restrict__ table3,
                                              const bf16* __restrict__ kv_pack, const bf16* __restrict__ w_mem,
@@ -159,6 +160,14 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
   const int64_t crow = tb * cstride + tpos;  // codes row of the token
   // a position outside [0, cstride) (a device position past the cache) reads no codes
   const bool codes_ok = tok_ok && tpos >= 0 && tpos < cstride;
+  // windows (seg, val of the codes' rows given): an n-gram whose first code lies in another segment
+  // than its last, or whose last is not valid, reads a zero row
+  bool ok2 = true, ok3 = true;
+  if (seg != nullptr && codes_ok) {
+    ok2 = ok3 = val[crow] != 0;
+    if (tpos >= 1) ok2 = ok2 && seg[crow - 1] == seg[crow];
+    if (tpos >= 2) ok3 = ok3 && seg[crow - 2] == seg[crow];
+  }
 
   // route-token mode (codes == null): table2 / table3 are the caller's route tokens [ntok, R, 256]
   // seen as 128-wide rows, the 2-gram row of (token, route) at 2 (token R + route) of table2 and
@@ -187,8 +196,8 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
       const int r = lane + 64 * k;
       int32_t r2 = -1, r3 = -1;
       if (codes_ok && r < R) {
-        if (tpos >= 1) r2 = r * 256 + cv[1][k] + 16 * cv[0][k];
-        if (tpos >= 2) r3 = r * 4096 + cv[2][k] + 16 * cv[1][k] + 256 * cv[0][k];
+        if (tpos >= 1 && ok2) r2 = r * 256 + cv[1][k] + 16 * cv[0][k];
+        if (tpos >= 2 && ok3) r3 = r * 4096 + cv[2][k] + 16 * cv[1][k] + 256 * cv[0][k];
       }
       rowsh[w][0][r & 3][r >> 2] = r2;
       rowsh[w][1][r & 3][r >> 2] = r3;
@@ -203,7 +212,7 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
   // fetch the two halves of one row, so the LDS pass that stores them writes 256 contiguous bytes.
   const int g_sub = ((lane >> 3) & 1) | ((lane >> 4) & 2), g_piece = (lane & 7) | ((lane >> 1) & 8);
   // every row of a token at t >= 2 exists (both orders), as does every route token: no mask
-  const bool all_rows = rows_mode || tpos >= 2;
+  const bool all_rows = rows_mode || (tpos >= 2 && ok2 && ok3);
   // 3-gram rows through a raw buffer descriptor (the table, at most 256 routes x 4096 rows x 256 B,
   // is < 4 GB, so row * 256 fits the 32-bit offset; every row index is in range, the descriptor's
   // size is left at its maximum)
@@ -461,7 +470,7 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
 template <int FR_TOK>
 __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(
     const bf16* __restrict__ q, const bf16* __restrict__ q_rows, float q_eps, const uint8_t* __restrict__ codes,
-    int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
+    const int32_t* __restrict__ seg, const uint8_t* __restrict__ val, int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
     const bf16* __restrict__ table2, const bf16* __restrict__ table3, const bf16* __restrict__ kv_pack,
     const bf16* __restrict__ w_mem, float eps, float scale, float sink, bf16* __restrict__ head_out,
     uint32_t full_blocks) {
@@ -469,23 +478,23 @@ __global__ __launch_bounds__(64 * FR_TOK, 8 / FR_TOK) void k_readout_fused(
   if constexpr (FR_TOK == 4) {
     if (blockIdx.x >= full_blocks) {
       readout_body<FR_TOK, true>(lds, static_cast<int64_t>(full_blocks) * FR_TOK + (blockIdx.x - full_blocks), q, q_rows,
-                                 q_eps, codes, B, T, R, cstride, pos0, pos0_dev, table2, table3, kv_pack, w_mem, eps,
+                                 q_eps, codes, seg, val, B, T, R, cstride, pos0, pos0_dev, table2, table3, kv_pack, w_mem, eps,
                                  scale, sink, head_out);
       return;
     }
   }
-  readout_body<FR_TOK, false>(lds, static_cast<int64_t>(blockIdx.x) * FR_TOK, q, q_rows, q_eps, codes, B, T, R, cstride,
+  readout_body<FR_TOK, false>(lds, static_cast<int64_t>(blockIdx.x) * FR_TOK, q, q_rows, q_eps, codes, seg, val, B, T, R, cstride,
                               pos0, pos0_dev, table2, table3, kv_pack, w_mem, eps, scale, sink, head_out);
 }
 
 // One token a block of eight waves, a route chunk a wave (up to 256 routes).
 __global__ __launch_bounds__(512, 1) void k_readout_token(
     const bf16* __restrict__ q, const bf16* __restrict__ q_rows, float q_eps, const uint8_t* __restrict__ codes,
-    int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
+    const int32_t* __restrict__ seg, const uint8_t* __restrict__ val, int64_t B, int64_t T, int32_t R, int64_t cstride, int64_t pos0, const int32_t* __restrict__ pos0_dev,
     const bf16* __restrict__ table2, const bf16* __restrict__ table3, const bf16* __restrict__ kv_pack,
     const bf16* __restrict__ w_mem, float eps, float scale, float sink, bf16* __restrict__ head_out) {
   __shared__ ReadoutLds<8> lds;
-  readout_body<8, true>(lds, blockIdx.x, q, q_rows, q_eps, codes, B, T, R, cstride, pos0, pos0_dev, table2, table3,
+  readout_body<8, true>(lds, blockIdx.x, q, q_rows, q_eps, codes, seg, val, B, T, R, cstride, pos0, pos0_dev, table2, table3,
                         kv_pack, w_mem, eps, scale, sink, head_out);
 }
 
@@ -515,7 +524,8 @@ using namespace lng;
 constexpr int64_t FR_ROUND = 4 * 2 * 256;  // tokens of a round of 4-token blocks, two a CU
 constexpr int64_t FR_TOKEN_MAX = 256, FR_SPLIT_MAX = 512;
 
-static int readout_launch(const void* q, const void* q_rows, float q_eps, const uint8_t* codes, int64_t B, int64_t T,
+static int readout_launch(const void* q, const void* q_rows, float q_eps, const uint8_t* codes, const int32_t* seg,
+                          const uint8_t* val, int64_t B, int64_t T,
                           int32_t R, int64_t cstride, int64_t pos0, const int32_t* pos0_dev, const void* table2,
                           const void* table3, const void* kv_pack, const void* w_mem, float eps, float scale,
                           float sink_logit, void* head_out, void* stream) {
@@ -539,8 +549,8 @@ static int readout_launch(const void* q, const void* q_rows, float q_eps, const 
   // a remainder of up to 512 tokens is split too: the last round is then as short.
   if (ntok <= FR_TOKEN_MAX) {
     hipLaunchKernelGGL(k_readout_token, dim3(static_cast<unsigned>(ntok)), dim3(512), 0, as_stream(stream),
-                       static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes, B, T, R, cstride, pos0,
-                       pos0_dev, static_cast<const bf16*>(table2), static_cast<const bf16*>(table3),
+                       static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes, seg, val, B, T, R, cstride,
+                       pos0, pos0_dev, static_cast<const bf16*>(table2), static_cast<const bf16*>(table3),
                        static_cast<const bf16*>(kv_pack), static_cast<const bf16*>(w_mem), eps, scale, sink_logit,
                        static_cast<bf16*>(head_out));
     return check_launch("memory_readout_fused (token)");
@@ -553,7 +563,7 @@ static int readout_launch(const void* q, const void* q_rows, float q_eps, const 
   }
   hipLaunchKernelGGL(k_readout_fused<FR_TOK>, dim3(static_cast<unsigned>(blocks)), dim3(64 * FR_TOK), 0,
                      as_stream(stream), static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes,
-                     B, T, R, cstride, pos0, pos0_dev, static_cast<const bf16*>(table2),
+                     seg, val, B, T, R, cstride, pos0, pos0_dev, static_cast<const bf16*>(table2),
                      static_cast<const bf16*>(table3), static_cast<const bf16*>(kv_pack),
                      static_cast<const bf16*>(w_mem), eps, scale, sink_logit, static_cast<bf16*>(head_out), static_cast<uint32_t>(full));
   return check_launch("memory_readout_fused");
@@ -564,7 +574,7 @@ extern "C" int lng_memory_readout_fused(const void* q, const void* q_rows, float
                                         const void* table2, const void* table3, const void* kv_pack,
                                         const void* w_mem, float eps, float scale, float sink_logit, void* head_out,
                                         void* stream) {
-  return readout_launch(q, q_rows, q_eps, codes, B, T, R, T, 0, nullptr, table2, table3, kv_pack, w_mem, eps, scale,
+  return readout_launch(q, q_rows, q_eps, codes, nullptr, nullptr, B, T, R, T, 0, nullptr, table2, table3, kv_pack, w_mem, eps, scale,
                         sink_logit, head_out, stream);
 }
 
@@ -576,7 +586,7 @@ extern "C" int lng_memory_readout_fused_at(const void* q, const void* q_rows, fl
   if (codes_len <= 0 || pos0 < 0) return fail(LNG_E_ARG, "memory_readout_fused_at: bad codes length or position");
   if (!pos0_dev && pos0 + n > codes_len)
     return fail(LNG_E_RANGE, "memory_readout_fused_at: positions pos0 .. pos0+n-1 past the codes");
-  return readout_launch(q, q_rows, q_eps, codes, B, n, R, codes_len, pos0, pos0_dev, table2, table3, kv_pack, w_mem,
+  return readout_launch(q, q_rows, q_eps, codes, nullptr, nullptr, B, n, R, codes_len, pos0, pos0_dev, table2, table3, kv_pack, w_mem,
                         eps, scale, sink_logit, head_out, stream);
 }
 
@@ -587,8 +597,18 @@ extern "C" int lng_memory_readout_fused_rows(const void* q, const void* q_rows, 
   if (B * n * static_cast<int64_t>(R) >= (int64_t{1} << 23))
     return fail(LNG_E_ARG, "memory_readout_fused_rows: route tokens must stay under 4 GB (B * n * R < 2^23)");
   const bf16* tok = static_cast<const bf16*>(route_tokens);
-  return readout_launch(q, q_rows, q_eps, nullptr, B, n, R, n, 0, nullptr, tok, tok + 128, kv_pack, w_mem, eps, scale,
+  return readout_launch(q, q_rows, q_eps, nullptr, nullptr, nullptr, B, n, R, n, 0, nullptr, tok, tok + 128, kv_pack, w_mem, eps, scale,
                         sink_logit, head_out, stream);
+}
+
+extern "C" int lng_memory_readout_fused_windows(const void* q, const void* q_rows, float q_eps, const uint8_t* win,
+                                                const int32_t* seg, const uint8_t* val, int64_t n, int32_t H, int32_t R,
+                                                const void* table2, const void* table3, const void* kv_pack,
+                                                const void* w_mem, float eps, float scale, float sink_logit,
+                                                void* head_out, void* stream) {
+  if (!win || !seg || !val || H < 1) return fail(LNG_E_ARG, "memory_readout_fused_windows: windows of at least one code");
+  return readout_launch(q, q_rows, q_eps, win, seg, val, n, 1, R, H, H - 1, nullptr, table2, table3, kv_pack, w_mem,
+                        eps, scale, sink_logit, head_out, stream);
 }
 
 extern "C" int lng_memory_readout_pack(const void* kv, void* kv_pack, void* stream) {

@@ -351,15 +351,18 @@ def _tree_memory(model, pos: int, state: DecodeState, h: Tensor, codes: Tensor, 
     # position 0 is not real and its n-grams read zero rows), the node codes cached at L .. L+n-1 and
     # the conv slots, in one launch (the code caches are uint8: codes have at most 8 bits)
     win, seg, val, slots = ops.tree_windows(cache, codes, idx32, hist, L, L_dev, rel)
-    tables = [m.tables[f"ngram_{o}"].weight for o in m.ngrams]
-    rt = ops.route_tokens(win, tables, m.ngrams, m.bits_per_route, 0, m.num_routes, seg, val, 1)
-    rt = rt[:, -1].view(b, n, r, -1)
-    if m._fused_shape_ok(h, tables=False):
+    if m._fused_shape_ok(h):
+        # the readout gathers the windows' rows itself
         q_raw = ops.linear(h, m._folded_query_weight())
-        head = ops.memory_readout_fused_rows(q_raw, rt.to(torch.bfloat16), m._fused_weights(),
-                                             m.readout_memory_norm.weight, m.readout_memory_norm.eps, m.softmax_scale,
-                                             m.readout_sink_logit, q_rows=h, q_eps=m.readout_query_norm.eps)
+        head = ops.memory_readout_fused_windows(q_raw, win, seg, val, m.tables["ngram_2"].weight,
+                                                m.tables["ngram_3"].weight, m._fused_weights(),
+                                                m.readout_memory_norm.weight, m.readout_memory_norm.eps,
+                                                m.softmax_scale, m.readout_sink_logit, q_rows=h,
+                                                q_eps=m.readout_query_norm.eps)
     else:
+        tables = [m.tables[f"ngram_{o}"].weight for o in m.ngrams]
+        rt = ops.route_tokens(win, tables, m.ngrams, m.bits_per_route, 0, m.num_routes, seg, val, 1)
+        rt = rt[:, -1].view(b, n, r, -1)
         key, value = m._project_memory(rt.to(m.readout_kv_proj.weight.dtype))
         head = m._manual_gqa(m._project_query(h), key, value)
     conv_in = state.conv_in[pos]

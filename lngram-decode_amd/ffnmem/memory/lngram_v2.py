@@ -589,8 +589,9 @@ class _RouteNgramMemoryBase(nn.Module):
         self._check_inference(q_btrm)
         plain = segment_ids is None and valid_tokens is None
         fused = plain and self._fused_shape_ok(hidden_states)
-        if plain and b * t and self.bits_per_route <= 8 and hidden_states.is_cuda and \
-                hidden_states.dtype in (torch.bfloat16, torch.float32):
+        if plain and self.bits_per_route <= 8 and hidden_states.is_cuda and \
+                hidden_states.dtype in (torch.bfloat16, torch.float32) and \
+                0 < 3 * hidden_states.numel() * hidden_states.element_size() <= self._NATIVE_WORKSPACE:
             layer = self._native_layer(hidden_states.dtype, hidden_states.device, fused)
             if layer is not None:
                 out = ops.memory_forward(layer, hidden_states,

@@ -118,6 +118,8 @@ SIGNATURES = {
     "lng_memory_readout_fused_at": (_int, [_p, _p, _f, _p, _i64, _i64, _i32, _i64, _i64, _p, _p, _p, _p, _p, _f, _f,
                                            _f, _p, _p]),
     "lng_memory_readout_fused_rows": (_int, [_p, _p, _f, _p, _i64, _i64, _i32, _p, _p, _f, _f, _f, _p, _p]),
+    "lng_memory_readout_fused_windows": (_int, [_p, _p, _f, _p, _p, _p, _i64, _i32, _i32, _p, _p, _p, _p, _f, _f, _f, _p,
+                                                _p]),
     "lng_fold_columns": (_int, [_p, _p, _i64, _i64, _p, _p]),
     "lng_memory_readout_pack": (_int, [_p, _p, _p]),
     "lng_gather_sum_scaled": (_int, [ctypes.POINTER(_p), _int, _i32, _p, _i64, _i64, _i32, _P32, _i32, _i32, _i32,

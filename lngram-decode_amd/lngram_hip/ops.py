@@ -834,6 +834,39 @@ def memory_readout_fused_rows(q: torch.Tensor, route_tokens: torch.Tensor, kv_pa
     return out
 
 
+def memory_readout_fused_windows(q: torch.Tensor, win: torch.Tensor, seg: torch.Tensor, val: torch.Tensor,
+                                 table2: torch.Tensor, table3: torch.Tensor, kv_pack: torch.Tensor, w_mem: torch.Tensor,
+                                 eps: float, scale: float, sink_logit: float, q_rows: torch.Tensor | None = None,
+                                 q_eps: float = 0.0) -> torch.Tensor:
+    """The fused readout of tokens with windows of their own (``lng_memory_readout_fused_windows``): q ``[B, n,
+    1024]``; ``win [B*n, H, R]`` uint8, ``seg`` int32 and ``val`` uint8 ``[B*n, H]`` from :func:`tree_windows`."""
+    dev = _dev(q, win, seg, val, table2, table3, kv_pack, w_mem, q_rows)
+    b, n = q.shape[0], q.shape[1]
+    m, hist, r = win.shape
+    qc = _c(q)
+    if qc.dtype != torch.bfloat16 or qc.shape[-1] != 1024 or m != b * n:
+        raise ValueError("fused readout expects a bf16 [B, n, 1024] query and a window per token")
+    if win.dtype != torch.uint8 or seg.dtype != torch.int32 or val.dtype != torch.uint8 or \
+            tuple(seg.shape) != (m, hist) or tuple(val.shape) != (m, hist) or \
+            not (win.is_contiguous() and seg.is_contiguous() and val.is_contiguous()):
+        raise ValueError("fused readout: contiguous windows uint8 [B*n, H, R], seg int32 and val uint8 [B*n, H]")
+    if table2.shape != (r * 256, 128) or table3.shape != (r * 4096, 128):
+        raise ValueError("fused readout expects tables [R*256,128] and [R*4096,128]")
+    if kv_pack.shape != (_lib.READOUT_PACK_ELEMS,) or kv_pack.dtype != torch.bfloat16 or w_mem.shape != (256,):
+        raise ValueError("fused readout weight shapes")
+    qr = None
+    if q_rows is not None:
+        qr = _c(q_rows)
+        if qr.dtype != torch.bfloat16 or qr.shape != qc.shape:
+            raise ValueError("fused readout: q_rows must be bf16 and shaped like q")
+    out = torch.empty(b, n, 1024, dtype=torch.bfloat16, device=dev)
+    t2, t3, kp, wmc = _c(table2), _c(table3), _c(kv_pack), _c(w_mem.to(torch.bfloat16))
+    check(lib().lng_memory_readout_fused_windows(_ptr(qc), _ptr(qr), float(q_eps), _ptr(win), _ptr(seg), _ptr(val), m,
+                                                 hist, r, _ptr(t2), _ptr(t3), _ptr(kp), _ptr(wmc), eps, scale,
+                                                 sink_logit, _ptr(out), _stream(dev)), "memory_readout_fused_windows")
+    return out
+
+
 def gather_sum_scaled(tables, codes: torch.Tensor, orders, bits: int, scale_log2: int, seed: int) -> torch.Tensor:
     """fp32 ``[B, T, mem_dim]``: per token, the sum of one row per (route, order) of tables grown
     ``2**scale_log2`` times per route (``lng_gather_sum_scaled``); ``codes [B, T, R]`` uint8,

@@ -90,3 +90,18 @@ def test_scaled_queries_and_device_positions(dev, n):
     big = ops.memory_readout_fused_at(q * 1000, codes, 9, *args)
     assert torch.isfinite(big.float()).all()
     assert torch.isfinite(ops.memory_readout_fused_at(q * 0, codes, 9, *args).float()).all()
+
+
+@pytest.mark.parametrize("n,H", [(1, 1), (16, 3), (300, 3), (700, 2), (64, 5)])
+def test_windows_equal_their_gathered_rows(dev, n, H):
+    R = 184
+    gen, t2, t3, kv, wm = _weights(R, dev)
+    q = torch.randn(1, n, 1024, generator=gen, device=dev).to(torch.bfloat16) * 3
+    win = torch.randint(0, 16, (n, H, R), generator=gen, device=dev, dtype=torch.uint8)
+    seg = torch.randint(0, 2, (n, H), generator=gen, device=dev, dtype=torch.int32)
+    val = (torch.rand(n, H, generator=gen, device=dev) > 0.2).to(torch.uint8)
+    tail = (ops.memory_readout_pack(kv), wm, EPS, 0.125, math.log(R))
+    got = ops.memory_readout_fused_windows(q, win, seg, val, t2, t3, *tail, q_rows=q, q_eps=EPS)
+    rows = ops.route_tokens(win, [t2, t3], (2, 3), 4, segment_ids=seg, valid_tokens=val, target_length=1)
+    want = ops.memory_readout_fused_rows(q, rows.view(1, n, R, 256), *tail, q_rows=q, q_eps=EPS)
+    assert torch.equal(got, want)
