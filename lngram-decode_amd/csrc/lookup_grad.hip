@@ -4,7 +4,7 @@
 // embedding backward of its lookup, :1084-1092).
 //
 // A position's windows are named by the position that ends them.  For each order, a route's windows
-// are sorted by the table row they read (window_sort.h); a wave takes 128 consecutive windows of a
+// are sorted by the table row they read (window_sort.h); a wave takes 64 consecutive windows of a
 // route's list, 16 at a time, and all the windows of one row at once:
 //   scores   C[m][n] = T_m . g_n, one 16x16x128 bf16 matrix product: T_m the row with address bit m
 //            flipped (m < 4 order) and T_12 the row itself, g_n the windows' gradient rows.  The
@@ -17,17 +17,20 @@
 // k_lg_out sums each output's windows in the reference's order (digit ascending) and applies the
 // slope.  A route's blocks run on one XCD, whose L2 holds the route's table rows.
 // Least traffic: the gradient read once (1.54 GB at 8 x 2048 positions, 184 routes) and the scores
-// written and read once (482 MB).  Measured there: k_lg_main 574 us for order 3 and 240 us for order 2,
-// k_lg_out 84, the lists 56; the order-by-order kernels took 1.9 ms (two copies of the gradient's
-// halves, surrogate 498 + 60 and 316, table gradients 600).  k_lg_main<3> waits on its table rows: at
-// four waves a SIMD an XCD works on four routes at once, whose blocks and streams pass its 4 MB L2 (59 %
-// of L2 requests miss).  Operands loaded straight into their lanes, 64 bytes of 16 rows an instruction,
-// took 659 and 278 us: a row is loaded by 16 lanes and staged.
+// written and read once (482 MB).  Measured there: k_lg_main 545 us for order 3 and 224 us for order 2,
+// k_lg_out 85, the lists 56, k_lg_merge 50; the order-by-order kernels took 1.9 ms (two copies of the
+// gradient's halves, surrogate 498 + 60 and 316, table gradients 600).  k_lg_main<3> waits on its table
+// rows: an XCD's 512 waves work on as many routes at once as it takes to fill them, 1 MB of rows each,
+// beside the gradient's and the scores' streams in its 4 MB L2.  Chunks of 128 windows keep four routes
+// in flight (574 and 240 us, 59 % of L2 requests miss), of 64 two; with 48 and 32 the rows cut by chunk
+// ends cost more than that gives (+12 and +24 us over all).  Rows requested two runs ahead gave nothing
+// (578).  Operands loaded straight into their lanes, 64 bytes of 16 rows an instruction, took 659 and
+// 278 us: a row is loaded by 16 lanes and staged.
 #include "window_sort.h"
 
 namespace lng {
 
-constexpr int LG_CHUNK = 128;  // windows of a wave
+constexpr int LG_CHUNK = 64;  // windows of a wave, an entry a lane
 
 // A staged tile: 16 rows of 16 16-byte pieces, piece p of row n in slot p ^ lg_swz(n).  Rows are loaded
 // and stored by 16 lanes each (whole lines) and read as matrix operands by lane (n, kg) in pieces
@@ -147,9 +150,7 @@ __global__ __launch_bounds__(256) void k_lg_main(LgArgs a) {
   const int lo = c * LG_CHUNK, nw = min(LG_CHUNK, total - lo);
   if (nw <= 0) return;
   const uint32_t* pm = o.perm + static_cast<int64_t>(r) * a.W;
-  uint32_t ent[2];  // the chunk's entries, 64 a register
-#pragma unroll
-  for (int i = 0; i < 2; ++i) ent[i] = pm[lo + min(64 * i + lane, nw - 1)];
+  const uint32_t ent = pm[lo + min(lane, nw - 1)];  // the chunk's entries
   const bf16* grad = a.grad + (ORDER - 2) * 128 + static_cast<int64_t>(r) * a.gstride + col * 8;
   const int64_t wstride = static_cast<int64_t>(a.R) * a.gstride;
   const bf16* table = o.table + (static_cast<int64_t>(r) << SH) * 128 + col * 8;
@@ -161,8 +162,7 @@ __global__ __launch_bounds__(256) void k_lg_main(LgArgs a) {
   char* gst = stage[wave][0];
   char* tst = stage[wave][1];
   auto at = [&](int q) {  // entry q of the chunk (q may differ between lanes)
-    const uint32_t x = __shfl(static_cast<int>(ent[0]), q & 63), y = __shfl(static_cast<int>(ent[1]), q & 63);
-    return q < 64 ? x : y;
+    return static_cast<uint32_t>(__shfl(static_cast<int>(ent), q));
   };
   // 16 rows into registers, 4 a load and 16 lanes a row: the gradients of windows 16 b ..; the table rows
   // of one address (row m has address bit m flipped, rows 4 ORDER .. 15 are the row itself)
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void k_lg_main(LgArgs a) {
   };
   const int nb = (nw + 15) / 16;
   u32x4 g[4], t[4];
-  uint32_t trow = __builtin_amdgcn_readfirstlane(ent[0]) & AM;  // the row that t holds
+  uint32_t trow = __builtin_amdgcn_readfirstlane(ent) & AM;  // the row that t holds
   bool fresh = true;                                            // t is not staged yet
   load_grad(0, g);
   if (scores != nullptr) load_rows(trow, t);
@@ -230,8 +230,7 @@ __global__ __launch_bounds__(256) void k_lg_main(LgArgs a) {
         // the next row's table rows are requested under this one's products
         const int q = 16 * b + j;
         if (q < nw) {
-          const uint32_t nxt =
-              __builtin_amdgcn_readlane(q < 64 ? ent[0] : ent[1], q & 63) & AM;
+          const uint32_t nxt = __builtin_amdgcn_readlane(ent, q) & AM;
           if (nxt != trow) {
             load_rows(nxt, t);
             trow = nxt;
@@ -267,11 +266,13 @@ __global__ __launch_bounds__(256) void k_lg_main(LgArgs a) {
 }
 
 // Rows cut by chunks: the chunk that a cut row begins in adds its part and the following chunks' in
-// order.  Rows that no window names are cleared.  A block takes 256 rows and a share of the chunks.
+// order.  Rows that no window names are cleared.  A block takes 256 rows and a share of the chunks; both
+// orders in one launch (50 us at 8 x 2048; one after the other 62, each waiting on dependent loads).
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_lg_merge(LgArgs a) {
+__device__ __forceinline__ void lg_merge(const LgArgs& a) {
   constexpr int SH = 4 * ORDER;
   const LgOrder& o = a.o[ORDER - 2];
+  if (o.out == nullptr) return;
   const int r = blockIdx.y;
   const uint32_t* st = o.start + static_cast<int64_t>(r) * ((1 << SH) + 1);
   bf16* out = o.out + (static_cast<int64_t>(r) << SH) * 128;
@@ -299,6 +300,12 @@ __global__ __launch_bounds__(256) void k_lg_merge(LgArgs a) {
     const bf16x2 v{static_cast<bf16>(s.x), static_cast<bf16>(s.y)};
     reinterpret_cast<bf16x2*>(out + static_cast<int64_t>(row) * 128)[lane] = v;
   }
+}
+__global__ __launch_bounds__(256) void k_lg_merge(LgArgs a) {
+  if (blockIdx.z != 0)
+    lg_merge<3>(a);
+  else
+    lg_merge<2>(a);
 }
 
 // grad_q[b, t, r, k] = the orders' sums, each slope * (((0 + S0(t)[k]) + S1(t)[k]) + ..) in the output's
@@ -443,8 +450,7 @@ extern "C" int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t g
   const unsigned blocks = static_cast<unsigned>(8 * cdiv(R, 8) * cdiv(a.chunks, 4));
   if (want_q || grad_table2) k_lg_main<2><<<blocks, 256, 0, s>>>(a);
   if (want_q || grad_table3) k_lg_main<3><<<blocks, 256, 0, s>>>(a);
-  if (grad_table2) k_lg_merge<2><<<dim3(16, static_cast<unsigned>(R)), 256, 0, s>>>(a);
-  if (grad_table3) k_lg_merge<3><<<dim3(16, static_cast<unsigned>(R)), 256, 0, s>>>(a);
+  if (grad_table2 || grad_table3) k_lg_merge<<<dim3(16, static_cast<unsigned>(R), 2), 256, 0, s>>>(a);
   if (grad_q) {
     const dim3 og(static_cast<unsigned>(cdiv(a.W, 64)), static_cast<unsigned>(cdiv(R, 16)));
     const float al_ = want_q ? alpha : 0.f;

@@ -1,5 +1,5 @@
 """The one-pass backward of the training lookup (``lng_lookup_grad``) against the order-by-order
-kernels and the fp64 oracle, at the edges of its 128-window chunks and 16-window batches.
+kernels and the fp64 oracle, at the edges of its 64-window chunks and 16-window batches.
 
 Tolerances: the route-logit gradient agrees with the direct kernels to fp32 rounding (norm-relative
 1e-6: sums of 128 exact products in another order) and with fp64 to 1e-5; a table row of n windows
@@ -22,9 +22,10 @@ CASES = [
     (1, 2, 3, 0, "random", torch.float32, torch.uint8, False),      # one order-2 window, none of order 3
     (2, 3, 9, 1, "random", torch.bfloat16, torch.int32, False),
     (1, 18, 5, 0, "constant", torch.float32, torch.uint8, False),   # 17 and 16 windows of one row
+    (1, 66, 8, 0, "random", torch.float32, torch.uint8, True),      # 65 and 64 windows: chunk edge
     (1, 130, 8, 0, "random", torch.float32, torch.int64, True),     # 129 and 128 windows: chunk edge
     (3, 131, 17, 2, "few", torch.float32, torch.uint8, False),      # rows cut by chunks
-    (2, 700, 3, 0, "constant", torch.float32, torch.uint8, False),  # one row over eleven chunks
+    (2, 700, 3, 0, "constant", torch.float32, torch.uint8, False),  # one row over 22 chunks
     (5, 391, 11, 0, "random", torch.bfloat16, torch.uint8, True),
     (1, 64, 256, 0, "few", torch.float32, torch.uint8, False),
 ]
