@@ -125,6 +125,9 @@ int lng_route_tokens(const void* codes, int codes_dtype, int64_t B, int64_t T, i
                      int32_t bits, const void* const* tables, int table_dtype, int32_t mem_dim,
                      const int32_t* segment_ids, const uint8_t* valid_tokens, int32_t target_length,
                      void* out, void* stream);
+/* Reads `bytes` of table rows in address order, so that a following gather of most of them finds them in
+ * the last-level cache instead of missing on them one by one.  Changes nothing. */
+int lng_prefetch_rows(const void* rows, size_t bytes, void* stream);
 
 /* The n-gram windows of a draft tree's nodes for the memory block of tree verification
  * (tree_ngram_codes / tree_route_tokens, drafting/tree.py:114-136, as tree_verify_step uses them,

@@ -133,6 +133,7 @@ SIGNATURES = {
                                      _i32, _f, _f, _int, _p, ctypes.c_size_t, _p, _int, _p]),
     "lng_table_grad": (_int, [_p, _int, _p, _int, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i64, _p, _p]),
     "lng_table_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32]),
+    "lng_prefetch_rows": (_int, [_p, ctypes.c_size_t, _p]),
     "lng_table_grad_rows": (_int, [_p, _int, _i64, _p, _int, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i64, _p,
                                    ctypes.c_size_t, _p, _int, _p]),
     "lng_lookup_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32, _int, _int]),

@@ -315,6 +315,29 @@ def online_mix(keys: torch.Tensor, nxt: torch.Tensor, q: torch.Tensor, deadline:
     return out
 
 
+# A gather whose output passes the caches (the line of the tiled gather's non-temporal stores) and whose
+# positions outnumber an order's rows per route reads most of its tables' rows: they are read in order
+# first, if they fit the 256 MB last-level cache together with the rows being written.  With fewer
+# positions the pass would read rows that no window names; tables past that cache would push their own
+# first rows out again.
+_PREFETCH_OUT = 32 << 20
+_PREFETCH_TABLES = 224 << 20
+
+
+def _prefetch_tables(tabs, orders, bits: int, route_start: int, route_end: int, positions: int, stream) -> None:
+    blocks = []
+    for tb, order in zip(tabs, orders):
+        if positions >= 1 << (bits * order):
+            rows = tb.shape[0]
+            lo, hi = (min(r << (bits * order), rows) for r in (route_start, route_end))
+            row_bytes = tb.shape[1] * tb.element_size()
+            blocks.append((tb.data_ptr() + lo * row_bytes, (hi - lo) * row_bytes))
+    if sum(n for _, n in blocks) <= _PREFETCH_TABLES:
+        for at, n in blocks:
+            if n:
+                check(lib().lng_prefetch_rows(at, n, stream), "prefetch_rows")
+
+
 def route_tokens(codes: torch.Tensor, tables, orders, bits: int, route_start: int = 0, route_end: int | None = None,
                  segment_ids=None, valid_tokens=None, target_length: int | None = None) -> torch.Tensor:
     """Route tokens ``[B, T_out, R', len(orders)*mem_dim]`` gathered from ``tables`` (one per order)."""
@@ -332,6 +355,8 @@ def route_tokens(codes: torch.Tensor, tables, orders, bits: int, route_start: in
     t_out = t if not target_length else int(target_length)
     out = torch.empty(b, t_out, route_end - route_start, len(orders) * mem_dim, dtype=dt, device=dev)
     tp = (ctypes.c_void_p * len(tabs))(*[tb.data_ptr() for tb in tabs])
+    if out.numel() * out.element_size() > _PREFETCH_OUT and len(tabs) == len(orders) and min(orders) > 0:
+        _prefetch_tables(tabs, orders, bits, route_start, route_end, b * t_out, _stream(dev))
     check(lib().lng_route_tokens(_ptr(cc), dtype_code(cc.dtype), b, t, r, route_start, route_end, _orders(orders),
                                  len(orders), bits, tp, dtype_code(dt), mem_dim, _ptr(seg), _ptr(val),
                                  int(target_length or 0), _ptr(out), _stream(dev)), "route_tokens")

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from lngram_hip import ops
+from lngram_hip._lib import check
 from oracle import memory as om
 
 pytestmark = pytest.mark.gpu
@@ -23,6 +24,7 @@ CASES = [
     (9, 129, 40, 1, 39, 32, (2, 3), 4, torch.float32, None, True),
     (2, 300, 97, 0, 97, 24, (2, 3), 4, torch.bfloat16, None, True),      # 48 bytes: one thread a piece
     (5, 391, 33, 0, 33, 128, (2, 3), 4, torch.bfloat16, None, True),     # 33.0 MB: non-temporal stores
+    (1, 4100, 20, 2, 19, 128, (2, 3), 4, torch.bfloat16, None, True),    # tables read ahead (4096 rows a route)
 ]
 
 
@@ -46,3 +48,11 @@ def test_rows_equal_the_oracle(dev, case, codes_dtype):
                       for i, tab in enumerate(tables)], -1)[:, :, r0:r1]
     want = want if tail is None else want[:, -tail:]
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("lo,n", [(0, 0), (1, 15), (0, 16), (8, 40), (3, 70001), (0, 64 << 20)])
+def test_reading_ahead_changes_nothing(dev, lo, n):
+    x = torch.arange(lo + n + 32, device=dev).to(torch.uint8)
+    want = x.clone()
+    check(ops.lib().lng_prefetch_rows(x.data_ptr() + lo, n, torch.cuda.current_stream(dev).cuda_stream), "prefetch_rows")
+    assert torch.equal(x, want)
