@@ -92,14 +92,18 @@ __device__ __forceinline__ float sumsq8(const bf16x8 v, float acc) {
 // and u (rows 0..15, phase B -> C); per wave the token's row indices [order][route parity]
 // [route / 2] (-1 = zero row); the memory-norm weight.
 //
-// SPLIT: the block's FR_TOK waves share one token (tok0), wave w taking route chunks w, w + FR_TOK, ..;
-// their softmax states and weighted sums are merged in LDS before phase C.
+// SPLIT: the block's FR_TOK waves share one token (tok0).  In a round of FR_TOK chunks wave w gathers and
+// scores chunk w; with every chunk's maximum in LDS it forms its probabilities under the running maximum
+// that a single wave would have there, and hands them over in LDS; each wave then sums 16 / FR_TOK of the
+// 16 feature tiles over the round's chunks in their order.  So a token's output has the same bits
+// however its routes are spread.
 template <int FR_TOK>
 struct ReadoutLds {
   __attribute__((aligned(16))) bf16 xs[FR_TOK * FR_TS];
   __attribute__((aligned(16))) int32_t rowsh[FR_TOK][2][4][FR_RQ + 4];  // rows 272 B apart
   __attribute__((aligned(16))) bf16 wms[FR_DT];
   float qscale[FR_TOK];
+  float cmax[FR_TOK][16];  // SPLIT: the round's chunk maxima by head
 };
 
 template <int FR_TOK, bool SPLIT>
@@ -291,18 +295,18 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
   for (int kk = 0; kk < 8; ++kk) qb[kk] = *reinterpret_cast<const bf16x8*>(&XS(SPLIT ? 0 : w, li, fr_col(lg, kk)));
   if (SPLIT) __syncthreads();  // every wave has the query before wave 0's rows replace it
 
+  // the running maximum and sum start at the sink logit, the sums at zero
+  constexpr float L2E = 1.4426950408889634f;
+  constexpr int NACC = SPLIT ? 16 / FR_TOK : 16;  // feature tiles of 16 that this wave sums
   float m_run = sink, l_part = 0.f;
-  f32x4 acc[16];
+  f32x4 acc[NACC];
 #pragma unroll
-  for (int ft = 0; ft < 16; ++ft) acc[ft] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ft = 0; ft < NACC; ++ft) acc[ft] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int c0 = c_first; c0 < R; c0 += C_STEP) {
-    stash(g);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (c0 + C_STEP < R) gather(c0 + C_STEP, g);
-
-    // scores: A = route rows (lane: route 16tt + li, features fr_col(lg, kk) ..+8), B = qkw
+  // scores of the chunk staged in this wave's region: s[tt][i] of route c0 + 16tt + 4lg + i and head li,
+  // sD the route's RMS scale; the result is the head's maximum over the chunk
+  auto score = [&](int c0, float (&s)[2][4], float (&sD)[2][4]) {
+    // A = route rows (lane: route 16tt + li, features fr_col(lg, kk) ..+8), B = qkw
     float sr[2];
     f32x4 sc[2];
 #pragma unroll
@@ -320,8 +324,6 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) sc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[kk], qb[kk], sc[tt], 0, 0, 0);
     }
-    // sc[tt][i]: route c0 + 16tt + 4lg + i, head hg = li
-    float sD[2][4], s[2][4];
     float cmax = -INFINITY;
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
@@ -333,20 +335,29 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
         cmax = fmaxf(cmax, s[tt][i]);
       }
     cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
-    const float m_new = fmaxf(m_run, cmax);
-    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * 1.4426950408889634f);
-    m_run = m_new;
-    float psum = 0.f;
+    return fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+  };
+  // probabilities under the running maximum m (times the row scales: the P of P . X) and their sum
+  auto probs = [&](const float (&s)[2][4], const float (&sD)[2][4], float m, float& psum) {
     bf16x8 pa;
+    psum = 0.f;
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f((s[tt][i] - m_new) * 1.4426950408889634f);
+        const float p = __builtin_amdgcn_exp2f((s[tt][i] - m) * L2E);
         psum += p;
         pa[4 * tt + i] = static_cast<bf16>(p * sD[tt][i]);
       }
+    return pa;
+  };
+  // the state after a chunk of wave region k: maximum m_new, sum psum, P pa; U += P . X with X transposed
+  // out of LDS: ds_read_b64_tr_b16 gives lane i of each 16-lane group element i%4 of the 8-byte chunks
+  // addressed by lanes i/4 + 4c (c = 0..3), i.e. X[4g + c][16ft + i] here.  The halves are joined with a
+  // shuffle (element-wise bit casts of the returned vector are miscompiled to element 0).
+  auto add_chunk = [&](int k, float m_new, float psum, const bf16x8 pa, int ft0) {
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * L2E);
+    m_run = m_new;
     l_part = l_part * alpha + psum;
     float aD[4];
 #pragma unroll
@@ -354,26 +365,68 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
     // the running max seldom moves past the sink logit: rescale only when some lane's did
     if (__ballot(alpha != 1.f) != 0ull) {
 #pragma unroll
-      for (int ft = 0; ft < 16; ++ft)
+      for (int ft = 0; ft < NACC; ++ft)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[ft][i] *= aD[i];
     }
-    // U += P . X with X transposed out of LDS: ds_read_b64_tr_b16 gives lane i of each
-    // 16-lane group element i%4 of the 8-byte chunks addressed by lanes i/4 + 4c
-    // (c = 0..3), i.e. X[4g + c][16ft + i] here.  The halves are joined with a shuffle
-    // (element-wise bit casts of the returned vector are miscompiled to element 0).
 #pragma unroll
-    for (int ft = 0; ft < 16; ++ft) {
-      const int col = 16 * ft + 4 * (li & 3);
+    for (int ft = 0; ft < NACC; ++ft) {
+      const int col = 16 * (ft0 + ft) + 4 * (li & 3);
       const bf16x4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-          (__attribute__((address_space(3))) bf16x4*)(&XS(w, 4 * lg + (li >> 2), col)));
+          (__attribute__((address_space(3))) bf16x4*)(&XS(k, 4 * lg + (li >> 2), col)));
       const bf16x4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-          (__attribute__((address_space(3))) bf16x4*)(&XS(w, 16 + 4 * lg + (li >> 2), col)));
+          (__attribute__((address_space(3))) bf16x4*)(&XS(k, 16 + 4 * lg + (li >> 2), col)));
       const bf16x8 b = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
       acc[ft] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, b, acc[ft], 0, 0, 0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+  };
+
+  if constexpr (SPLIT) {
+    auto& cmx = lds.cmax;
+    // P and sums of the round's chunks, over the row indices: every wave has issued its last gather
+    // (a round's gathers go out before its first barrier)
+    bf16x8* ph = reinterpret_cast<bf16x8*>(&rowsh[0][0][0][0]);
+    float* sh = reinterpret_cast<float*>(ph + 64 * FR_TOK);
+    static_assert(64 * FR_TOK * (sizeof(bf16x8) + sizeof(float)) <= sizeof(lds.rowsh), "hand-off fits the row indices");
+    static_assert(2 * 32 * FR_TOK >= FR_MAXR, "row indices are read in the first round at the latest");
+    for (int cb = 0; cb < R; cb += C_STEP) {
+      const int c0 = cb + 32 * w;
+      float s[2][4], sD[2][4], cmax = -INFINITY;
+      if (c0 < R) {
+        stash(g);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (c0 + C_STEP < R) gather(c0 + C_STEP, g);
+        cmax = score(c0, s, sD);
+      }
+      if (lg == 0) cmx[w][li] = cmax;
+      __syncthreads();
+      const int n_ch = min(FR_TOK, (R - cb + 31) >> 5);  // chunks of this round
+      if (w < n_ch) {
+        float m = m_run, psum;
+        for (int k = 0; k <= w; ++k) m = fmaxf(m, cmx[k][li]);
+        const bf16x8 pa = probs(s, sD, m, psum);
+        ph[w * 64 + lane] = pa;
+        sh[w * 64 + lane] = psum;
+      }
+      __syncthreads();
+      for (int k = 0; k < n_ch; ++k)
+        add_chunk(k, fmaxf(m_run, cmx[k][li]), sh[k * 64 + lane], ph[k * 64 + lane], NACC * w);
+      __syncthreads();  // before the next round's rows, or the value projection's operand, replace these
+    }
+  } else {
+    for (int c0 = 0; c0 < R; c0 += 32) {
+      stash(g);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (c0 + 32 < R) gather(c0 + 32, g);
+      float s[2][4], sD[2][4], psum;
+      const float m_new = fmaxf(m_run, score(c0, s, sD));
+      const bf16x8 pa = probs(s, sD, m_new, psum);
+      add_chunk(w, m_new, psum, pa, 0);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 
   // phase-C operands (wave w: head h = w & 3, head-dim tiles dt0 .. dt0 + NDT-1), loaded before
@@ -389,57 +442,17 @@ __device__ __forceinline__ void readout_body(ReadoutLds<FR_TOK>& lds, int64_t to
   // normalise and stage u = w_mem . U / l for the value projection
   float lt = l_part + __shfl_xor(l_part, 16, 64);
   lt += __shfl_xor(lt, 32, 64);
-  if constexpr (SPLIT) {
-    // head li's (m, l) of every wave (every m is at least the sink), then each wave's sums scaled to
-    // the common maximum and total, as [head][256] fp32 in its region, are added up
-    float2* ml = reinterpret_cast<float2*>(&rowsh[0][0][0][0]);  // the row indices are spent
-    __syncthreads();
-    if (lg == 0) ml[w * 16 + li] = float2{m_run, lt};
-    __syncthreads();
-    float m_all = sink;
+  lt += __builtin_amdgcn_exp2f((sink - m_run) * L2E);
+  const float inv = 1.0f / lt;
+  float iD[4];
 #pragma unroll
-    for (int k = 0; k < FR_TOK; ++k) m_all = fmaxf(m_all, ml[k * 16 + li].x);
-    float l_all = __builtin_amdgcn_exp2f((sink - m_all) * 1.4426950408889634f);
+  for (int i = 0; i < 4; ++i) iD[i] = __shfl(inv, 4 * lg + i, 64);
 #pragma unroll
-    for (int k = 0; k < FR_TOK; ++k)
-      l_all += ml[k * 16 + li].y * __builtin_amdgcn_exp2f((ml[k * 16 + li].x - m_all) * 1.4426950408889634f);
-    const float fac = __builtin_amdgcn_exp2f((m_run - m_all) * 1.4426950408889634f) / l_all;
-    float fD[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fD[i] = __shfl(fac, 4 * lg + i, 64);
-    float* mine = reinterpret_cast<float*>(&XS(w, 0, 0));  // 16 rows of 272 fp32: the region's 32 x 544 B
-#pragma unroll
-    for (int ft = 0; ft < 16; ++ft)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) mine[(4 * lg + i) * 272 + 16 * ft + li] = acc[ft][i] * fD[i];
-    __syncthreads();
-    // a thread: one feature of 64 / FR_TOK heads
-    constexpr int NH = 64 / FR_TOK;
-    const int f = threadIdx.x & 255, h0 = (threadIdx.x >> 8) * NH;
-    float u[NH];
-#pragma unroll
-    for (int hd = 0; hd < NH; ++hd) {
-      u[hd] = 0.f;
-#pragma unroll
-      for (int k = 0; k < FR_TOK; ++k) u[hd] += reinterpret_cast<const float*>(&XS(k, 0, 0))[(h0 + hd) * 272 + f];
-    }
-    __syncthreads();
+  for (int ft = 0; ft < NACC; ++ft) {
+    const int f = 16 * (SPLIT ? NACC * w + ft : ft) + li;
     const float wm = to_f32(wms[f]);
 #pragma unroll
-    for (int hd = 0; hd < NH; ++hd) XS(0, h0 + hd, f) = static_cast<bf16>(u[hd] * wm);
-  } else {
-    lt += __builtin_amdgcn_exp2f((sink - m_run) * 1.4426950408889634f);
-    const float inv = 1.0f / lt;
-    float iD[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) iD[i] = __shfl(inv, 4 * lg + i, 64);
-#pragma unroll
-    for (int ft = 0; ft < 16; ++ft) {
-      const int f = 16 * ft + li;
-      const float wm = to_f32(wms[f]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) XS(w, 4 * lg + i, f) = static_cast<bf16>(acc[ft][i] * iD[i] * wm);
-    }
+    for (int i = 0; i < 4; ++i) XS(SPLIT ? 0 : w, 4 * lg + i, f) = static_cast<bf16>(acc[ft][i] * iD[i] * wm);
   }
   __syncthreads();
 
