@@ -9,6 +9,8 @@
 // fp32 runs on fp32 MFMA tiles; mixed types and odd K on a VALU tile kernel.
 #include "gemm_tile.h"
 
+#include <type_traits>
+
 namespace lng {
 
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_ROUTER = 2 };
@@ -767,13 +769,13 @@ __global__ __launch_bounds__(512, 1) void k_gemm_proj_bf16(const bf16* __restric
 // ---------------------------------------------------------------------------------------
 // Tiles for more rows than the skinny kernel's and fewer than fill the chip with 256-row tiles (K % 64
 // == 0): BN x BM of 4 waves (gemm_tile.h).  Bound by the latency of a K stage's loads while blocks are
-// few, then by LDS reads; rowsq (row-statistics partials, as k_gemm_proj_bf16 writes them) needs BN =
+// few, then by LDS reads; rowsq (row-statistics partials, as the 256-row kernels write them) needs BN =
 // 128.  XRMS scales row m by rsqrt(mean(x_m^2) + eps) before rounding.
 template <int EPI, bool XRMS, int BN, int BM, int WN, int WM>
 __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, const bf16* __restrict__ X, int64_t N,
                                                    int64_t M, int64_t K, int n_tiles, void* __restrict__ out,
                                                    float* __restrict__ logits, void* __restrict__ codes, int codes_dt,
-                                                   int64_t routes, float* __restrict__ rowsq, float x_eps) {
+                                                   int64_t routes, float* __restrict__ rowsq, int chains, float x_eps) {
   using G = TileGemm<bf16, BN, BM, WN, WM, 1, 3>;
   __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
   const int nt = static_cast<int>(blockIdx.x) % n_tiles;
@@ -783,15 +785,21 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wn = wave % WN, wm = wave / WN;
   const int rsel = lane & 15, psel = lane >> 4;
-  float ps[G::FM];
+  // row statistics: the tile's bf16 rows go through LDS (the ring, once every wave has left it), rows
+  // of 32 groups of 4 columns, 264 B apart
+  constexpr int RLD = BN + 4;
+  static_assert(BN != 128 || BM * RLD <= G::LDS_ELEMS, "the rows fit the ring");
+  const bool stats = EPI == EPI_BF16 && BN == 128 && rowsq != nullptr;
+  if (stats) __syncthreads();
 #pragma unroll
   for (int j = 0; j < G::FM; ++j) {
-    const int64_t m = m0 + wm * (BM / WM) + j * 16 + rsel;
+    const int ml = wm * (BM / WM) + j * 16 + rsel;
+    const int64_t m = m0 + ml;
     const float rs = XRMS ? __builtin_amdgcn_rsqf(g.xss[j] / static_cast<float>(K) + x_eps) : 1.f;
-    ps[j] = 0.f;
 #pragma unroll
     for (int i = 0; i < G::FN; ++i) {
-      const int64_t n = n0 + wn * (BN / WN) + i * 16 + 4 * psel;
+      const int nl = wn * (BN / WN) + i * 16 + 4 * psel;
+      const int64_t n = n0 + nl;
       f32x4 v = g.acc[i][j];
       if (XRMS) {
 #pragma unroll
@@ -800,13 +808,7 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
       if (EPI == EPI_BF16) {
         const bf16x4 pk = {static_cast<bf16>(v[0]), static_cast<bf16>(v[1]), static_cast<bf16>(v[2]),
                            static_cast<bf16>(v[3])};
-        if (rowsq) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float r = static_cast<float>(pk[e]);
-            ps[j] = fmaf(r, r, ps[j]);
-          }
-        }
+        if (stats) *reinterpret_cast<bf16x4*>(ring + ml * RLD + nl) = pk;
         if (m < M && n < N) *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + m * N + n) = pk;  // N % 4 == 0
       } else if (m < M && n < N) {
         if (logits) *reinterpret_cast<f32x4*>(logits + m * N + n) = v;
@@ -820,26 +822,35 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
       }
     }
   }
-  if (EPI == EPI_BF16 && rowsq) {
-    // partial nt of row m: its 128 columns, summed over the lanes of a row, then over the WN waves
-    float* red = reinterpret_cast<float*>(ring);
-    __syncthreads();  // every wave has left the ring
-#pragma unroll
-    for (int j = 0; j < G::FM; ++j) {
-      float v = ps[j];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      if (psel == 0) red[wn * BM + wm * (BM / WM) + j * 16 + rsel] = v;
-    }
+  if (stats) {
+    // partial nt of row m: its 128 columns (zeros past N) in `chains` chains, chain c the column groups
+    // c, c + chains, .. in order: the order of the lanes of k_gemm_proj_bf16 (2) or k_gemm_dma256_bf16 (4),
+    // so that a shape's statistics do not depend on the tile that forms them
     __syncthreads();
-    if (static_cast<int>(threadIdx.x) < BM && m0 + threadIdx.x < M) {
+    auto partial = [&](auto n_chains) {
+      constexpr int C = decltype(n_chains)::value;
+      const int ml = static_cast<int>(threadIdx.x) / C, c = static_cast<int>(threadIdx.x) % C;
+      if (ml >= BM) return;
+      bf16x4 p[32 / C];
+#pragma unroll
+      for (int u = 0; u < 32 / C; ++u) p[u] = *reinterpret_cast<const bf16x4*>(ring + ml * RLD + 4 * (c + C * u));
       float v = 0.f;
 #pragma unroll
-      for (int w = 0; w < WN; ++w) v += red[w * BM + threadIdx.x];
-      rowsq[static_cast<int64_t>(nt) * M + m0 + threadIdx.x] = v;
-      // the partials come in pairs (256 columns): an odd last one has an empty partner
-      if (nt == n_tiles - 1 && (n_tiles & 1)) rowsq[static_cast<int64_t>(nt + 1) * M + m0 + threadIdx.x] = 0.f;
-    }
+      for (int u = 0; u < 32 / C; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v = fmaf(static_cast<float>(p[u][e]), static_cast<float>(p[u][e]), v);
+#pragma unroll
+      for (int d = 1; d < C; d *= 2) v += __shfl_xor(v, d, 64);
+      if (c == 0 && m0 + ml < M) {
+        rowsq[static_cast<int64_t>(nt) * M + m0 + ml] = v;
+        // the partials come in pairs (256 columns): an odd last one has an empty partner
+        if (nt == n_tiles - 1 && (n_tiles & 1)) rowsq[static_cast<int64_t>(nt + 1) * M + m0 + ml] = 0.f;
+      }
+    };
+    if (chains == 2)
+      partial(std::integral_constant<int, 2>{});
+    else
+      partial(std::integral_constant<int, 4>{});
   }
 }
 
@@ -1095,14 +1106,18 @@ static int pick_tile(int64_t N, int64_t M, int64_t K, bool rowsq) {
   return blocks(128, 64) <= 768 ? TILE_128_64 : TILE_NONE;
 }
 
+// The projection kernel takes M >= 1024 (at least 4 tiles of rows), K % 64 == 0 and N % 8 == 0.
+static bool proj_shape(int64_t N, int64_t M, int64_t K) { return M >= 1024 && N >= 64 && K % PK == 0 && N % 8 == 0; }
+
 template <int EPI, bool XRMS>
 static int launch_tile(int tile, const bf16* w, const bf16* x, int64_t N, int64_t M, int64_t K, void* out,
                        float* logits, void* codes, int codes_dt, int64_t routes, float* rowsq, float x_eps,
                        hipStream_t s) {
+  const int chains = proj_shape(N, M, K) ? 2 : 4;  // of the 256-row kernel that the shape would take
   auto go = [&](auto* kern, int64_t bn, int64_t bm) {
     const int n_tiles = static_cast<int>(cdiv(N, bn));
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, x, N, M, K,
-                       n_tiles, out, logits, codes, codes_dt, routes, rowsq, x_eps);
+                       n_tiles, out, logits, codes, codes_dt, routes, rowsq, chains, x_eps);
     return check_launch("gemm_bf16_tile");
   };
   if (EPI == EPI_BF16 && tile == TILE_128_32) return go(&k_gemm_tile<EPI, XRMS, 128, 32, 4, 1>, 128, 32);
@@ -1150,9 +1165,6 @@ static int launch_mfma(const bf16* w, const bf16* x, int64_t N, int64_t M, int64
                        routes);
   return check_launch("gemm_bf16");
 }
-
-// The projection kernel takes M >= 1024 (at least 4 tiles of rows), K % 64 == 0 and N % 8 == 0.
-static bool proj_shape(int64_t N, int64_t M, int64_t K) { return M >= 1024 && N >= 64 && K % PK == 0 && N % 8 == 0; }
 
 static int launch_proj(const bf16* w, const bf16* x, int64_t N, int64_t M, int64_t K, bf16* out, float* rowsq,
                        hipStream_t s, bool x_rms = false, float x_eps = 0.f) {

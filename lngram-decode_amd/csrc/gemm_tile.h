@@ -29,7 +29,7 @@ struct TileGemm {
   static_assert((SLOTS - 2) * LOADS <= 60, "vmcnt");
 
   f32x4 acc[FN][FM];
-  float xss[FM];  // XRMS: this lane's share of the sum of squares of x row 16 j + (lane & 15)
+  float xss[FM];  // XRMS: sum of squares of x row 16 j + (lane & 15)
 
   __device__ __forceinline__ static f32x4 mma(Frag a, Frag b, f32x4 c) {
     if constexpr (sizeof(T) == 2) {
@@ -120,21 +120,41 @@ struct TileGemm {
             for (int j = 0; j < FM; ++j) acc[i][j] = mma(a[i], b[j], acc[i][j]);
         }
         if constexpr (XRMS) {
+          // a row's sum in two chains, its even and its odd pieces in order, as the lanes of
+          // k_gemm_proj_bf16's 32x32x16 fragments form it: lane groups 0, 1 and 2, 3 exchange pieces and
+          // take one of two row fragments each (of a last single one, the same)
 #pragma unroll
-          for (int j = 0; j < FM; ++j)
+          for (int j = 0; j < FM; j += 2) {
+            const u32x4 lo = __builtin_bit_cast(u32x4, b[j]), hi = __builtin_bit_cast(u32x4, b[j + 1 < FM ? j + 1 : j]);
+            uint32_t pc[2][4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              const bf16x2 v = {b[j][2 * q], b[j][2 * q + 1]};
-              xss[j] = __builtin_amdgcn_fdot2_f32_bf16(v, v, xss[j], false);
+              const auto r = __builtin_amdgcn_permlane32_swap(lo[q], hi[q], false, false);
+              pc[0][q] = r[0];
+              pc[1][q] = r[1];
             }
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const bf16x2 v = __builtin_bit_cast(bf16x2, pc[half][q]);
+                xss[j] = __builtin_amdgcn_fdot2_f32_bf16(v, v, xss[j], false);
+              }
+          }
         }
       }
     }
     if constexpr (XRMS) {
 #pragma unroll
-      for (int j = 0; j < FM; ++j) {  // the row's other k pieces
-        xss[j] += __shfl_xor(xss[j], 16, 64);
-        xss[j] += __shfl_xor(xss[j], 32, 64);
+      for (int j = 0; j < FM; j += 2) {
+        xss[j] += __shfl_xor(xss[j], 16, 64);  // the row's other pieces
+        if (j + 1 < FM) {
+          const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, xss[j]),
+                                                          __builtin_bit_cast(uint32_t, xss[j]), false, false);
+          const uint32_t r0 = r[0], r1 = r[1];  // (a bit cast of the element itself takes element 0)
+          xss[j] = __builtin_bit_cast(float, r0);
+          xss[j + 1] = __builtin_bit_cast(float, r1);
+        }
       }
     }
   }

@@ -1,0 +1,50 @@
+"""A row of a bf16 projection has the same bits in every tile that may form it: its product, its row
+statistics and its row scale, against the 256-row kernels with the row among many others (M past the
+tiles' range), or with K padded by zeros to a multiple of 32 that the tiles do not take."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from lngram_hip import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(m, k, n, dev):
+    gen = torch.Generator().manual_seed(m + k + n)
+    return (torch.randn(m, k, generator=gen).to(torch.bfloat16).to(dev),
+            torch.randn(n, k, generator=gen).to(torch.bfloat16).to(dev))
+
+
+@pytest.mark.parametrize("k,n", [(1024, 1024), (256, 1000), (64, 136)])
+def test_rows_of_the_projection_tiles(dev, k, n):
+    x, w = _inputs(50000 if n < 200 else 8192, k, n, dev)      # past the tiles: 256-row projection kernel
+    want, stats, scaled = ops.linear(x, w), ops.linear_rowsq(x, w)[1], ops.linear_rowscale(x, w, 1e-5)
+    for m in (1024, 1281, 1500, 2331, 4000, 6000):             # 64 x 32, 64 x 64, 128 x 32 and 128 x 64 tiles
+        y, sq = ops.linear_rowsq(x[:m], w)
+        assert torch.equal(y, want[:m]) and torch.equal(ops.linear(x[:m], w), want[:m]), m
+        assert torch.equal(sq, stats[:, :m]), m
+        assert torch.equal(ops.linear_rowscale(x[:m], w, 1e-5), scaled[:m]), m
+
+
+@pytest.mark.parametrize("m,k,n", [(65, 64, 1024), (200, 1024, 1024), (777, 192, 1000), (1023, 64, 72), (300, 128, 12)])
+def test_rows_of_fewer_than_the_projection_kernels(dev, m, k, n):
+    x, w = _inputs(m, k, n, dev)
+    pad = [torch.cat((t, torch.zeros(len(t), 32, dtype=t.dtype, device=dev)), 1) for t in (x, w)]  # K % 64 == 32
+    for got, want in zip(ops.linear_rowsq(x, w), ops.linear_rowsq(*pad)):
+        assert torch.equal(got, want)
+    assert torch.equal(ops.linear(x, w), ops.linear(*pad))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_values_that_are_not_finite_stay_in_their_row(dev, bad):
+    for m in (300, 1100, 2331, 4000):
+        x, w = _inputs(m, 128, 1024, dev)
+        want = ops.linear_rowsq(x, w)
+        x[m // 2, 5] = bad
+        got = ops.linear_rowsq(x, w)
+        assert not torch.isfinite(got[0][m // 2].float()).any() and not torch.isfinite(got[1][:, m // 2]).any()
+        keep = torch.arange(m, device=dev) != m // 2
+        assert torch.equal(got[0][keep], want[0][keep]) and torch.equal(got[1][:, keep], want[1][:, keep])
