@@ -854,10 +854,9 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
   }
 }
 
-// fp32 on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products and sums): K % 32 == 0.  512 x 128 x
-// 128 takes 3.3 us and 32768 x 256 x 1024 143 us (120 TFLOP/s); the VALU tile below 18.9 and 393 (few
-// blocks, a scalar LDS read for every two FMAs).  Same error against fp64: 2.03e-7 relative at K = 128,
-// 5.74e-7 at K = 1024, over twelve seeds.
+// fp32 on the matrix cores (v_mfma_f32_16x16x4_f32, whose four products are four fmaf in K order): K %
+// 32 == 0, bit for bit the VALU tile's results below.  512 x 128 x 128 takes 3.1 us and 32768 x 256 x
+// 1024 135 us (127 TFLOP/s); the VALU tile 18.9 and 393 (few blocks, a scalar LDS read for every two FMAs).
 // codes (N % 4 == 0): also the 4-bit route codes, bit i of route r the sign of output 4 r + i.
 template <int BN, int BM>
 __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__ W, const float* __restrict__ X,

@@ -48,3 +48,24 @@ def test_values_that_are_not_finite_stay_in_their_row(dev, bad):
         assert not torch.isfinite(got[0][m // 2].float()).any() and not torch.isfinite(got[1][:, m // 2]).any()
         keep = torch.arange(m, device=dev) != m // 2
         assert torch.equal(got[0][keep], want[0][keep]) and torch.equal(got[1][:, keep], want[1][:, keep])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 32), (5, 33, 64), (64, 32, 128), (512, 256, 1024), (1100, 1024, 96),
+                                   (4100, 260, 160), (300, 33, 32)])
+@pytest.mark.parametrize("kind", ["normal", "wide", "small"])
+def test_fp32_products_are_fma_chains(dev, m, n, k, kind):
+    """K padded by 16 zeros takes the VALU tile, one fmaf after another in K order: the matrix cores'
+    fp32 products give the same bits, denormal sums among them."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=gen), torch.randn(n, k, generator=gen)
+    if kind == "wide":
+        x, w = (t * torch.exp2(torch.randint(-20, 21, t.shape, generator=gen).float()) for t in (x, w))
+    if kind == "small":
+        x, w = x * 1e-30, w * 1e-10
+    x, w = x.to(dev), w.to(dev)
+    px, pw = (torch.cat((t, torch.zeros(len(t), 16, device=dev)), 1) for t in (x, w))
+    got, want = ops.linear(x, w), ops.linear(px, pw)
+    assert torch.equal(got, want) and (got != 0).any()
+    if n % 4 == 0:
+        for a, b in zip(ops.router_codes(x, w, 4), ops.router_codes(px, pw, 4)):
+            assert torch.equal(a, b)
