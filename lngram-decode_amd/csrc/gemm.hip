@@ -1180,7 +1180,12 @@ static int launch_proj(const bf16* w, const bf16* x, int64_t N, int64_t M, int64
   return check_launch("gemm_bf16_proj");
 }
 
-static bool tile_f32_shape(int64_t N, int64_t K) { return K % 32 == 0 && N * K * 4 < (int64_t{1} << 31); }
+// Whole stages of rows read 16 bytes at a time, outputs written 4 at a time where N allows: other K and
+// buffers that are not 16-byte aligned take the VALU tile, which reads single elements.
+static bool tile_f32_shape(const void* x, const void* w, const void* y, int64_t N, int64_t K) {
+  auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  return K % 32 == 0 && N * K * 4 < (int64_t{1} << 31) && al(x) && al(w) && (al(y) || N % 4);
+}
 
 static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N, int64_t K, float* y, hipStream_t s,
                            void* codes = nullptr, int codes_dt = 0) {
@@ -1199,7 +1204,7 @@ static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N,
 template <typename TA, typename TB, typename TO>
 static int launch_f32(const void* x, const void* w, int64_t M, int64_t N, int64_t K, void* y, hipStream_t s) {
   if constexpr (sizeof(TA) == 4 && sizeof(TB) == 4 && sizeof(TO) == 4) {
-    if (tile_f32_shape(N, K))
+    if (tile_f32_shape(x, w, y, N, K))
       return launch_tile_f32(static_cast<const float*>(x), static_cast<const float*>(w), M, N, K, static_cast<float*>(y), s);
   }
   dim3 grid(static_cast<unsigned>(cdiv(N, 64)), static_cast<unsigned>(cdiv(M, 64)));
@@ -1334,7 +1339,7 @@ int lng_router_codes(const void* x, int x_dtype, const void* w, int w_dtype, int
       return rc;
   } else {
     if (!logits) return fail(LNG_E_ARG, "router_codes: fp32 router needs a logits buffer");
-    if (x_dtype == LNG_F32 && w_dtype == LNG_F32 && codes && bits == 4 && tile_f32_shape(N, K))
+    if (x_dtype == LNG_F32 && w_dtype == LNG_F32 && codes && bits == 4 && tile_f32_shape(x, w, logits, N, K))
       return launch_tile_f32(static_cast<const float*>(x), static_cast<const float*>(w), M, N, K, logits, s, codes,
                              codes_dtype);
     int rc;

@@ -69,3 +69,25 @@ def test_fp32_products_are_fma_chains(dev, m, n, k, kind):
     if n % 4 == 0:
         for a, b in zip(ops.router_codes(x, w, 4), ops.router_codes(px, pw, 4)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which", ["x", "w", "y"])
+@pytest.mark.parametrize("m,n,k", [(70, 64, 128), (300, 36, 32)])
+def test_fp32_buffers_of_any_alignment(dev, which, m, n, k):
+    """fp32 buffers need 4-byte alignment only: views one element into their storage, and through the C
+    ABI an output one element in."""
+    gen = torch.Generator().manual_seed(m)
+
+    def at(shape, off):
+        return torch.empty(shape[0] * shape[1] + 4, device=dev)[off:off + shape[0] * shape[1]].view(shape)
+
+    x, w = torch.randn(m, k, generator=gen).to(dev), torch.randn(n, k, generator=gen).to(dev)
+    want, codes = ops.linear(x, w), ops.router_codes(x, w, 4)[1]
+    x2, w2, y = at((m, k), which == "x").copy_(x), at((n, k), which == "w").copy_(w), at((m, n), which == "y")
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    assert ops.lib().lng_linear(x2.data_ptr(), w2.data_ptr(), ops.dtype_code(torch.float32), m, n, k, y.data_ptr(), stream) == 0
+    assert torch.equal(y, want)
+    if which != "y":
+        assert torch.equal(ops.linear(x2, w2), want)
+        for a, b in zip(ops.router_codes(x2, w2, 4), (want, codes)):
+            assert torch.equal(a, b)
