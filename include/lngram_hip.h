@@ -238,11 +238,11 @@ int32_t lng_linear_rowsq_partials(int64_t N);
 int lng_linear_rowsq(const void* x, const void* w, int64_t M, int64_t N, int64_t K, void* y, float* rowsq,
                      void* stream);
 
-/* fp32 y[M,N] = (x[M,K] . (w[N,K] diag(norm_w))^T) * rsqrt(mean_k(x[m,k]^2) + eps) for bf16 x and fp32
- * w, norm_w: the SSM's input projection u = W_in RMSNorm(x.float()) (DiagonalSSM.inputs, ssm.py:41-43)
- * from the bf16 embeddings.  Each fp32 weight is split into three bf16 pieces in the workspace
- * (lng_linear_split_workspace_bytes; 0 unless N % 4 == 0 and K % 64 == 0), whose products with x are
- * exact; sums are fp32, in one order for every M.  x, y and workspace 16-byte aligned. */
+/* fp32 y[M,N] = RMSNorm(x[M,K]) . w[N,K]^T for bf16 x and fp32 w, norm_w: the SSM's input projection
+ * u = W_in RMSNorm(x.float()) (DiagonalSSM.inputs, ssm.py:41-43) from the bf16 embeddings, bit for bit
+ * lng_rmsnorm of the rows in fp32 and lng_linear of its result.  x, w and y 16-byte aligned.  Shapes:
+ * lng_linear_split_workspace_bytes(N, K) != 0 (N % 4 == 0, K % 64 == 0, K <= 4096).  The workspace is not
+ * used any more and may be NULL. */
 size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K);
 int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t M, int64_t N, int64_t K, float eps,
                      void* workspace, size_t workspace_bytes, float* y, void* stream);

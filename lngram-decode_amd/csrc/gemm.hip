@@ -776,7 +776,7 @@ __global__ __launch_bounds__(256) void k_gemm_tile(const bf16* __restrict__ W, c
                                                    int64_t M, int64_t K, int n_tiles, void* __restrict__ out,
                                                    float* __restrict__ logits, void* __restrict__ codes, int codes_dt,
                                                    int64_t routes, float* __restrict__ rowsq, int chains, float x_eps) {
-  using G = TileGemm<bf16, BN, BM, WN, WM, 1, 3>;
+  using G = TileGemm<bf16, BN, BM, WN, WM, 3>;
   __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
   const int nt = static_cast<int>(blockIdx.x) % n_tiles;
   const int64_t n0 = static_cast<int64_t>(nt) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
@@ -862,7 +862,7 @@ template <int BN, int BM>
 __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__ W, const float* __restrict__ X,
                                                        int64_t N, int64_t M, int64_t K, int n_tiles,
                                                        float* __restrict__ Y, void* __restrict__ codes, int codes_dt) {
-  using G = TileGemm<float, BN, BM, 2, 2, 1, 3>;
+  using G = TileGemm<float, BN, BM, 2, 2, 3>;
   __shared__ __attribute__((aligned(16))) float ring[G::LDS_ELEMS];
   const int64_t n0 = static_cast<int64_t>(blockIdx.x % n_tiles) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
   G g;
@@ -895,49 +895,159 @@ __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__
   }
 }
 
-// y = (x . w^T) * rsqrt(mean(x^2) + eps) in fp32 for bf16 x and an fp32 weight split into three bf16
-// pieces (8 + 8 + 8 bits: every product is exact, the sums are fp32); w3 = [3][N][K].
-template <int BN, int BM, int WN, int WM, int SLOTS>
-__global__ __launch_bounds__(64 * WN * WM) void k_gemm_split3(const bf16* __restrict__ w3, const bf16* __restrict__ X,
-                                                              int64_t N, int64_t M, int64_t K, int n_tiles, float eps,
-                                                              float* __restrict__ Y) {
-  using G = TileGemm<bf16, BN, BM, WN, WM, 3, SLOTS>;
-  __shared__ __attribute__((aligned(16))) bf16 ring[G::LDS_ELEMS];
+// y = RMSNorm(x) . w^T in fp32 for bf16 x: bit for bit k_rmsnorm<float> of the rows in fp32 and the fp32
+// product of what it writes, in one pass over the bf16 rows (K % 64 == 0).  A block first forms its rows'
+// scales; in the K loop a lane turns the bf16 elements of its x operand into the normalised fp32 ones
+// (x * r * norm_w, each product rounded) and multiplies as TileGemm<float> does: K 32 a stage, w rows of
+// 128 B and x rows of 64 B straight into LDS.  32768 x 256 x 1024: 158 us (109 TFLOP/s; the fp32 product
+// alone 135).  Bound by the fp32 matrix rate and what a wave's operands wait for beside it; x pieces
+// turned into fp32 once a block, through registers into the ring, took 169 to 198 us.  The weight as
+// three bf16 pieces (exact products, the row scale on the sums) takes 60, but its sums round otherwise.
+constexpr int NG_MAXK = 4096;
+template <int BN, int BM, int WN, int WM>
+__device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, const float* norm_w, int64_t N, int64_t M,
+                                              int64_t K, int n_tiles, float eps, float* Y) {
+  using G = TileGemm<float, BN, BM, WN, WM, 3>;
+  constexpr int NWAVE = WN * WM, FN = G::FN, FM = G::FM, SLOTS = 3, K_ST = 32;
+  constexpr int W_LOADS = BN / 8 / NWAVE;                               // 8 w rows an instruction
+  constexpr int X_LOADS = (BM / 16 + NWAVE - 1) / NWAVE;                // 16 x rows: the first BM / 16 waves of each
+  constexpr int SLOT = BN * 128 + X_LOADS * NWAVE * 16 * 64;            // bytes
+  static_assert(BN % (8 * NWAVE) == 0 && BM % (8 * NWAVE) == 0 && W_LOADS + X_LOADS <= 60, "tile split");
+  // one LDS object: with several the compiler tells them apart by alias scopes, and then waits for every
+  // load in flight to LDS before it reads the ring
+  __shared__ __attribute__((aligned(16))) char ring[SLOTS * SLOT + BM * 4 + NG_MAXK * 4];
+  float* scale = reinterpret_cast<float*>(ring + SLOTS * SLOT);
+  float* nw = scale + BM;  // norm_w[K]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int wn = wave % WN, wm = wave / WN, rsel = lane & 15, psel = lane >> 4;
   const int64_t n0 = static_cast<int64_t>(blockIdx.x % n_tiles) * BN, m0 = static_cast<int64_t>(blockIdx.x / n_tiles) * BM;
-  G g;
-  g.template run<true>(ring, w3, X, N, M, K, n0, m0);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wn = wave % WN, wm = wave / WN;
+  const int nk = static_cast<int>(K / K_ST);
+  auto clip = [](int64_t b) { return static_cast<int>(b < 0x7fffffffll ? b : 0x7fffffffll); };
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(W + n0 * K), 0,
+                                                                       clip((N - n0) * K * 4), BUF_DW3);
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(X + m0 * K), 0,
+                                                                       clip((M - m0) * K * 2), BUF_DW3);
+  // x rows: 4 pieces of 16 bytes, piece p of row r in slot p ^ ((r >> 2) & 3)
+  uint32_t w_off[W_LOADS], x_off[X_LOADS];
 #pragma unroll
-  for (int j = 0; j < G::FM; ++j) {
-    const int64_t m = m0 + wm * (BM / WM) + j * 16 + (lane & 15);
-    const float r = 1.0f / sqrtf(g.xss[j] / static_cast<float>(K) + eps);
+  for (int d = 0; d < W_LOADS; ++d) {
+    const int r = (d * NWAVE + wave) * 8 + (lane >> 3);
+    w_off[d] = static_cast<uint32_t>((r * K + 4 * ((lane & 7) ^ G::swz(r))) * 4);
+  }
+#pragma unroll
+  for (int d = 0; d < X_LOADS; ++d) {
+    const int r = (d * NWAVE + wave) * 16 + (lane >> 2);  // past BM: rows that nobody reads
+    x_off[d] = static_cast<uint32_t>((r * K + 8 * ((lane & 3) ^ ((r >> 2) & 3))) * 2);
+  }
+  auto issue = [&](int kt, int slot) {
+    char* dst = ring + slot * SLOT;
+#pragma unroll
+    for (int d = 0; d < W_LOADS; ++d)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          wrs, (__attribute__((address_space(3))) void*)(dst + (d * NWAVE + wave) * 1024), 16,
+          w_off[d] + static_cast<uint32_t>(kt) * 128, 0, 0, 0);
+#pragma unroll
+    for (int d = 0; d < X_LOADS; ++d)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          xrs, (__attribute__((address_space(3))) void*)(dst + BN * 128 + (d * NWAVE + wave) * 1024), 16,
+          x_off[d] + static_cast<uint32_t>(kt) * 64, 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < SLOTS - 1; ++s) issue(s, s);  // nk >= 2
+  for (int i = threadIdx.x; i < K; i += 64 * NWAVE) nw[i] = norm_w[i];
+  // row scales in k_rmsnorm's order: 64 chains (elements 64 apart) and their sums pairwise.  A lane has 8
+  // chains of a row, 8 lanes a row, so that its loads are whole pieces.
+#pragma unroll
+  for (int g = 0; g < BM / 8 / NWAVE; ++g) {
+    const int r = (g * NWAVE + wave) * 8 + (lane >> 3);
+    float ss[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss[j] = 0.f;
+    if (m0 + r < M) {
+      const bf16* row = X + (m0 + r) * K + 8 * (lane & 7);
+#pragma unroll 8
+      for (int64_t c = 0; c < K; c += 64) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float f = static_cast<float>(v[j]);
+          ss[j] = fmaf(f, f, ss[j]);
+        }
+      }
+    }
+    float s = ((ss[0] + ss[1]) + (ss[2] + ss[3])) + ((ss[4] + ss[5]) + (ss[6] + ss[7]));
+#pragma unroll
+    for (int d = 1; d < 8; d *= 2) s += __shfl_xor(s, d, 64);
+    if ((lane & 7) == 0) scale[r] = 1.0f / sqrtf(s / static_cast<float>(K) + eps);
+  }
+  __syncthreads();
+  float rs[FM];
+#pragma unroll
+  for (int j = 0; j < FM; ++j) rs[j] = scale[wm * (BM / WM) + j * 16 + rsel];
+  f32x4 acc[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto stage = [&](int kt, int slot) {
+    if (nk - 1 - kt > 0)  // one later stage in flight
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(W_LOADS + X_LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // stage kt has landed for every wave, and every wave has read the slot of stage kt - 1
+    __builtin_amdgcn_s_barrier();
+    if (kt + SLOTS - 1 < nk) issue(kt + SLOTS - 1, (slot + SLOTS - 1) % SLOTS);
+    const float* ws = reinterpret_cast<const float*>(ring + slot * SLOT);
+    const bf16* xs = reinterpret_cast<const bf16*>(ring + slot * SLOT + BN * 128);
+    const float* np = nw + kt * K_ST + psel;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // products take k 16 h + 4 e + psel (TileGemm<float>::operand)
+      f32x4 a[FN], b[FM];
+#pragma unroll
+      for (int i = 0; i < FN; ++i) a[i] = G::operand(ws, wn * (BN / WN) + i * 16 + rsel, h, psel, G::swz(rsel));
+#pragma unroll
+      for (int j = 0; j < FM; ++j) {
+        const bf16* row = xs + (wm * (BM / WM) + j * 16 + rsel) * K_ST;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = 4 * e + psel;  // of the half's 16: piece 2 h + k / 8
+          const float x = static_cast<float>(row[8 * ((2 * h + (e >> 1)) ^ ((rsel >> 2) & 3)) + (k & 7)]);
+          b[j][e] = (x * rs[j]) * np[16 * h + 4 * e];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = G::mma(a[i], b[j], acc[i][j]);
+    }
+  };
+  // the slots in turn, as in TileGemm
+  int kt = 0;
+  for (; kt + SLOTS <= nk; kt += SLOTS) {
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) stage(kt + s, s);
+  }
+#pragma unroll
+  for (int s = 0; s < SLOTS - 1; ++s)
+    if (kt + s < nk) stage(kt + s, s);
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int64_t m = m0 + wm * (BM / WM) + j * 16 + rsel;
     if (m >= M) continue;
 #pragma unroll
-    for (int i = 0; i < G::FN; ++i) {
-      const int64_t n = n0 + wn * (BN / WN) + i * 16 + 4 * (lane >> 4);
-      if (n >= N) continue;  // N % 4 == 0
-      f32x4 v = g.acc[i][j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] *= r;
-      *reinterpret_cast<f32x4*>(Y + m * N + n) = v;
+    for (int i = 0; i < FN; ++i) {
+      const int64_t n = n0 + wn * (BN / WN) + i * 16 + 4 * psel;
+      if (n < N) *reinterpret_cast<f32x4*>(Y + m * N + n) = acc[i][j];  // N % 4 == 0
     }
   }
 }
 
-// w3[p][n][k]: bf16 pieces of fp32(w[n, k] * s[k]), largest first; a piece past a non-finite one is 0
-__global__ __launch_bounds__(256) void k_split3(const float* __restrict__ w, const float* __restrict__ s, int64_t n,
-                                                int64_t K, bf16* __restrict__ w3) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= n) return;
-  float f = w[i] * s[i % K];
-#pragma unroll
-  for (int p = 0; p < 3; ++p) {
-    const bf16 b = static_cast<bf16>(f);
-    w3[p * n + i] = b;
-    f -= static_cast<float>(b);
-    if (!(fabsf(f) <= 3.0e38f)) f = 0.f;
-  }
+template <int BN, int BM, int WN, int WM>
+__global__ __launch_bounds__(64 * WN * WM) void k_norm_gemm_f32(const float* __restrict__ W, const bf16* __restrict__ X,
+                                                                const float* __restrict__ norm_w, int64_t N, int64_t M,
+                                                                int64_t K, int n_tiles, float eps, float* __restrict__ Y) {
+  norm_gemm_f32<BN, BM, WN, WM>(W, X, norm_w, N, M, K, n_tiles, eps, Y);
 }
 
 // fp32 VALU tile GEMM: 64x64 tile per 256-thread block, 4x4 outputs per thread,
@@ -1274,38 +1384,38 @@ int lng_linear_rowscale(const void* x, const void* w, int64_t M, int64_t N, int6
                      as_stream(stream), true, eps);
 }
 
-static bool split3_shape(int64_t N, int64_t K) {
-  return N > 0 && K > 0 && N % 4 == 0 && K % 64 == 0 && 3 * N * K * 2 < (int64_t{1} << 31);
+// whole stages, whole 16-byte outputs, the norm's weights in LDS
+static bool split_shape(int64_t N, int64_t K) {
+  return N > 0 && K > 0 && N % 4 == 0 && K % 64 == 0 && K <= NG_MAXK && N * K * 4 < (int64_t{1} << 31);
 }
-size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K) {
-  return split3_shape(N, K) ? static_cast<size_t>(3 * N * K * 2) : 0;
-}
+size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K) { return split_shape(N, K) ? 16 : 0; }
 
 int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t M, int64_t N, int64_t K, float eps,
-                     void* workspace, size_t workspace_bytes, float* y, void* stream) {
-  if (M < 0 || !split3_shape(N, K))
-    return fail(LNG_E_ARG, "linear_split: needs N % 4 == 0 and K % 64 == 0 (lng_linear_split_workspace_bytes)");
+                     void*, size_t, float* y, void* stream) {
+  if (M < 0 || !split_shape(N, K))
+    return fail(LNG_E_ARG, "linear_split: needs N % 4 == 0, K % 64 == 0 and K <= 4096 (lng_linear_split_workspace_bytes)");
   if (M == 0) return LNG_OK;
-  if (!x || !norm_w || !w || !workspace || !y) return fail(LNG_E_ARG, "linear_split: null buffer");
-  if (workspace_bytes < lng_linear_split_workspace_bytes(N, K)) return fail(LNG_E_ARG, "linear_split: workspace too small");
+  if (!x || !norm_w || !w || !y) return fail(LNG_E_ARG, "linear_split: null buffer");
   auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!al(x) || !al(workspace) || !al(y)) return fail(LNG_E_ARG, "linear_split: buffers must be 16-byte aligned");
+  if (!al(x) || !al(w) || !al(y)) return fail(LNG_E_ARG, "linear_split: x, w and y must be 16-byte aligned");
   hipStream_t s = as_stream(stream);
-  bf16* w3 = static_cast<bf16*>(workspace);
   const bf16* xp = static_cast<const bf16*>(x);
-  hipLaunchKernelGGL(k_split3, dim3(static_cast<unsigned>(cdiv(N * K, 256))), dim3(256), 0, s, w, norm_w, N * K, K, w3);
-  auto go = [&](auto* kern, int64_t bn, int64_t bm, int threads) {
+  auto go = [&](auto* kern, int64_t bn, int64_t bm) {
     const int n_tiles = static_cast<int>(cdiv(N, bn));
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(threads), 0, s, w3, xp, N, M, K,
-                       n_tiles, eps, y);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, xp, norm_w, N, M,
+                       K, n_tiles, eps, y);
     return check_launch("linear_split");
   };
-  // by blocks, as pick_tile (N 256, K 1024, the split included; us):  M  200  2048  4096  8192  32768
-  //   32 x 32 9.1 12.4 19.1 30.6 112;  64 x 64 15.2 15.7 17.0 20.9 68.5;  64 x 128 18.6 18.4 19.8 20.9 61.0
-  // norm pass, fp32 copy and VALU product before: 165 190 193 216 474
-  if (cdiv(N, 32) * cdiv(M, 32) <= 768) return go(&k_gemm_split3<32, 32, 2, 2, 3>, 32, 32, 256);
-  if (cdiv(N, 64) * cdiv(M, 64) <= 512) return go(&k_gemm_split3<64, 64, 2, 2, 2>, 64, 64, 256);
-  return go(&k_gemm_split3<64, 128, 2, 4, 2>, 64, 128, 512);
+  // by blocks (N 256, K 1024; us):   M  200  1000  2331  8192  32768
+  //   32 x 32                         15.4  16.2  28.5  67.7    238
+  //   64 x 64                         30.0  30.2  30.7  52.8    169
+  //   128 x 64                        44.8  45.2  45.7  49.6    158
+  // fp32 copy, norm pass and VALU product: 164 170 181 212 473
+  const int64_t b32 = cdiv(N, 32) * cdiv(M, 32);
+  if (b32 <= 640) return go(&k_norm_gemm_f32<32, 32, 2, 2>, 32, 32);
+  if (b32 <= 1024) return go(&k_norm_gemm_f32<64, 64, 2, 2>, 64, 64);
+  if (N <= 64) return go(&k_norm_gemm_f32<64, 64, 2, 2>, 64, 64);  // (N 64, K 256, 32768 rows: 16.8; 128 x 64 24.1)
+  return go(&k_norm_gemm_f32<128, 64, 2, 2>, 128, 64);
 }
 
 int lng_linear(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, void* y, void* stream) {

@@ -1,30 +1,28 @@
-// GEMM tiles: bf16 projections between the skinny kernel's rows and the one-tile-per-CU kernels', bf16
-// rows against fp32 weights split into bf16 pieces, and fp32.
+// GEMM tiles: bf16 projections between the skinny kernel's rows and the one-tile-per-CU kernels', and fp32.
 //
 // y[m, n] = sum_k x[m, k] * w[n, k]: a block of WN x WM waves computes BN (w rows) x BM (x rows), wave
 // (wn, wm) its BN/WN x BM/WM part in 16x16 fragments, accumulating in K order whatever the tile, so the
 // results equal the other kernels' (bf16: 16x16x32 products; fp32: 16x16x4 products, bit for bit four
 // fmaf in K order).  K advances 128 bytes a stage through a ring of SLOTS LDS stages filled by buffer
 // loads straight into LDS; rows past N or M lie outside the buffers and read as zero.
-// NP > 1: w is NP consecutive [N, K] matrices whose products with the same x rows add up.
 #pragma once
 
 #include "common.h"
 
 namespace lng {
 
-template <typename T, int BN, int BM, int WN, int WM, int NP, int SLOTS>
+template <typename T, int BN, int BM, int WN, int WM, int SLOTS>
 struct TileGemm {
   static constexpr int NWAVE = WN * WM, NT = 64 * NWAVE;
   static constexpr int K_ST = 128 / sizeof(T);          // k of a stage: 64 bf16 or 32 fp32
   static constexpr int PE = 16 / sizeof(T);             // elements of a piece
   typedef T Frag __attribute__((ext_vector_type(PE)));  // an operand lane's share of 4 pieces' k
-  static constexpr int ROWS = NP * BN + BM;             // LDS rows of a stage, the w pieces first
+  static constexpr int ROWS = BN + BM;                  // LDS rows of a stage, w's first
   static constexpr int FN = BN / WN / 16, FM = BM / WM / 16;
   static constexpr int LOADS = ROWS / 8 / NWAVE;        // 8 rows an instruction
-  static constexpr int W_LOADS = NP * BN / 8 / NWAVE;
+  static constexpr int W_LOADS = BN / 8 / NWAVE;
   static constexpr int LDS_ELEMS = SLOTS * ROWS * K_ST;
-  static_assert(ROWS % (8 * NWAVE) == 0 && NP * BN % (8 * NWAVE) == 0 && BN % (16 * WN) == 0 && BM % (16 * WM) == 0, "tile split");
+  static_assert(ROWS % (8 * NWAVE) == 0 && BN % (8 * NWAVE) == 0 && BN % (16 * WN) == 0 && BM % (16 * WM) == 0, "tile split");
   static_assert((SLOTS - 2) * LOADS <= 60, "vmcnt");
 
   f32x4 acc[FN][FM];
@@ -75,10 +73,8 @@ struct TileGemm {
     const int wn = wave % WN, wm = wave / WN;
     const int nk = static_cast<int>(K / K_ST);
     auto clip = [](int64_t b) { return static_cast<int>(b < 0x7fffffffll ? b : 0x7fffffffll); };
-    // one buffer over the pieces: a w row past N is another piece's row or zero, and only feeds columns
-    // past N
     const __amdgpu_buffer_rsrc_t wrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(W + n0 * K), 0, clip((NP * N - n0) * K * ES), BUF_DW3);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(W + n0 * K), 0, clip((N - n0) * K * ES), BUF_DW3);
     const __amdgpu_buffer_rsrc_t xrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(X + m0 * K), 0, clip((M - m0) * K * ES), BUF_DW3);
     // load d of this wave covers stage rows (d NWAVE + wave) 8 ..: the first W_LOADS are w's
@@ -86,7 +82,7 @@ struct TileGemm {
 #pragma unroll
     for (int d = 0; d < LOADS; ++d) {
       const int r = (d * NWAVE + wave) * 8 + (lane >> 3);
-      const int64_t rr = r < NP * BN ? r / BN * N + r % BN : r - NP * BN;
+      const int64_t rr = r < BN ? r : r - BN;
       voff[d] = static_cast<uint32_t>((rr * K + PE * ((lane & 7) ^ swz(r))) * ES);
     }
     auto issue = [&](int kt, int to_slot) {
@@ -121,18 +117,14 @@ struct TileGemm {
         Frag b[FM];
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-          b[j] = operand(st, NP * BN + wm * (BM / WM) + j * 16 + rsel, h, psel, swz(rsel));
+          b[j] = operand(st, BN + wm * (BM / WM) + j * 16 + rsel, h, psel, swz(rsel));
+        Frag a[FN];
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-          Frag a[FN];
+        for (int i = 0; i < FN; ++i) a[i] = operand(st, wn * (BN / WN) + i * 16 + rsel, h, psel, swz(rsel));
 #pragma unroll
-          for (int i = 0; i < FN; ++i)
-            a[i] = operand(st, p * BN + wn * (BN / WN) + i * 16 + rsel, h, psel, swz(rsel));
+        for (int i = 0; i < FN; ++i)
 #pragma unroll
-          for (int i = 0; i < FN; ++i)
-#pragma unroll
-            for (int j = 0; j < FM; ++j) acc[i][j] = mma(a[i], b[j], acc[i][j]);
-        }
+          for (int j = 0; j < FM; ++j) acc[i][j] = mma(a[i], b[j], acc[i][j]);
         if constexpr (XRMS) {
           // a row's sum in two chains, its even and its odd pieces in order, as the lanes of
           // k_gemm_proj_bf16's 32x32x16 fragments form it: lane groups 0, 1 and 2, 3 exchange pieces and

@@ -476,21 +476,18 @@ def linear_rowscale(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tenso
 
 
 def norm_linear_fp32(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
-    """fp32 ``W RMSNorm(x.float())`` (``model.RMSNorm`` with weight ``norm_w``) for fp32 ``w [N, K]``: bf16
-    rows in one pass (``lng_linear_split``: exact products, the row scale applied to the sums), else
-    the norm and the product."""
+    """fp32 ``W RMSNorm(x.float())`` (``model.RMSNorm`` with weight ``norm_w``) for fp32 ``w [N, K]``: the
+    norm and the product, for bf16 rows in one pass with the same bits (``lng_linear_split``)."""
     dev = _dev(x, norm_w, w)
     k = x.shape[-1]
     n = w.shape[0]
     if w.shape[1] != k or tuple(norm_w.shape) != (k,):
         raise ValueError(f"weight {tuple(w.shape)} and norm {tuple(norm_w.shape)} do not match input dim {k}")
-    nws = lib().lng_linear_split_workspace_bytes(n, k) if x.dtype == torch.bfloat16 else 0
-    if not nws:
+    if x.dtype != torch.bfloat16 or not lib().lng_linear_split_workspace_bytes(n, k):
         return linear(rmsnorm(x.float(), norm_w.float(), eps), w.float())
     x2, nw, wc = _c(x.reshape(-1, k)), _c(norm_w.float()), _c(w.float())
-    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
     out = torch.empty(*x.shape[:-1], n, dtype=torch.float32, device=dev)
-    check(lib().lng_linear_split(_ptr(x2), _ptr(nw), _ptr(wc), x2.shape[0], n, k, float(eps), _ptr(ws), nws, _ptr(out),
+    check(lib().lng_linear_split(_ptr(x2), _ptr(nw), _ptr(wc), x2.shape[0], n, k, float(eps), None, 0, _ptr(out),
                                  _stream(dev)), "linear_split")
     return out
 

@@ -91,3 +91,19 @@ def test_fp32_buffers_of_any_alignment(dev, which, m, n, k):
         assert torch.equal(ops.linear(x2, w2), want)
         for a, b in zip(ops.router_codes(x2, w2, 4), (want, codes)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (33, 4, 64), (200, 36, 128), (2560, 256, 192), (2561, 256, 64),
+                                   (4097, 260, 128), (8192, 256, 1024), (20000, 64, 256), (3, 8, 4096)])
+def test_norm_and_product_in_one_pass(dev, m, n, k):
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = (torch.randn(m, k, generator=gen) * torch.exp2(torch.randint(-30, 30, (m, 1), generator=gen).float()))
+    x = x.to(torch.bfloat16).to(dev)
+    if m > 4:
+        x[1], x[2, 3], x[3, k - 1] = 0.0, float("inf"), float("nan")
+    w, nw = (torch.randn(n, k, generator=gen) * 0.02).to(dev), (torch.rand(k, generator=gen) + 0.5).to(dev)
+    assert ops.lib().lng_linear_split_workspace_bytes(n, k) > 0
+    got = ops.norm_linear_fp32(x, nw, w, 1e-5)
+    want = ops.linear(ops.rmsnorm(x.float(), nw, 1e-5), w)
+    assert torch.equal(torch.nan_to_num(got, 7.0), torch.nan_to_num(want, 7.0))
+    assert torch.equal(got.isnan(), want.isnan()) and (m <= 4 or bool(got[2:4].isnan().all()))
