@@ -187,8 +187,7 @@ def memory_step(model, pos: int, state: DecodeState, h: Tensor, codes_new: Tenso
     conv_in = state.conv_in[pos]
     if (route_tokens is None and route_codes_ctx is None and 0 < h.shape[0] * n <= 64 and m._fused_shape_ok(h)
             and tuple(h.shape) == (state.batch, n, m.hidden_size) and tuple(codes_new.shape) == (state.batch, n, m.num_routes)
-            and cache.is_contiguous() and conv_in.is_contiguous() and conv_in.dtype == torch.bfloat16
-            and tuple(cache.shape[:2]) == tuple(conv_in.shape[:2]) == (state.batch, state.max_len)
+            and ops.memory_step_caches_ok(cache, conv_in, state.batch, state.max_len, m.num_routes, m.hidden_size)
             and cache.device == conv_in.device == h.device == codes_new.device):
         layer = m._native_layer(h.dtype, h.device, True)
         if layer is not None:

@@ -405,12 +405,25 @@ def memory_forward(layer, h: torch.Tensor, codes: torch.Tensor, max_workspace: i
     return out
 
 
+def memory_step_caches_ok(code_cache: torch.Tensor, conv_cache: torch.Tensor, batch: int, max_len: int, routes: int,
+                          hidden: int) -> bool:
+    """Whether the caches are those that :func:`memory_step` writes: uint8 codes ``[batch, max_len, routes]`` and
+    bf16 conv inputs ``[batch, max_len, hidden]``, contiguous."""
+    return (code_cache.dtype == torch.uint8 and conv_cache.dtype == torch.bfloat16
+            and tuple(code_cache.shape) == (batch, max_len, routes) and tuple(conv_cache.shape) == (batch, max_len, hidden)
+            and code_cache.is_contiguous() and conv_cache.is_contiguous())
+
+
 def memory_step(layer, h: torch.Tensor, codes: torch.Tensor, pos0: int, code_cache: torch.Tensor,
                 conv_cache: torch.Tensor) -> torch.Tensor:
     """The cached step's output ``[B, n, hidden]`` (``lng_memory_step``): ``codes [B, n, R]`` into
     ``code_cache`` and the projected rows into ``conv_cache`` at ``pos0`` on."""
     dev = _dev(h, codes, code_cache, conv_cache)
     b, n, d = h.shape
+    if d != layer.hidden or tuple(codes.shape) != (b, n, layer.routes) or \
+            not memory_step_caches_ok(code_cache, conv_cache, b, code_cache.shape[1], layer.routes, d):
+        raise ValueError("memory_step: h [B, n, hidden], codes [B, n, R], a uint8 [B, S, R] code cache and a bf16 "
+                         "[B, S, hidden] conv cache")
     hc, cc = _c(h), _codes_ok(codes)
     nws = 2 * (-(-b * n * d * h.element_size() // 256) * 256)
     ws = torch.empty(nws, dtype=torch.uint8, device=dev)
