@@ -433,7 +433,7 @@ int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t grad_stride,
 
 /* ---------------------------------------------------------------- the layer's launches in one call */
 /* One memory layer (RouteNgramMemoryV2, lngram_v2.py:842-1010) in one dtype (bf16 or f32): shapes and
- * device pointers of its weights, contiguous and 16-byte aligned.  fused: the shape of
+ * device pointers of its weights, contiguous and 16-byte aligned; hidden = q_heads * head_dim.  fused: the shape of
  * lng_memory_readout_fused, w_q then being readout_q_proj.weight with the query norm folded in
  * (lng_fold_columns) and kv the packed key/value weight (lng_memory_readout_pack). */
 typedef struct lng_memory_layer {
@@ -454,8 +454,9 @@ int lng_memory_forward(const lng_memory_layer* layer, const void* h, const void*
 
 /* memory_step (ffnmem/infer.py:152-182) of a fused layer for B * n <= 64 new positions at pos0: their
  * codes [B, n, R] into code_cache [B, max_len, R], the readout over the cache, the output projection
- * into conv_cache [B, max_len, hidden] and the conv over its window.  The workspace holds two
- * [B * n, hidden] buffers (each rounded up to 256 bytes). */
+ * into conv_cache [B, max_len, hidden] and the conv over its window.  The caches have these shapes: they
+ * are strided by the layer's routes and hidden.  The workspace holds two [B * n, hidden] buffers (each
+ * rounded up to 256 bytes). */
 int lng_memory_step(const lng_memory_layer* layer, const void* h, const void* codes, int codes_dtype, int64_t B,
                     int64_t n, int64_t pos0, uint8_t* code_cache, void* conv_cache, int64_t max_len, void* workspace,
                     size_t workspace_bytes, void* out, void* stream);

@@ -184,14 +184,11 @@ def memory_step(model, pos: int, state: DecodeState, h: Tensor, codes_new: Tenso
     if L + n > state.max_len:
         raise ValueError(f"cache full: {L} + {n} > {state.max_len}")
     cache = state.codes[pos]
-    conv_in = state.conv_in[pos]
-    if (route_tokens is None and route_codes_ctx is None and 0 < h.shape[0] * n <= 64 and m._fused_shape_ok(h)
-            and tuple(h.shape) == (state.batch, n, m.hidden_size) and tuple(codes_new.shape) == (state.batch, n, m.num_routes)
-            and ops.memory_step_caches_ok(cache, conv_in, state.batch, state.max_len, m.num_routes, m.hidden_size)
-            and cache.device == conv_in.device == h.device == codes_new.device):
+    if route_tokens is None and route_codes_ctx is None and 0 < h.shape[0] * n <= 64 and m._fused_shape_ok(h):
         layer = m._native_layer(h.dtype, h.device, True)
-        if layer is not None:
-            return ops.memory_step(layer, h, codes_new, L, cache, conv_in)
+        out = None if layer is None else ops.memory_step(layer, h, codes_new, L, cache, state.conv_in[pos])
+        if out is not None:
+            return out
     cache[:, L:L + n] = codes_new.to(cache.dtype)
     if route_tokens is not None and m._fused_shape_ok(h, tables=False):
         # rows from the caller (host-RAM serving, staged verify blocks): the same fused readout

@@ -8,6 +8,7 @@ are rejected: there is no CPU path in the product.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import threading
 
@@ -364,27 +365,41 @@ def route_tokens(codes: torch.Tensor, tables, orders, bits: int, route_start: in
 
 
 # ----------------------------------------------------------------------------- the layer in one call
+@functools.lru_cache(maxsize=64)
+def _layer_shape(dtype: torch.dtype, hidden: int, routes: int, bits: int, orders: tuple, mem_dim: int, q_heads: int,
+                 kv_heads: int, head_dim: int, conv_k: int, conv_dilation: int, fused: int, **floats) -> tuple:
+    """``lng_memory_layer`` without its pointers, and what its tables and weights have to be: (last dimension,
+    elements) of each; a size of 0 where ``hidden`` is not the heads' width, which no weight meets."""
+    L = _lib.MemoryLayer(hidden=hidden, routes=routes, bits=bits, n_orders=len(orders), mem_dim=mem_dim, q_heads=q_heads,
+                         kv_heads=kv_heads, head_dim=head_dim, conv_k=conv_k, conv_dilation=conv_dilation, fused=fused,
+                         dtype=dtype_code(dtype), **floats)
+    for i, o in enumerate(orders):
+        L.orders[i] = o
+    inner, dt = q_heads * head_dim, len(orders) * mem_dim
+    d = hidden if hidden == inner else 0
+    kv = (_lib.READOUT_PACK_ELEMS,) * 2 if fused else (dt, 2 * kv_heads * head_dim * dt)
+    weights = {"w_q": (d, d * inner), "q_norm": (d, d), "kv": kv, "mem_norm": (dt, dt), "w_o": (inner, d * inner),
+               "conv_norm": (d, d), "conv_w": (conv_k, d * conv_k)}
+    return L, [(mem_dim, (routes << (bits * o)) * mem_dim) for o in orders], weights
+
+
 def memory_layer(dtype: torch.dtype, device: torch.device, shape: dict, floats: dict, tables, weights: dict):
-    """``lng_memory_layer`` of a layer whose weights are all ``dtype`` on ``device``, contiguous and 16-byte
-    aligned; None when one is not.  The tensors have to outlive the calls that take it."""
-    L = _lib.MemoryLayer()
-    for t in (*tables, *weights.values()):
-        if t.dtype != dtype or t.device != device or not t.is_contiguous() or t.data_ptr() % 16:
-            return None
-    for k, v in weights.items():
-        setattr(L, k, v.data_ptr())
+    """``lng_memory_layer`` of a layer whose weights are all ``dtype`` on ``device``, contiguous, 16-byte
+    aligned and of the sizes that ``shape`` gives them; None when one is not.  The tensors have to outlive
+    the calls that take it."""
+    proto, table_sizes, weight_sizes = _layer_shape(dtype, **shape, **floats)
+    L = _lib.MemoryLayer.from_buffer_copy(proto)
     for i, t in enumerate(tables):
+        if (t.size(-1), t.numel()) != table_sizes[i] or t.dtype != dtype or t.device != device \
+                or not t.is_contiguous() or t.data_ptr() % 16:
+            return None
         L.tables[i] = t.data_ptr()
-    for k, v in shape.items():
-        if k == "orders":
-            for i, o in enumerate(v):
-                L.orders[i] = o
-            L.n_orders = len(v)
-        else:
-            setattr(L, k, v)
-    for k, v in floats.items():
-        setattr(L, k, v)
-    L.dtype = dtype_code(dtype)
+    for k, t in weights.items():
+        p = t.data_ptr()
+        if (t.size(-1), t.numel()) != weight_sizes[k] or t.dtype != dtype or t.device != device \
+                or not t.is_contiguous() or p % 16:
+            return None
+        setattr(L, k, p)
     return L
 
 
@@ -392,7 +407,9 @@ def memory_forward(layer, h: torch.Tensor, codes: torch.Tensor, max_workspace: i
     """The layer's output ``[B, T, hidden]`` (``lng_memory_forward``), or None when the intermediates
     take more than ``max_workspace`` bytes."""
     dev = _dev(h, codes)
-    b, t, _ = h.shape
+    b, t, d = h.shape
+    if d != layer.hidden or dtype_code(h.dtype) != layer.dtype or codes.shape != (b, t, layer.routes):
+        raise ValueError("memory_forward: h [B, T, hidden] in the layer's dtype, codes [B, T, R]")
     L = ctypes.byref(layer)
     nws = lib().lng_memory_forward_workspace_bytes(L, b, t)
     if not 0 < nws <= max_workspace:
@@ -405,32 +422,27 @@ def memory_forward(layer, h: torch.Tensor, codes: torch.Tensor, max_workspace: i
     return out
 
 
-def memory_step_caches_ok(code_cache: torch.Tensor, conv_cache: torch.Tensor, batch: int, max_len: int, routes: int,
-                          hidden: int) -> bool:
-    """Whether the caches are those that :func:`memory_step` writes: uint8 codes ``[batch, max_len, routes]`` and
-    bf16 conv inputs ``[batch, max_len, hidden]``, contiguous."""
-    return (code_cache.dtype == torch.uint8 and conv_cache.dtype == torch.bfloat16
-            and tuple(code_cache.shape) == (batch, max_len, routes) and tuple(conv_cache.shape) == (batch, max_len, hidden)
-            and code_cache.is_contiguous() and conv_cache.is_contiguous())
-
-
 def memory_step(layer, h: torch.Tensor, codes: torch.Tensor, pos0: int, code_cache: torch.Tensor,
-                conv_cache: torch.Tensor) -> torch.Tensor:
+                conv_cache: torch.Tensor):
     """The cached step's output ``[B, n, hidden]`` (``lng_memory_step``): ``codes [B, n, R]`` into
-    ``code_cache`` and the projected rows into ``conv_cache`` at ``pos0`` on."""
-    dev = _dev(h, codes, code_cache, conv_cache)
+    ``code_cache`` and the projected rows into ``conv_cache`` at ``pos0`` on.  None when these are not the
+    layer's: contiguous uint8 ``[B, S, R]`` and bf16 ``[B, S, hidden]`` caches with the new positions inside,
+    on the device of ``h [B, n, hidden]``."""
     b, n, d = h.shape
-    if d != layer.hidden or tuple(codes.shape) != (b, n, layer.routes) or \
-            not memory_step_caches_ok(code_cache, conv_cache, b, code_cache.shape[1], layer.routes, d):
-        raise ValueError("memory_step: h [B, n, hidden], codes [B, n, R], a uint8 [B, S, R] code cache and a bf16 "
-                         "[B, S, hidden] conv cache")
+    r, s = layer.routes, code_cache.shape[1]
+    dev = h.device
+    if d != layer.hidden or dtype_code(h.dtype) != layer.dtype or codes.shape != (b, n, r) \
+            or code_cache.shape != (b, s, r) or conv_cache.shape != (b, s, d) or pos0 + n > s or code_cache.dtype != torch.uint8 or conv_cache.dtype != torch.bfloat16 \
+            or not code_cache.is_contiguous() or not conv_cache.is_contiguous() \
+            or not dev == codes.device == code_cache.device == conv_cache.device:
+        return None
     hc, cc = _c(h), _codes_ok(codes)
     nws = 2 * (-(-b * n * d * h.element_size() // 256) * 256)
     ws = torch.empty(nws, dtype=torch.uint8, device=dev)
     out = torch.empty(h.shape, dtype=h.dtype, device=dev)
     check(lib().lng_memory_step(ctypes.byref(layer), _ptr(hc), _ptr(cc), dtype_code(cc.dtype), b, n, int(pos0),
-                                _ptr(code_cache), _ptr(conv_cache), code_cache.shape[1], _ptr(ws), nws, _ptr(out),
-                                _stream(dev)), "memory_step")
+                                _ptr(code_cache), _ptr(conv_cache), s, _ptr(ws), nws, _ptr(out), _stream(dev)),
+          "memory_step")
     return out
 
 
