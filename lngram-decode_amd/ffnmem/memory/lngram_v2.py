@@ -117,7 +117,7 @@ class _SurrogateLookup(torch.autograd.Function):
         ctx.cfg = cfg
         ctx.save_for_backward(q_logits, codes_chunk, *masks_and_tables)
         return ops.route_tokens(route_codes, [t.detach() for t in masks_and_tables[n:]], orders, bits, route_start,
-                                route_end, segment_ids, valid_tokens, None)
+                                route_end, segment_ids, valid_tokens, None, read_ahead=True)
 
     @staticmethod
     def backward(ctx, grad: Tensor):

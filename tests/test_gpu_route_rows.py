@@ -24,7 +24,7 @@ CASES = [
     (9, 129, 40, 1, 39, 32, (2, 3), 4, torch.float32, None, True),
     (2, 300, 97, 0, 97, 24, (2, 3), 4, torch.bfloat16, None, True),      # 48 bytes: one thread a piece
     (5, 391, 33, 0, 33, 128, (2, 3), 4, torch.bfloat16, None, True),     # 33.0 MB: non-temporal stores
-    (1, 4100, 20, 2, 19, 128, (2, 3), 4, torch.bfloat16, None, True),    # tables read ahead (4096 rows a route)
+    (1, 4100, 20, 2, 19, 128, (2, 3), 4, torch.bfloat16, None, True),    # as many positions as rows a route
 ]
 
 
@@ -48,6 +48,26 @@ def test_rows_equal_the_oracle(dev, case, codes_dtype):
                       for i, tab in enumerate(tables)], -1)[:, :, r0:r1]
     want = want if tail is None else want[:, -tail:]
     assert torch.equal(got.cpu(), want)
+
+
+def test_only_the_training_lookup_reads_ahead(dev, monkeypatch):
+    """A gather cannot tell whether its tables are cached: only the step that knows they are not, because its
+    backward came between, reads them first."""
+    from ffnmem.memory.lngram_v2 import RouteNgramMemoryV2
+
+    seen = []
+    real = ops._prefetch_tables
+    monkeypatch.setattr(ops, "_prefetch_tables", lambda *a: seen.append(1) or real(*a))
+    m = RouteNgramMemoryV2(1024, num_routes=20, readout_num_kv_heads=4, readout_head_dim=64, table_init_std_scale=1.0,
+                           device=dev, dtype=torch.bfloat16)
+    codes = torch.randint(0, 16, (1, 4100, 20), dtype=torch.uint8, device=dev)
+    q = torch.randn(1, 4100, 20, 4, device=dev, requires_grad=True)
+    tables = [m.tables[f"ngram_{o}"].weight.detach() for o in (2, 3)]
+    with torch.no_grad():
+        want = ops.route_tokens(codes, tables, (2, 3), 4)
+        m.eval()._lookup_route_chunk(codes, q, 0, 20, None, None)
+    assert not seen
+    assert torch.equal(m.train()._lookup_route_chunk(codes, q, 0, 20, None, None).detach(), want) and seen
 
 
 @pytest.mark.parametrize("lo,n", [(0, 0), (1, 15), (0, 16), (8, 40), (3, 70001), (0, 64 << 20)])
