@@ -168,20 +168,25 @@ __device__ __forceinline__ void store8(bf16* p, const float (&v)[8]) {
 }
 
 // TT positions x all channels a block of 256 threads.  The rows' loads of a wave go out together, then
-// their sums; a thread forms 8 channels of one output from its four rows (the block's rows are in L1 by
-// then).  A lane sums 8 consecutive elements, 512 apart, as k_conv_slots does.  4 x 128 x 128 fp32: 24.5
-// us with one wave-serial pass over the rows and 16 of 128 threads sliding over the positions.
-template <typename T, int TT>
-__global__ __launch_bounds__(256) void k_causal_conv_k4d3(const T* __restrict__ mixed, const T* __restrict__ norm_w,
+// their sums.  NO: outputs of a thread, 3 apart, for 8 channels: their NO + 3 rows, the norm's weights
+// and the taps loaded once.  1 where a block has few channels (all its threads at work, the rows in L1 by
+// then), (TT + 2) / 3 for wide rows, whose loads bound the block.  A lane sums 8 consecutive elements, 512
+// apart, as k_conv_slots does.  4 x 128 x 128 fp32: 24.5 us with one wave-serial pass over the rows and 16
+// of 128 threads sliding over the positions.
+template <typename T, int TT, int NO>
+__global__ __launch_bounds__(NO == 1 ? 256 : 512) void k_causal_conv_k4d3(const T* __restrict__ mixed, const T* __restrict__ norm_w,
                                                           const T* __restrict__ conv_w, ConvWin W, int32_t d,
                                                           float eps, int residual, T* __restrict__ out) {
   constexpr int NR = TT + C43_HALO, RPW = (NR + 3) / 4;
-  __shared__ float scale[RPW * 4];
+  __shared__ float scale[NR];
   const int64_t b = blockIdx.y;
   const int64_t p0 = conv_p0(W);
-  const int64_t t0 = p0 + static_cast<int64_t>(blockIdx.x) * TT;
+  // neighbouring tiles, which share halo rows, on one XCD (blocks go to the 8 XCDs in turn)
+  const unsigned bx = NO > 1 && gridDim.x % 8 == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int64_t t0 = p0 + static_cast<int64_t>(bx) * TT;
   const int64_t T_len = min(W.len, p0 + W.n);  // rows read and outputs end here
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nwave = NO == 1 ? 4 : static_cast<int>(blockDim.x) >> 6;  // 4 or more
   const T* base = mixed + b * W.stride * d;
   if (p0 < 0) return;
   float ss[RPW];
@@ -191,7 +196,7 @@ __global__ __launch_bounds__(256) void k_causal_conv_k4d3(const T* __restrict__ 
     float v[RPW][8];
 #pragma unroll
     for (int k = 0; k < RPW; ++k) {
-      const int i = wave + 4 * k;
+      const int i = wave + nwave * k;
       const int64_t t = t0 - C43_HALO + i;
       if (i < NR && t >= 0 && t < T_len) {
         load8(base + t * d + c, v[k]);
@@ -207,22 +212,25 @@ __global__ __launch_bounds__(256) void k_causal_conv_k4d3(const T* __restrict__ 
   }
 #pragma unroll
   for (int k = 0; k < RPW; ++k) {
-    const int i = wave + 4 * k;
+    const int i = wave + nwave * k;
     const int64_t t = t0 - C43_HALO + i;
     const float s = wave_sum(ss[k]);
-    if (lane == 0) scale[i] = t >= 0 && t < T_len ? 1.0f / sqrtf(s / static_cast<float>(d) + eps) : 0.f;
+    if (lane == 0 && i < NR) scale[i] = t >= 0 && t < T_len ? 1.0f / sqrtf(s / static_cast<float>(d) + eps) : 0.f;
   }
   __syncthreads();
   const int nch = d >> 3;
-  for (int e = threadIdx.x; e < TT * nch; e += 256) {
+  constexpr int GROUPS = NO == 1 ? TT : 3;  // a thread's first position: any, or one of three
+  static_assert(NO == 1 || 3 * NO >= TT, "positions covered");
+  for (int e = threadIdx.x; e < GROUPS * nch; e += NO == 1 ? 256 : static_cast<int>(blockDim.x)) {
     const int tt = e / nch, c = (e - tt * nch) * 8;
     const int64_t t = t0 + tt;
     if (t >= T_len) break;  // later items of this thread lie later still
-    float nw[8], x[4][8];  // x[k]: the row of tap k, at t - 9 + 3 k
+    float nw[8], x[NO + 3][8];  // x[k]: the row at t - 9 + 3 k
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (t - C43_HALO + 3 * k >= 0) {
-        load8(base + (t - C43_HALO + 3 * k) * d + c, x[k]);
+    for (int k = 0; k < NO + 3; ++k) {
+      const int64_t tr = t - C43_HALO + 3 * k;
+      if (tr >= 0 && tr < T_len && tt + 3 * k < NR) {
+        load8(base + tr * d + c, x[k]);
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[k][j] = 0.f;
@@ -240,22 +248,30 @@ __global__ __launch_bounds__(256) void k_causal_conv_k4d3(const T* __restrict__ 
         w[j + 1][k] = p[4 + k];
       }
     }
-    float o[8];
+    float h[4][8];  // normalised rows of an output's taps
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float h[4];
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        h[k] = t - C43_HALO + 3 * k >= 0 ? norm_elem<T, true>(x[k][j], scale[tt + 3 * k], nw[j]) : 0.f;
-      float acc = w[j][0] * h[0];
-      acc = fmaf(w[j][1], h[1], acc);
-      acc = fmaf(w[j][2], h[2], acc);
-      acc = fmaf(w[j][3], h[3], acc);
-      const float y = round_to<T>(acc);
-      const float act = round_to<T>(y / (1.0f + expf(-y)));
-      o[j] = residual ? x[3][j] + act : act;
+      for (int j = 0; j < 8; ++j)
+        h[k][j] = t - C43_HALO + 3 * k >= 0 ? norm_elem<T, true>(x[k][j], scale[tt + 3 * k], nw[j]) : 0.f;
+#pragma unroll
+    for (int q = 0; q < NO; ++q) {
+      const int64_t to = t + 3 * q;
+      if (to >= T_len || tt + 3 * q >= TT) break;
+      float o[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        h[(q + 3) & 3][j] = norm_elem<T, true>(x[q + 3][j], scale[tt + 3 * q + C43_HALO], nw[j]);
+        float acc = w[j][0] * h[q & 3][j];
+        acc = fmaf(w[j][1], h[(q + 1) & 3][j], acc);
+        acc = fmaf(w[j][2], h[(q + 2) & 3][j], acc);
+        acc = fmaf(w[j][3], h[(q + 3) & 3][j], acc);
+        const float y = round_to<T>(acc);
+        const float act = round_to<T>(y / (1.0f + expf(-y)));
+        o[j] = residual ? x[q + 3][j] + act : act;
+      }
+      store8(out + (b * W.n + to - p0) * d + c, o);
     }
-    store8(out + (b * W.n + t - p0) * d + c, o);
   }
 }
 
@@ -689,15 +705,34 @@ static int conv_launch(const void* mixed, const void* norm_w, const void* conv_w
     // 8 positions a block (17 rows) until 16 fill the chip twice over (25 rows, less of them halo)
     const bool small = B * cdiv(n, 16) < 512;
     dim3 g43(static_cast<unsigned>(cdiv(n, small ? 8 : 16)), static_cast<unsigned>(B));
+    // several outputs a thread from 384 channels on (fp32, us; one a thread / several / one wave-serial pass
+    // over the rows with 128 threads sliding over the positions):
+    //   rows       2048                 8192                 16384
+    //   256 wide    5.7 /  6.7 / 23.1   11.1 / 12.1 / 21.5   17.7 / 19.9 / 25.0
+    //   512         8.5 /  7.3 / 20.1   17.7 / 14.4 / 24.1   34.4 / 25.6 / 30.4
+    //   1024       13.4 /  9.5 / 23.2   37.6 / 23.6 / 37.9   72.5 / 43.4 / 44.2
+    //   2048       28.4 / 15.3 / 52.5   69.0 / 42.0 / 69.3  139.6 / 77.8 / 83.1
+    // The 3 d / 8 items of a block of a small launch in as few even rounds of up to 512 threads; in a large
+    // one more threads only push rows out of the L2 (1024 wide, 16384 rows: 49.8).
+    const bool wide = d >= 384;
+    const int64_t items = 3 * (d / 8), even = cdiv(cdiv(items, cdiv(items, 512)), 64) * 64;
+    const unsigned threads = wide && small && even > 256 ? static_cast<unsigned>(even) : 256;
     auto go = [&](auto* kern, auto* type) {
       using T = std::remove_pointer_t<decltype(type)>;
-      hipLaunchKernelGGL(kern, g43, dim3(256), 0, s, static_cast<const T*>(mixed), static_cast<const T*>(norm_w),
+      hipLaunchKernelGGL(kern, g43, dim3(threads), 0, s, static_cast<const T*>(mixed), static_cast<const T*>(norm_w),
                          static_cast<const T*>(conv_w), W, d, eps, residual, static_cast<T*>(out));
     };
+    auto pick = [&](auto* type) {
+      using T = std::remove_pointer_t<decltype(type)>;
+      if (small)
+        go(wide ? &k_causal_conv_k4d3<T, 8, 3> : &k_causal_conv_k4d3<T, 8, 1>, type);
+      else
+        go(wide ? &k_causal_conv_k4d3<T, 16, 6> : &k_causal_conv_k4d3<T, 16, 1>, type);
+    };
     if (dtype == LNG_F32)
-      go(small ? &k_causal_conv_k4d3<float, 8> : &k_causal_conv_k4d3<float, 16>, static_cast<float*>(nullptr));
+      pick(static_cast<float*>(nullptr));
     else
-      go(small ? &k_causal_conv_k4d3<bf16, 8> : &k_causal_conv_k4d3<bf16, 16>, static_cast<bf16*>(nullptr));
+      pick(static_cast<bf16*>(nullptr));
     return check_launch("causal_conv_k4d3");
   }
   dim3 grid(static_cast<unsigned>(cdiv(n, CONV_TT)), static_cast<unsigned>(B));
