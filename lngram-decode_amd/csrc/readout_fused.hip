@@ -535,7 +535,7 @@ __global__ __launch_bounds__(256) void k_readout_pack(const bf16* __restrict__ k
 using namespace lng;
 
 constexpr int64_t FR_ROUND = 4 * 2 * 256;  // tokens of a round of 4-token blocks, two a CU
-constexpr int64_t FR_TOKEN_MAX = 256, FR_SPLIT_MAX = 512;
+constexpr int64_t FR_TOKEN_MAX = 256;
 
 static int readout_launch(const void* q, const void* q_rows, float q_eps, const uint8_t* codes, const int32_t* seg,
                           const uint8_t* val, int64_t B, int64_t T,
@@ -552,14 +552,18 @@ static int readout_launch(const void* q, const void* q_rows, float q_eps, const 
   // buffer offsets are 32-bit: the token-major activations (2 KB per token) stay under 4 GB; the
   // 3-gram table (R <= 256 routes x 4096 rows x 256 B) always does
   if (ntok > (int64_t{1} << 21)) return fail(LNG_E_ARG, "memory_readout_fused: more than 2^21 tokens per launch");
-  // Few tokens leave the chip idle while each waits for its own chain of six chunks (184 routes), so
-  // their routes are split over a block's waves.  Times in us (184 routes), tokens:
-  //                            8     64    200    256    400    512    700   2331
-  //   four tokens a block   18.7   18.8   19.3   19.7   20.4   20.7   21.3   47.1
-  //   a token a block of 4  11.7   11.9   12.6   13.1   17.8   19.5   28.4   45.9 (the last 283 tokens)
-  //   a token a block of 8  10.5   10.8   11.8   12.4   24.0   26.3   38.4
-  // (one block of 8 waves or two of 4 fit a CU).  Past a whole round of 4-token blocks (2 x 256 of them)
-  // a remainder of up to 512 tokens is split too: the last round is then as short.
+  // Few tokens leave the chip idle while each waits for its own chain of 32-route chunks (six of 184
+  // routes), so their routes are split over a block's waves: eight up to 256 tokens (one block a CU), four
+  // up to 512 (two), with a single chunk only the former.  Past a whole round of 4-token blocks (512 of
+  // them) a remainder that fits one split block a CU, or few more where a token is long, is split too: the
+  // last round is then shorter.  Times in us, four tokens a block / split, for tokens of
+  //   routes           8        256           257           512          2304          2331          2560
+  //      8       9.5/7.8    9.6/8.1       9.6/10.1     9.8/10.9      20.8/20.2     20.8/21.9     21.2/22.8
+  //     64      11.1/8.0   11.2/8.5     11.3/10.6     11.9/11.5      27.6/26.2     27.6/27.9     27.8/29.4
+  //    128      14.5/8.8   15.3/9.7     15.5/11.8     16.4/15.0      37.4/33.6     37.5/36.9     38.1/38.6
+  //    184     18.7/10.1  19.7/11.8     19.3/14.5     20.4/19.7      47.1/42.4     47.3/46.3     47.8/49.0
+  //    256     21.4/11.0  23.5/14.3     23.6/16.8     24.3/23.4      60.4/52.6     60.7/57.8     61.0/60.2
+  const int64_t chunks = cdiv(R, 32);
   if (ntok <= FR_TOKEN_MAX) {
     hipLaunchKernelGGL(k_readout_token, dim3(static_cast<unsigned>(ntok)), dim3(512), 0, as_stream(stream),
                        static_cast<const bf16*>(q), static_cast<const bf16*>(q_rows), q_eps, codes, seg, val, B, T, R, cstride,
@@ -570,7 +574,8 @@ static int readout_launch(const void* q, const void* q_rows, float q_eps, const 
   }
   int64_t full = blocks;
   const int64_t rem = ntok % FR_ROUND;
-  if (FR_TOK == 4 && rem <= FR_SPLIT_MAX) {
+  const int64_t most = ntok < FR_ROUND ? (chunks > 1 ? 512 : 0) : 256 + (chunks > 4 ? 64 * (chunks - 4) : 0);
+  if (FR_TOK == 4 && rem <= most) {
     full = (ntok - rem) / 4;
     blocks = full + rem;
   }
