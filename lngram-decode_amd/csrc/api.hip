@@ -109,9 +109,9 @@ __global__ void k_ngram_rows(CodeView codes, int64_t B, int64_t T, int32_t R, in
 constexpr int RR_POS = 64;
 constexpr int64_t RR_NT_BYTES = int64_t{32} << 20;  // past the eight L2s together
 // Below this many bytes a launch is one short wave of blocks and its time is the chain codes -> index
-// -> row -> store, which one thread a piece walks without the barrier (a tree's 1.5 MB: 4.8 against
-// 5.1 us).
-constexpr int64_t RR_MIN_BYTES = int64_t{4} << 20;
+// -> row -> store, which one thread a piece walks without the barrier (4.2 MB, 8 routes: 4.6 us against
+// 5.7; 5.9 MB, 184 routes: 5.4 against 6.0; 8.4 MB: 6.3 either way; 24 MB: 13.8 against 9.8).
+constexpr int64_t RR_MIN_BYTES = int64_t{8} << 20;
 template <bool NT>
 __global__ __launch_bounds__(256) void k_route_rows(CodeView codes, int64_t T, int64_t t_first, int64_t T_out,
                                                     int64_t W, int32_t R, int32_t rs, int32_t rw, OrderList ords,

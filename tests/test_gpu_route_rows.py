@@ -24,6 +24,9 @@ CASES = [
     (9, 129, 40, 1, 39, 32, (2, 3), 4, torch.float32, None, True),
     (2, 300, 97, 0, 97, 24, (2, 3), 4, torch.bfloat16, None, True),      # 48 bytes: one thread a piece
     (5, 391, 33, 0, 33, 128, (2, 3), 4, torch.bfloat16, None, True),     # 33.0 MB: non-temporal stores
+    (1, 63, 300, 0, 300, 128, (2, 3), 4, torch.bfloat16, None, True),    # past the tiled copy's line: one short tile
+    (1, 96, 201, 3, 201, 64, (1, 2, 3, 4), 2, torch.bfloat16, None, True),
+    (3, 260, 3, 0, 3, 1024, (1,), 4, torch.float32, None, False),        # 4 KB rows: one row a block pass
     (1, 4100, 20, 2, 19, 128, (2, 3), 4, torch.bfloat16, None, True),    # as many positions as rows a route
 ]
 
