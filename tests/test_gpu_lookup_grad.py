@@ -113,3 +113,42 @@ def test_other_shapes_take_the_orders_kernels(dev, R, exact):
     per = [ops.surrogate_grad(args[0][..., i * 128:(i + 1) * 128].contiguous(), None, args[1], args[2], args[3][i],
                               args[4][i], o, 4, 0, 0.8, 1.2, exact) for i, o in enumerate((2, 3))]
     assert torch.equal(gq, per[0] + per[1]) and gt[0].shape == args[3][0].shape
+
+
+@pytest.mark.parametrize("mean", [0.0, 1.0])        # rows with a common part: their scores cancel
+def test_no_further_from_fp64_than_order_by_order(dev, mean):
+    B, T, R = 2, 200, 64
+    codes, tables, q, grad, masks, args = _inputs((B, T, R, 0, "random", torch.float32, torch.uint8, False), dev)
+    tables = [(t.float() * 0.04 + mean).to(torch.bfloat16) for t in tables]
+    args = args[:3] + ([t.to(dev) for t in tables],) + args[4:]
+    g, qd, cd, td, md = args[:5]
+    gq, _ = ops.lookup_grad(*args, (True, False, False))
+    per = [ops.surrogate_grad(g[..., i * 128:(i + 1) * 128].contiguous(), None, qd, cd, td[i], md[i], o, 4, 0, 0.8, 1.2,
+                              False, workspace=False) for i, o in enumerate((2, 3))]
+    ref = 0
+    for i, o in enumerate((2, 3)):
+        rows = om.route_rows(codes.numpy(), [o], 4, 0, R)[..., 0]
+        hard = tables[i][torch.from_numpy(rows.clip(0))] * torch.from_numpy(rows >= 0)[..., None]
+        ref = ref + om.surrogate_grad(grad[..., i * 128:(i + 1) * 128].double(), hard.double(), q.double(), codes.numpy(),
+                                      tables[i].double(), masks[i], o, 4, 0, 0.8, 1.2, False).double()
+    one, many = (float((x.cpu().double() - ref).norm()) for x in (gq, per[0] + per[1]))
+    assert one <= 1.02 * many                        # 102 400 sums: the two norms are known to under 1 %
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_values_that_are_not_finite_stay_where_they_are(dev, bad):
+    case = (1, 130, 8, 0, "random", torch.float32, torch.uint8, False)
+    codes, _, _, grad, _, args = _inputs(case, dev)
+    gq, gt = ops.lookup_grad(*args, (True, True, True))
+    t, r = 60, 3
+    args[0][0, t, r, 7] = bad                        # the order-2 part of one window's gradient
+    bq, bt = ops.lookup_grad(*args, (True, True, True))
+    keep = torch.ones(1, 130, 8, dtype=torch.bool)
+    keep[0, t - 1:t + 1, r] = False                  # the logits of its two positions
+    assert torch.equal(bq[keep], gq[keep]) and not torch.isfinite(bq[~keep]).all(-1).any()
+    row = r * 256 + int(codes[0, t - 1, r] + 16 * codes[0, t, r])
+    rows = torch.arange(bt[0].shape[0]) != row
+    # a row's own sum may add its windows in another order from call to call
+    assert torch.isfinite(bt[0][rows].float()).all() and not torch.isfinite(bt[0][row, 7].float())
+    assert om.rel_err(bt[0][rows].float().cpu(), gt[0][rows].float().cpu()) < 2.0 ** -8
+    assert torch.isfinite(bt[1].float()).all()
