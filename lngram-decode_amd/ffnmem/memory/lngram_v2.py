@@ -8,7 +8,7 @@ methods that the reference's callers use (``quantize_route_logits``,
 ``lngram_hip``; tensors must be on a ROCm device.
 
 Scope: the eval-mode forward, and the training-mode lookup with its surrogate route gradient
-(``_LngramSurrogate``, ``lngram_v2.py:328-464``: ``_lookup_route_chunk`` with route logits under
+(``lngram_v2.py:328-464``, here ``_SurrogateLookup``: ``_lookup_route_chunk`` with route logits under
 autograd gives the route logits their counterfactual gradient and the tables their gather
 gradient, both on gfx950 kernels).  The readout after the lookup has no backward here, so the
 module's forward in training mode, dropout and the context-parallel / streaming-state /
@@ -413,9 +413,10 @@ class _RouteNgramMemoryBase(nn.Module):
         """Route tokens ``[B, T, route_end-route_start, len(ngrams)*mem_dim]`` (``lngram_v2.py:1047-1113``):
         ``lng_route_tokens`` gathers every order's row (zero where masked) in one pass.
 
-        In training with route logits under autograd, each order's rows come from ``_TableRows``
-        (table gradient on the backward) through ``_LngramSurrogate`` (route-logit gradient), as in
-        the reference (``:1093-1109``)."""
+        In training with route logits under autograd, ``_SurrogateLookup`` gives the rows of all orders
+        the tables' gather gradients and the route logits' surrogate gradient (the reference's
+        ``:1093-1109``); tables that were given different types or widths go order by order, through
+        ``_TableRows`` and ``_LngramSurrogate``."""
         self._check_dropout()
         if self._use_surrogate(q_logits_btrm):
             if target_length is not None:

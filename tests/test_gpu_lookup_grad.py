@@ -152,3 +152,31 @@ def test_values_that_are_not_finite_stay_where_they_are(dev, bad):
     assert torch.isfinite(bt[0][rows].float()).all() and not torch.isfinite(bt[0][row, 7].float())
     assert om.rel_err(bt[0][rows].float().cpu(), gt[0][rows].float().cpu()) < 2.0 ** -8
     assert torch.isfinite(bt[1].float()).all()
+
+
+def test_tables_of_two_types_go_order_by_order(dev):
+    """A module whose tables were given different types by hand: rows and gradients of each order's own path."""
+    from ffnmem.memory.lngram_v2 import RouteNgramMemoryV2
+
+    R, B, T = 5, 2, 40
+    m = RouteNgramMemoryV2(1024, num_routes=R, readout_num_kv_heads=4, readout_head_dim=64, table_init_std_scale=1.0,
+                           device=dev, dtype=torch.float32).train()
+    t2, t3 = (m.tables[f"ngram_{o}"] for o in (2, 3))
+    t3.to(torch.bfloat16)
+    gen = torch.Generator(device=dev).manual_seed(3)
+    codes = torch.randint(0, 16, (B, T, R), generator=gen, device=dev, dtype=torch.uint8)
+    q = torch.randn(B, T, R, 4, generator=gen, device=dev, requires_grad=True)
+    grad = torch.randn(B, T, R, 256, generator=gen, device=dev)
+    rows = m._lookup_route_chunk(codes, q, 0, R, None, None)
+    gq, g2, g3 = torch.autograd.grad(rows, [q, t2.weight, t3.weight], grad)
+    want_q = 0
+    for i, (o, tab, g) in enumerate(((2, t2.weight, g2), (3, t3.weight, g3))):
+        part, w = grad[..., i * 128:(i + 1) * 128], tab.detach()
+        assert torch.equal(rows[..., i * 128:(i + 1) * 128], ops.route_tokens(codes, [w], [o], 4).float())
+        valid = m._valid_mask(o, B, T, dev, None, None)
+        part = part.to(w.dtype)                      # the concatenation's backward gives each part its own type
+        want_q = want_q + ops.surrogate_grad(part, None, q.detach(), codes, w, valid, o, 4, 0, m.q_surrogate_temperature,
+                                             m.q_surrogate_scale, False)
+        want = ops.table_grad_rows(part, codes, valid, o, 4, 0, w.shape[0], w.dtype)
+        assert g.dtype == w.dtype and om.rel_err(g.float().cpu(), want.float().cpu()) < (1e-6 if i == 0 else 2.0 ** -8)
+    assert om.rel_err(gq.cpu(), want_q.cpu()) < 1e-6
