@@ -64,3 +64,35 @@ def test_values_that_are_not_finite_stay_in_their_token(dev, bad):
         assert not torch.isfinite(got[0, 100].float()).all()
         got[0, 100] = want[0, 100]
         assert torch.equal(got, want)
+
+
+def test_trees_of_many_sequences_equal_their_chains(dev):
+    """Draft-tree verification of 17 sequences (272 nodes: past the one-token blocks of the readout and the
+    skinny projections) against chain decodes of 17 rows, bit for bit."""
+    from drafting.tree import tree16
+    from ffnmem.infer import DecodeState, memory_codes, memory_model, memory_step, tree_memory_step
+    from lngram_hip import workloads as wl
+
+    parent, b, L = tree16().parent, 17, 5
+    n = len(parent)
+    w = wl.SB.with_shape(b, L + n)
+    mem, h = wl.build_memory(w, seed=0, device=dev), wl.make_hidden(w, seed=1, device=dev)
+    h_norm = ops.rmsnorm(h, torch.ones(w.d_model, dtype=w.dtype, device=dev), w.norm_eps)
+    model, rows = memory_model(mem), torch.arange(b, device=dev)
+    with torch.no_grad():
+        st = DecodeState.empty(model, b, L + n)
+        memory_step(model, 0, st, h[:, :L].contiguous(), memory_codes(model, 0, st, h_norm=h_norm[:, :L].contiguous()))
+        st.length = L
+        base = st.index_select(rows)
+        hn = h[:, L:].contiguous()
+        codes = memory_codes(model, 0, st, h_norm=h_norm[:, L:].contiguous())
+        got = tree_memory_step(model, 0, st, hn, codes, parent)
+        for i in (0, 3, n - 1):
+            path = [i]
+            while parent[path[0]] >= 0:
+                path.insert(0, parent[path[0]])
+            sti = base.index_select(rows)
+            for p in path:
+                out = memory_step(model, 0, sti, hn[:, p:p + 1].contiguous(), codes[:, p:p + 1].contiguous())
+                sti.length += 1
+            assert torch.equal(got[:, i:i + 1], out), i
