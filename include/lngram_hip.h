@@ -286,7 +286,10 @@ int lng_causal_conv_rowsq(const void* mixed, const float* rowsq, int32_t n_parti
  *   kv_pack  [LNG_READOUT_PACK_ELEMS] bf16, readout_kv_proj.weight in the kernel's operand
  *            order, made by lng_memory_readout_pack (once per weight version)
  *   w_mem    [256]           readout_memory_norm.weight
- *   head_out [N_tok, 16*64]  attention output (input of readout_o_proj) */
+ *   head_out [N_tok, 16*64]  attention output (input of readout_o_proj)
+ * A token's output does not depend on how many tokens share the launch, nor on its place among them:
+ * every form of the kernel (one token, four or eight a block, a token's routes split over waves) sums the
+ * route chunks in the same order. */
 #define LNG_READOUT_PACK_ELEMS 131072
 int lng_memory_readout_fused(const void* q, const void* q_rows, float q_eps, const uint8_t* codes, int64_t B,
                              int64_t T, int32_t R, const void* table2, const void* table3, const void* kv_pack,
@@ -421,7 +424,8 @@ int lng_table_grad_rows(const void* grad_memory, int mem_dtype, int64_t grad_str
  * reading of grad_memory [B, T, R, 2 * mem_dim] (order 2's half first, rows grad_stride elements
  * apart).  Any of the three gradients may be null (not wanted).  Serves the shapes for which
  * lng_lookup_grad_workspace_bytes gives a size (bf16 rows of 128, 4-bit codes, exact = 0, R <= 256,
- * B*T < 2^20); rows and tables 16-byte aligned, the workspace (written before it is read) 256-byte. */
+ * B*T < 2^20).  grad_q is the same in every call; as in lng_table_grad_rows the order in which a row's
+ * windows are summed varies between calls, and with it the rounding of the table gradients.  Rows and tables 16-byte aligned, the workspace (written before it is read) 256-byte. */
 size_t lng_lookup_grad_workspace_bytes(int64_t B, int64_t T, int32_t R, int32_t mem_dim, int32_t bits, int mem_dtype,
                                        int exact);
 int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t grad_stride, const void* q_logits, int q_dtype,

@@ -180,3 +180,17 @@ def test_tables_of_two_types_go_order_by_order(dev):
         want = ops.table_grad_rows(part, codes, valid, o, 4, 0, w.shape[0], w.dtype)
         assert g.dtype == w.dtype and om.rel_err(g.float().cpu(), want.float().cpu()) < (1e-6 if i == 0 else 2.0 ** -8)
     assert om.rel_err(gq.cpu(), want_q.cpu()) < 1e-6
+
+
+def test_the_logits_gradient_repeats_and_a_table_row_keeps_its_bound(dev):
+    """The order of a row's windows may vary between calls: the logits' gradient does not depend on it, a
+    table row of n windows by n * 2^-24 * sum|g| and one bf16 rounding at most."""
+    codes, tables, q, grad, masks, args = _inputs((2, 700, 9, 0, "few", torch.float32, torch.uint8, False), dev)
+    first = ops.lookup_grad(*args, (True, True, True))
+    mass = ops.lookup_grad(args[0].abs(), *args[1:], (False, True, True))[1]
+    for _ in range(5):
+        gq, gt = ops.lookup_grad(*args, (True, True, True))
+        assert torch.equal(gq, first[0])
+        for a, b, m in zip(gt, first[1], mass):
+            bound = 2 * 1400 * 2.0 ** -24 * 1.01 * m.float() + 2.0 ** -7 * torch.maximum(a.float().abs(), b.float().abs())
+            assert bool(((a.float() - b.float()).abs() <= bound).all())
