@@ -1192,15 +1192,18 @@ static int launch_skinny(const bf16* w, const bf16* x, int64_t N, int64_t M, int
 
 // The tile of a shape, by the blocks it makes: a block's K loop takes about 5 us at K = 1024 however
 // small the tile, so the smallest tile that still fits the chip at 2-3 blocks a CU wins, and past that
-// the larger tile's fewer operand bytes.  Measured at K = 1024 (us; N 1024: the 128-row DMA tile up to
-// M 1000, then the 256-row projection tile; N 736: the router on the 128-row tile, M 8192 on the wide
-// one):
-//   M             200    500    777   1500   2331   4095   6000   8192
-//   N 1024 before 15.8   16.0   16.2   21.4   22.0   22.2   23.2   25.1
-//          here    5.0    5.5    6.4    8.4   13.0   15.5   23.3  (29.7: not taken)
-//   N 736  before 15.8   15.9   15.8   16.0   16.2   16.6   25.1   26.3
-//          here    5.2    5.6    6.2    7.9    9.2   13.2   20.8   22.1
-//   N 1024 with row statistics before: 34.3 35.6 35.7 21.7 22.0 23.1 24.7; here 7.2 7.3 7.6 9.1 14.1 16.0 24.3
+// the larger tile's fewer operand bytes.  Measured (us; before: the 128-row DMA tile up to M 1000, then the
+// 256-row projection tile, and for the router the 128-row tile up to M 4095, then the wide one):
+//   M                              200    777   1500   2331   4095   6000   8192
+//   N 1024, K 1024 before         15.8   16.0   21.1   21.6   22.5   23.6   25.0
+//                  here            4.0    5.5    7.2   12.4   15.3   21.1  (24.0: not taken)
+//     with row statistics before  34.2   35.8   21.9   22.4   23.0   23.8   24.8
+//                  here            6.6    7.0    8.7   14.3   16.1   21.8  (24.4: not taken)
+//   router N 736, K 1024 before   16.1   16.2   16.4   16.7   17.2   27.7   27.8
+//                  here            4.1    5.6    8.2    9.2   13.9   20.2   21.0
+//   router N 724, K 2304 before   30.7   31.2   31.4   31.4   32.0   49.7   50.1
+//                  here            8.5   12.2   17.8   18.1   27.2   40.5   42.1
+// The lines lie in blocks, not in M, so they hold for the longer K too: every block's time grows with it.
 enum { TILE_NONE, TILE_32_32, TILE_64_32, TILE_64_64, TILE_128_32, TILE_128_64 };
 static int pick_tile(int64_t N, int64_t M, int64_t K, bool rowsq) {
   if (M <= SK_MAXM || K % 64 != 0 || N % 4 != 0 || N * K * 2 >= (int64_t{1} << 31)) return TILE_NONE;
@@ -1305,8 +1308,10 @@ static int launch_tile_f32(const float* x, const float* w, int64_t M, int64_t N,
                        n_tiles, y, codes, codes_dt);
     return check_launch("gemm_f32_tile");
   };
-  // small tiles while they make few blocks a CU: 584 blocks of 32 x 32 took 18.8 us at 2331 x 256 x 1024
-  // against 24.2 in 64 x 64; 8192 of them 177 us at 32768 x 256 x 1024 against 143 (128 x 64: 138)
+  // small tiles while they make few blocks a CU, 32 x 32 against 64 x 64 (us): 512 blocks 15.2 to 22.4
+  // (2048 x 256 x 1024) and 14.3 to 21.9 (512 x 1024 x 1024); 1024 blocks 8.5 to 8.2 (2048 x 512 x 256)
+  // and 5.8 to 5.7 (8192 x 128 x 128), but 5.8 to 7.7 where 64 columns would be half padding (32768 x 32
+  // x 128); 2048 blocks 46.8 to 39.8 (8192 x 256 x 1024); 8192 blocks 159 to 135 (32768 x 256 x 1024)
   if (cdiv(N, 32) * cdiv(M, 32) <= 1024) return go(&k_gemm_tile_f32<32, 32>, 32, 32);
   return go(&k_gemm_tile_f32<64, 64>, 64, 64);
 }
