@@ -1317,7 +1317,9 @@ __device__ void sl_write(const lng_drafter& D, int j, int K, const DrChildren& C
 
 // The shortlist drafts of P positions given their full-vocabulary logits [P, V] and top-k: the
 // candidates' logits are read from the logits; an empty list keeps the full-vocabulary top-k
-// (full_ids / full_sc).                                            grid (P)
+// (full_ids / full_sc).  256 threads, unlike the list block of k_sm_attend: this launch follows a pass over
+// the whole vocabulary and serves only the shapes that the listed scoring (k_sl_score) does not take, and
+// sl_topk and sl_write, which it shares with k_sl_score, are written for 256.          grid (P)
 __global__ __launch_bounds__(256) void k_draft_shortlist(lng_drafter D, DrWin W, SlArgs S,
                                                          const float* __restrict__ logits,
                                                          const int64_t* __restrict__ full_ids,

@@ -77,6 +77,11 @@ class KernelTimer:
     every launch, or every ``every``-th one (a timing event pair costs a few microseconds of
     device time, so a long timed loop brackets a sample of its launches).
 
+    While a timer is active, the memory layer runs op by op, so that each op has a launch of its
+    own to bracket; without one it runs as one library call (:func:`memory_forward`,
+    :func:`memory_step`).  The kernels are the same, the host work of a call is not: a short call
+    timed with a timer active takes longer than the call that users make.
+
         with ops.KernelTimer("memory_readout_fused", every=5) as kt:
             ...                       # launches 0, 5, 10, ... are bracketed by events
         kt.mean_ms()                  # average device duration per bracketed launch (synchronises)

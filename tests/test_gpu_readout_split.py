@@ -2,8 +2,8 @@
 lines between its forms, route counts around the 32-route chunks, the first positions (no rows), and
 the cached and supplied-row modes.
 
-Against fp64 the readout is bf16 operands with fp32 sums (2e-2 norm-relative, the layer's bound); a
-token's output in one form against another differs by roundings of the same bf16 values (2^-7)."""
+Against fp64 the readout is bf16 operands with fp32 sums (2e-2 norm-relative, the layer's bound); one
+form against another is held to 2^-7 here, and bit for bit in ``test_gpu_readout_bits.py``."""
 
 from __future__ import annotations
 
