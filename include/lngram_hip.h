@@ -240,9 +240,9 @@ int lng_linear_rowsq(const void* x, const void* w, int64_t M, int64_t N, int64_t
 
 /* fp32 y[M,N] = RMSNorm(x[M,K]) . w[N,K]^T for bf16 x and fp32 w, norm_w: the SSM's input projection
  * u = W_in RMSNorm(x.float()) (DiagonalSSM.inputs, ssm.py:41-43) from the bf16 embeddings, bit for bit
- * lng_rmsnorm of the rows in fp32 and lng_linear of its result.  x, w and y 16-byte aligned.  Shapes:
- * lng_linear_split_workspace_bytes(N, K) != 0 (N % 4 == 0, K % 64 == 0, K <= 4096).  The workspace is not
- * used any more and may be NULL. */
+ * lng_rmsnorm of the rows in fp32 and lng_linear of its result.  x and y 16-byte aligned.  Shapes:
+ * lng_linear_split_workspace_bytes(N, K) != 0 (N % 4 == 0, K % 64 == 0).  The workspace (16-byte aligned)
+ * takes a copy of a w that is not 16-byte aligned; with an aligned w it may be NULL. */
 size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K);
 int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t M, int64_t N, int64_t K, float eps,
                      void* workspace, size_t workspace_bytes, float* y, void* stream);

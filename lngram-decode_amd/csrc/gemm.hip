@@ -903,8 +903,9 @@ __global__ __launch_bounds__(256) void k_gemm_tile_f32(const float* __restrict__
 // alone 135).  Bound by the fp32 matrix rate and what a wave's operands wait for beside it; x pieces
 // turned into fp32 once a block, through registers into the ring, took 169 to 198 us.  The weight as
 // three bf16 pieces (exact products, the row scale on the sums) takes 60, but its sums round otherwise.
+// NWL: the norm's weights in LDS (K <= 4096), otherwise read from memory as they are used.
 constexpr int NG_MAXK = 4096;
-template <int BN, int BM, int WN, int WM>
+template <int BN, int BM, int WN, int WM, bool NWL>
 __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, const float* norm_w, int64_t N, int64_t M,
                                               int64_t K, int n_tiles, float eps, float* Y) {
   using G = TileGemm<float, BN, BM, WN, WM, 3>;
@@ -915,7 +916,7 @@ __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, con
   static_assert(BN % (8 * NWAVE) == 0 && BM % (8 * NWAVE) == 0 && W_LOADS + X_LOADS <= 60, "tile split");
   // one LDS object: with several the compiler tells them apart by alias scopes, and then waits for every
   // load in flight to LDS before it reads the ring
-  __shared__ __attribute__((aligned(16))) char ring[SLOTS * SLOT + BM * 4 + NG_MAXK * 4];
+  __shared__ __attribute__((aligned(16))) char ring[SLOTS * SLOT + BM * 4 + (NWL ? NG_MAXK * 4 : 0)];
   float* scale = reinterpret_cast<float*>(ring + SLOTS * SLOT);
   float* nw = scale + BM;  // norm_w[K]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -954,7 +955,8 @@ __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, con
   };
 #pragma unroll
   for (int s = 0; s < SLOTS - 1; ++s) issue(s, s);  // nk >= 2
-  for (int i = threadIdx.x; i < K; i += 64 * NWAVE) nw[i] = norm_w[i];
+  if constexpr (NWL)
+    for (int i = threadIdx.x; i < K; i += 64 * NWAVE) nw[i] = norm_w[i];
   // row scales in k_rmsnorm's order: 64 chains (elements 64 apart) and their sums pairwise.  A lane has 8
   // chains of a row, 8 lanes a row, so that its loads are whole pieces.
 #pragma unroll
@@ -996,6 +998,11 @@ __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, con
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // stage kt has landed for every wave, and every wave has read the slot of stage kt - 1
     __builtin_amdgcn_s_barrier();
+    float nv[8];  // from memory ahead of the ring's loads, so that waiting for them leaves those in flight
+    if constexpr (!NWL) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nv[e] = norm_w[kt * K_ST + psel + 4 * e];
+    }
     if (kt + SLOTS - 1 < nk) issue(kt + SLOTS - 1, (slot + SLOTS - 1) % SLOTS);
     const float* ws = reinterpret_cast<const float*>(ring + slot * SLOT);
     const bf16* xs = reinterpret_cast<const bf16*>(ring + slot * SLOT + BN * 128);
@@ -1013,7 +1020,7 @@ __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, con
         for (int e = 0; e < 4; ++e) {
           const int k = 4 * e + psel;  // of the half's 16: piece 2 h + k / 8
           const float x = static_cast<float>(row[8 * ((2 * h + (e >> 1)) ^ ((rsel >> 2) & 3)) + (k & 7)]);
-          b[j][e] = (x * rs[j]) * np[16 * h + 4 * e];
+          b[j][e] = (x * rs[j]) * (NWL ? np[16 * h + 4 * e] : nv[4 * h + e]);
         }
       }
 #pragma unroll
@@ -1043,11 +1050,16 @@ __device__ __forceinline__ void norm_gemm_f32(const float* W, const bf16* X, con
   }
 }
 
-template <int BN, int BM, int WN, int WM>
+template <int BN, int BM, int WN, int WM, bool NWL>
 __global__ __launch_bounds__(64 * WN * WM) void k_norm_gemm_f32(const float* __restrict__ W, const bf16* __restrict__ X,
                                                                 const float* __restrict__ norm_w, int64_t N, int64_t M,
                                                                 int64_t K, int n_tiles, float eps, float* __restrict__ Y) {
-  norm_gemm_f32<BN, BM, WN, WM>(W, X, norm_w, N, M, K, n_tiles, eps, Y);
+  norm_gemm_f32<BN, BM, WN, WM, NWL>(W, X, norm_w, N, M, K, n_tiles, eps, Y);
+}
+
+__global__ __launch_bounds__(256) void k_copy_f32(const float* __restrict__ src, int64_t n, float* __restrict__ dst) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
 }
 
 // fp32 VALU tile GEMM: 64x64 tile per 256-thread block, 4x4 outputs per thread,
@@ -1389,26 +1401,36 @@ int lng_linear_rowscale(const void* x, const void* w, int64_t M, int64_t N, int6
                      as_stream(stream), true, eps);
 }
 
-// whole stages, whole 16-byte outputs, the norm's weights in LDS
+// whole stages, whole 16-byte outputs
 static bool split_shape(int64_t N, int64_t K) {
-  return N > 0 && K > 0 && N % 4 == 0 && K % 64 == 0 && K <= NG_MAXK && N * K * 4 < (int64_t{1} << 31);
+  return N > 0 && K > 0 && N % 4 == 0 && K % 64 == 0 && N * K * 4 < (int64_t{1} << 31);
 }
-size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K) { return split_shape(N, K) ? 16 : 0; }
+// room for an aligned copy of w
+size_t lng_linear_split_workspace_bytes(int64_t N, int64_t K) {
+  return split_shape(N, K) ? static_cast<size_t>(N * K * 4) : 0;
+}
 
 int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t M, int64_t N, int64_t K, float eps,
-                     void*, size_t, float* y, void* stream) {
+                     void* workspace, size_t workspace_bytes, float* y, void* stream) {
   if (M < 0 || !split_shape(N, K))
-    return fail(LNG_E_ARG, "linear_split: needs N % 4 == 0, K % 64 == 0 and K <= 4096 (lng_linear_split_workspace_bytes)");
+    return fail(LNG_E_ARG, "linear_split: needs N % 4 == 0 and K % 64 == 0 (lng_linear_split_workspace_bytes)");
   if (M == 0) return LNG_OK;
   if (!x || !norm_w || !w || !y) return fail(LNG_E_ARG, "linear_split: null buffer");
   auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!al(x) || !al(w) || !al(y)) return fail(LNG_E_ARG, "linear_split: x, w and y must be 16-byte aligned");
+  if (!al(x) || !al(y)) return fail(LNG_E_ARG, "linear_split: x and y must be 16-byte aligned");
   hipStream_t s = as_stream(stream);
+  if (!al(w)) {  // the kernel reads whole 16-byte pieces of it
+    if (!workspace || !al(workspace) || workspace_bytes < lng_linear_split_workspace_bytes(N, K))
+      return fail(LNG_E_ARG, "linear_split: a w that is not 16-byte aligned needs the workspace, 16-byte aligned");
+    float* copy = static_cast<float*>(workspace);
+    hipLaunchKernelGGL(k_copy_f32, dim3(static_cast<unsigned>(cdiv(N * K, 256))), dim3(256), 0, s, w, N * K, copy);
+    w = copy;
+  }
   const bf16* xp = static_cast<const bf16*>(x);
-  auto go = [&](auto* kern, int64_t bn, int64_t bm) {
+  auto go = [&](auto* lds, auto* mem, int64_t bn, int64_t bm) {
     const int n_tiles = static_cast<int>(cdiv(N, bn));
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, xp, norm_w, N, M,
-                       K, n_tiles, eps, y);
+    hipLaunchKernelGGL(K <= NG_MAXK ? lds : mem, dim3(static_cast<unsigned>(n_tiles * cdiv(M, bm))), dim3(256), 0, s, w, xp,
+                       norm_w, N, M, K, n_tiles, eps, y);
     return check_launch("linear_split");
   };
   // by blocks (N 256, K 1024; us):   M  200  1000  2331  8192  32768
@@ -1417,10 +1439,10 @@ int lng_linear_split(const void* x, const float* norm_w, const float* w, int64_t
   //   128 x 64                        44.8  45.2  45.7  49.6    158
   // fp32 copy, norm pass and VALU product: 164 170 181 212 473
   const int64_t b32 = cdiv(N, 32) * cdiv(M, 32);
-  if (b32 <= 640) return go(&k_norm_gemm_f32<32, 32, 2, 2>, 32, 32);
-  if (b32 <= 1024) return go(&k_norm_gemm_f32<64, 64, 2, 2>, 64, 64);
-  if (N <= 64) return go(&k_norm_gemm_f32<64, 64, 2, 2>, 64, 64);  // (N 64, K 256, 32768 rows: 16.8; 128 x 64 24.1)
-  return go(&k_norm_gemm_f32<128, 64, 2, 2>, 128, 64);
+  if (b32 <= 640) return go(&k_norm_gemm_f32<32, 32, 2, 2, true>, &k_norm_gemm_f32<32, 32, 2, 2, false>, 32, 32);
+  if (b32 <= 1024 || N <= 64)  // (N 64, K 256, 32768 rows: 16.8; 128 x 64 24.1)
+    return go(&k_norm_gemm_f32<64, 64, 2, 2, true>, &k_norm_gemm_f32<64, 64, 2, 2, false>, 64, 64);
+  return go(&k_norm_gemm_f32<128, 64, 2, 2, true>, &k_norm_gemm_f32<128, 64, 2, 2, false>, 128, 64);
 }
 
 int lng_linear(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, void* y, void* stream) {

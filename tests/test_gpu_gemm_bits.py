@@ -94,7 +94,8 @@ def test_fp32_buffers_of_any_alignment(dev, which, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 256, 1024), (33, 4, 64), (200, 36, 128), (2560, 256, 192), (2561, 256, 64),
-                                   (4097, 260, 128), (8192, 256, 1024), (20000, 64, 256), (3, 8, 4096)])
+                                   (4097, 260, 128), (8192, 256, 1024), (20000, 64, 256), (3, 8, 4096),
+                                   (33, 36, 4160), (1100, 1028, 4160), (5000, 260, 8192)])
 def test_norm_and_product_in_one_pass(dev, m, n, k):
     gen = torch.Generator().manual_seed(m + n + k)
     x = (torch.randn(m, k, generator=gen) * torch.exp2(torch.randint(-30, 30, (m, 1), generator=gen).float()))
@@ -107,3 +108,32 @@ def test_norm_and_product_in_one_pass(dev, m, n, k):
     want = ops.linear(ops.rmsnorm(x.float(), nw, 1e-5), w)
     assert torch.equal(torch.nan_to_num(got, 7.0), torch.nan_to_num(want, 7.0))
     assert torch.equal(got.isnan(), want.isnan()) and (m <= 4 or bool(got[2:4].isnan().all()))
+
+
+@pytest.mark.parametrize("which", ["x", "w", "both"])
+def test_norm_and_product_of_rows_at_odd_addresses(dev, which):
+    """The pass reads whole 16-byte pieces; other views of x and w go op by op, or through an aligned copy of w."""
+    m, n, k = 100, 36, 128
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(dev)
+    w, nw = (torch.randn(n, k, generator=gen) * 0.02).to(dev), (torch.rand(k, generator=gen) + 0.5).to(dev)
+    want = ops.norm_linear_fp32(x, nw, w, 1e-5)
+
+    def at(t, odd):
+        return torch.empty(t.numel() + 8, dtype=t.dtype, device=dev)[odd:odd + t.numel()].view(t.shape).copy_(t)
+
+    x2, w2 = at(x, int(which != "w")), at(w, int(which != "x"))
+    assert torch.equal(ops.norm_linear_fp32(x2, nw, w2, 1e-5), want)
+    nws = ops.lib().lng_linear_split_workspace_bytes(n, k)
+    y, ws = torch.empty(m, n, device=dev), torch.empty(nws, dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+
+    def call(xt, space, size):
+        return ops.lib().lng_linear_split(xt.data_ptr(), nw.data_ptr(), w2.data_ptr(), m, n, k, 1e-5, space, size,
+                                          y.data_ptr(), stream)
+
+    if which == "w":
+        assert call(x2, None, 0) == -1 and call(x2, ws.data_ptr(), nws - 1) == -1
+        assert call(x2, ws.data_ptr(), nws) == 0 and torch.equal(y, want)
+    else:
+        assert call(x2, ws.data_ptr(), nws) == -1
