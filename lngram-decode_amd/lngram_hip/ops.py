@@ -517,11 +517,9 @@ def norm_linear_fp32(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, eps
     n = w.shape[0]
     if w.shape[1] != k or tuple(norm_w.shape) != (k,):
         raise ValueError(f"weight {tuple(w.shape)} and norm {tuple(norm_w.shape)} do not match input dim {k}")
-    x2, nw, wc = _c(x.reshape(-1, k)), _c(norm_w.float()), _c(w.float())
-    # the pass reads whole 16-byte pieces; a view that starts between them goes op by op
-    if (x.dtype != torch.bfloat16 or not lib().lng_linear_split_workspace_bytes(n, k)
-            or (x2.data_ptr() | wc.data_ptr()) & 15):
+    if x.dtype != torch.bfloat16 or not lib().lng_linear_split_workspace_bytes(n, k):
         return linear(rmsnorm(x.float(), norm_w.float(), eps), w.float())
+    x2, nw, wc = _c(x.reshape(-1, k)), _c(norm_w.float()), _c(w.float())
     out = torch.empty(*x.shape[:-1], n, dtype=torch.float32, device=dev)
     check(lib().lng_linear_split(_ptr(x2), _ptr(nw), _ptr(wc), x2.shape[0], n, k, float(eps), None, 0, _ptr(out),
                                  _stream(dev)), "linear_split")

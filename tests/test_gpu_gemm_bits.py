@@ -112,7 +112,8 @@ def test_norm_and_product_in_one_pass(dev, m, n, k):
 
 @pytest.mark.parametrize("which", ["x", "w", "both"])
 def test_norm_and_product_of_rows_at_odd_addresses(dev, which):
-    """The pass reads whole 16-byte pieces; other views of x and w go op by op, or through an aligned copy of w."""
+    """The kernel reads whole 16-byte pieces: other views of x and w are copied by the binding, and the library
+    takes a w of its own through an aligned copy in the workspace."""
     m, n, k = 100, 36, 128
     gen = torch.Generator().manual_seed(3)
     x = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(dev)
