@@ -425,7 +425,8 @@ int lng_table_grad_rows(const void* grad_memory, int mem_dtype, int64_t grad_str
  * apart).  Any of the three gradients may be null (not wanted).  Serves the shapes for which
  * lng_lookup_grad_workspace_bytes gives a size (bf16 rows of 128, 4-bit codes, exact = 0, R <= 256,
  * B*T < 2^20).  grad_q is the same in every call; as in lng_table_grad_rows the order in which a row's
- * windows are summed varies between calls, and with it the rounding of the table gradients.  Rows and tables 16-byte aligned, the workspace (written before it is read) 256-byte. */
+ * windows are summed varies between calls, and with it the rounding of the table gradients.  Rows and
+ * tables 16-byte aligned, the workspace (written before it is read) 256-byte. */
 size_t lng_lookup_grad_workspace_bytes(int64_t B, int64_t T, int32_t R, int32_t mem_dim, int32_t bits, int mem_dtype,
                                        int exact);
 int lng_lookup_grad(const void* grad_memory, int mem_dtype, int64_t grad_stride, const void* q_logits, int q_dtype,

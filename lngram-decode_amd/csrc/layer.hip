@@ -68,8 +68,8 @@ struct Fwd {  // workspace offsets of one forward
 bool layer_ok(const lng_memory_layer* L) {
   return L && (L->dtype == LNG_BF16 || L->dtype == LNG_F32) && L->hidden > 0 && L->routes > 0 && L->n_orders >= 1 &&
          L->n_orders <= 4 && L->mem_dim > 0 && L->q_heads > 0 && L->kv_heads > 0 && L->head_dim > 0 &&
-         L->q_heads % L->kv_heads == 0 && int64_t{L->q_heads} * L->head_dim == L->hidden && L->conv_k > 0 && L->conv_dilation > 0 && L->w_q && L->q_norm && L->kv &&
-         L->mem_norm && L->w_o && L->conv_norm && L->conv_w &&
+         L->q_heads % L->kv_heads == 0 && int64_t{L->q_heads} * L->head_dim == L->hidden && L->conv_k > 0 &&
+         L->conv_dilation > 0 && L->w_q && L->q_norm && L->kv && L->mem_norm && L->w_o && L->conv_norm && L->conv_w &&
          (!L->fused || (L->dtype == LNG_BF16 && L->n_orders == 2 && L->orders[0] == 2 && L->orders[1] == 3 &&
                         L->mem_dim == 128 && L->bits == 4 && L->q_heads == 16 && L->kv_heads == 4 && L->head_dim == 64));
 }

@@ -174,9 +174,9 @@ __device__ __forceinline__ void store8(bf16* p, const float (&v)[8]) {
 // apart, as k_conv_slots does.  4 x 128 x 128 fp32: 24.5 us with one wave-serial pass over the rows and 16
 // of 128 threads sliding over the positions.
 template <typename T, int TT, int NO>
-__global__ __launch_bounds__(NO == 1 ? 256 : 512) void k_causal_conv_k4d3(const T* __restrict__ mixed, const T* __restrict__ norm_w,
-                                                          const T* __restrict__ conv_w, ConvWin W, int32_t d,
-                                                          float eps, int residual, T* __restrict__ out) {
+__global__ __launch_bounds__(NO == 1 ? 256 : 512) void k_causal_conv_k4d3(
+    const T* __restrict__ mixed, const T* __restrict__ norm_w, const T* __restrict__ conv_w, ConvWin W, int32_t d, float eps,
+    int residual, T* __restrict__ out) {
   constexpr int NR = TT + C43_HALO, RPW = (NR + 3) / 4;
   __shared__ float scale[NR];
   const int64_t b = blockIdx.y;

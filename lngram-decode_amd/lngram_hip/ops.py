@@ -441,7 +441,8 @@ def memory_step(layer, h: torch.Tensor, codes: torch.Tensor, pos0: int, code_cac
     r, s = layer.routes, code_cache.shape[1]
     dev = h.device
     if d != layer.hidden or dtype_code(h.dtype) != layer.dtype or codes.shape != (b, n, r) \
-            or code_cache.shape != (b, s, r) or conv_cache.shape != (b, s, d) or pos0 + n > s or code_cache.dtype != torch.uint8 or conv_cache.dtype != torch.bfloat16 \
+            or code_cache.shape != (b, s, r) or conv_cache.shape != (b, s, d) or pos0 + n > s \
+            or code_cache.dtype != torch.uint8 or conv_cache.dtype != torch.bfloat16 \
             or not code_cache.is_contiguous() or not conv_cache.is_contiguous() \
             or not dev == codes.device == code_cache.device == conv_cache.device:
         return None
